@@ -1419,190 +1419,267 @@ __global__ void k_of_finish(const float4 *__restrict__ x, float4 *__restrict__ o
 }
 
 // ---------------------------------------------------------------------------
-// Passes over 3^4 neighbourhoods with LDS-staged planes.  A workgroup owns a
-// TX x TY x 2 column of cells (64 x 2 x 2, or 32 x 4 x 2 on grids whose
-// width would leave 64-wide tiles largely empty) for a segment of t and
-// marches through it, keeping the haloed planes t-1, t, t+1 ((TX+2) x (TY+2)
-// x 4 cells each) in a ring of three LDS slots, so the 81 reads per cell hit
-// LDS instead of the vector caches.  Interior cells have all 81 neighbours in
-// the grid.
+// ---------------------------------------------------------------------------
+// Passes over 3^4 neighbourhoods.  Lane l of a wavefront owns cell 62 w - 1 + l
+// of the t-planes (cells numbered x fastest, so the x neighbours are the
+// neighbouring lanes and lanes 1 .. 62 are written) and marches it through a
+// t segment.  A plane's 9 (z, y) rows are loaded once, one step ahead, and
+// added to the sums of the outputs t+1, t and t-1 of that plane, which are in
+// flight together (each sum still takes its planes, rows and cells in order);
+// the x neighbours come from a DPP lane shift that is an operand of the
+// addition.  No LDS and no barriers; the lanes need no tile shape, so a grid
+// of any width fills them (62 of 64).
 //  MARCH_BOX81: knCvExpolBlur4d (optflow4d.cpp:613-626): unmarked interior
 //    cells take the 3^4 box mean, summed in the reference's loop order (t,
-//    z, y, x outermost to innermost, FP32, starting from zero); other cells
-//    are copied.  `aux` is the marker grid.
+//    z, y, x outermost to innermost, FP32, starting from zero).  `mask` holds
+//    those cells, one word per wavefront and t step (k_box_mask, which also
+//    gives both buffers of the alternating passes the cells that never
+//    change, so the passes write the others only and a wavefront without any
+//    returns at once).
 //  MARCH_BLUR1: the Gaussian blur of k_blur4d for a window of s = 1 (never
 //    clipped for an interior cell), same order and operations; other cells
-//    are left unchanged.  `aux` is the weight table by squared distance.
+//    are left unchanged.  The products with the weight of a row's x
+//    neighbours are formed once and shifted, and the weight sum is one number.
+// Bound by VALU issue: 324 additions per cell (box) or 540 operations (blur)
+// where the LDS form it replaced read 81 values of 16 bytes per cell.
 enum { MARCH_BOX81 = 0, MARCH_BLUR1 = 1 };
-template <int TX>
-struct BoxTile {
-    static constexpr int X = TX, Y = TX == 64 ? 2 : 4, Z = 2;
-    static constexpr int HX = X + 2, HY = Y + 2, HZ = Z + 2;
-    static constexpr int PLANE = HX * HY * HZ;        // 1056 / 816 cells
-    static constexpr int LOADS = (PLANE + 255) / 256;  // per thread and plane
-    static_assert(X * Y * Z == 256, "one cell per thread");
+constexpr int M3_OUT = 62;  // cells a wavefront writes per t step
+
+struct March3 {
+    int nw;            // wavefronts along the cells of a t-plane
+    int nwg;           // workgroups (of 4) of them
+    int seglen, nseg;  // t segments (seglen <= 64: a lane holds each step's mask)
+    int total;         // nwg * nseg
+};
+struct Blur3W {
+    float w[5];  // weight by squared distance 0..4
+    float sum;   // of the 81, in the reference's order
 };
 
-struct BoxMarch {
-    int tx;                    // tile width: 64 or 32
-    int ntx, nty, ntz, ntile;  // column tiles
-    int seglen, nseg;          // t segments
-};
-
-template <class T, int OP, int TX>
-__global__ void __launch_bounds__(256)
-k_march3_lds(const T *__restrict__ a, T *__restrict__ out, const float *__restrict__ aux,
-             Dims4 D, BoxMarch B, float eps)
+// the value of the lane below / above (0 beyond the wavefront's ends)
+__device__ __forceinline__ float lane_below(float v)
 {
-    typedef VOps<T> O;
-    typedef BoxTile<TX> BT;
-    constexpr int BX_X = BT::X, BX_Y = BT::Y, BX_Z = BT::Z;
-    constexpr int BX_HX = BT::HX, BX_HY = BT::HY;
-    constexpr int BX_PLANE = BT::PLANE, BX_LOADS = BT::LOADS;
-    __shared__ T pl[3][BX_PLANE];
-    const int tile = blockIdx.x % B.ntile;
-    const int seg = blockIdx.x / B.ntile;
-    const int bx = tile % B.ntx, by = (tile / B.ntx) % B.nty, bz = tile / (B.ntx * B.nty);
-    const int x0 = bx * BX_X, y0 = by * BX_Y, z0 = bz * BX_Z;
-    const int t0 = seg * B.seglen;
-    const int t1 = min(t0 + B.seglen, D.T);
-    const int tx = threadIdx.x % BX_X, ty = (threadIdx.x / BX_X) % BX_Y,
-              tz = threadIdx.x / (BX_X * BX_Y);
-    const int gx = x0 + tx, gy = y0 + ty, gz = z0 + tz;
-    const bool own = gx < D.X && gy < D.Y && gz < D.Z;
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_above(float v)
+{
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float4 lane_below(const float4 &v)
+{
+    return make_float4(lane_below(v.x), lane_below(v.y), lane_below(v.z), lane_below(v.w));
+}
+__device__ __forceinline__ float4 lane_above(const float4 &v)
+{
+    return make_float4(lane_above(v.x), lane_above(v.y), lane_above(v.z), lane_above(v.w));
+}
 
-    // halo cells this thread stages: e = threadIdx.x + 256 m
-    int64_t hoff[BX_LOADS];  // offset inside a t-plane, -1: outside the grid
-#pragma unroll
-    for (int m = 0; m < BX_LOADS; ++m) {
-        const int e = threadIdx.x + 256 * m;
-        hoff[m] = -1;
-        if (e < BX_PLANE) {
-            const int hx = e % BX_HX, hy = (e / BX_HX) % BX_HY, hz = e / (BX_HX * BX_HY);
-            const int x = x0 + hx - 1, y = y0 + hy - 1, z = z0 + hz - 1;
-            if (x >= 0 && x < D.X && y >= 0 && y < D.Y && z >= 0 && z < D.Z)
-                hoff[m] = x + (int64_t)D.X * y + D.sz * z;
-        }
-    }
-    T st[BX_LOADS];
-    auto fetch = [&](int p) {
-#pragma unroll
-        for (int m = 0; m < BX_LOADS; ++m)
-            st[m] = (p >= 0 && p < D.T && hoff[m] >= 0) ? a[hoff[m] + D.st * p] : O::zero();
-    };
-    auto stash = [&](int p) {
-        T *s = pl[(p + 3) % 3];
-#pragma unroll
-        for (int m = 0; m < BX_LOADS; ++m) {
-            const int e = threadIdx.x + 256 * m;
-            if (e < BX_PLANE) s[e] = st[m];
-        }
-    };
-    // planes t0-1 and t0 (t0-1 may be -1: never read, see below)
-    fetch(t0 - 1);
-    stash(t0 - 1);
-    fetch(t0);
-    stash(t0);
-    const int cl = (tx + 1) + BX_HX * ((ty + 1) + BX_HY * (tz + 1));
-    for (int t = t0; t < t1; ++t) {
-        fetch(t + 1);
-        __syncthreads();  // every wave is done with plane t-2's slot
-        stash(t + 1);
-        __syncthreads();
-        if (!own) continue;
-        const int64_t c = gx + (int64_t)D.X * gy + D.sz * gz + D.st * t;
-        const bool in = interior(D, gx, gy, gz, t);
-        if (OP == MARCH_BOX81) {
-            if (!in || aux[c] != 0.f) {
-                out[c] = pl[t % 3][cl];
-                continue;
-            }
-            T val = O::zero();
-            for (int vt = -1; vt <= 1; ++vt) {
-                const T *s = pl[(t + vt + 3) % 3];
-#pragma unroll
-                for (int zk = -1; zk <= 1; ++zk)
-#pragma unroll
-                    for (int yj = -1; yj <= 1; ++yj)
-#pragma unroll
-                        for (int xi = -1; xi <= 1; ++xi)
-                            val = O::add(val, s[cl + xi + BX_HX * (yj + BX_HY * zk)]);
-            }
-            const double f = 1. / 81.0;
-            if constexpr (sizeof(T) == 16) {
-                const float4 v = *(const float4 *)&val;
-                ((float4 *)out)[c] = make_float4((float)(v.x * f), (float)(v.y * f),
-                                                 (float)(v.z * f), (float)(v.w * f));
-            } else {
-                ((float *)out)[c] = (float)(*(const float *)&val * f);
-            }
-        } else {
-            if (!in) continue;
-            T val = O::zero();
-            float weight = 0.f;
-            for (int vt = -1; vt <= 1; ++vt) {
-                const T *s = pl[(t + vt + 3) % 3];
-                // z not unrolled: 9 taps in flight keep the Vec4 form at
-                // 2 or more waves per SIMD
-#pragma unroll 1
-                for (int zk = -1; zk <= 1; ++zk)
-#pragma unroll
-                    for (int yj = -1; yj <= 1; ++yj)
-#pragma unroll
-                        for (int xi = -1; xi <= 1; ++xi) {
-                            const float w = aux[vt * vt + zk * zk + yj * yj + xi * xi];
-                            weight = weight + w;
-                            val = O::add(val, O::muls(s[cl + xi + BX_HX * (yj + BX_HY * zk)], w));
-                        }
-            }
-            if (weight > eps) {
-                if constexpr (sizeof(T) == 16) {
-                    const float4 v = *(const float4 *)&val;
-                    ((float4 *)out)[c] = make_float4(v.x / weight, v.y / weight, v.z / weight,
-                                                     v.w / weight);
-                } else {
-                    ((float *)out)[c] = *(const float *)&val / weight;
-                }
-            } else {
-                out[c] = pl[t % 3][cl];
-            }
-        }
+// Keeps the order of a sum's rows: the lane shifts become operands of the
+// additions only while each stands next to its use, and without this the
+// compiler moves all of them to the front (4 registers and 8 moves per row).
+__device__ __forceinline__ void m3_pin(float &c, float &val) { asm volatile("" : "+v"(c), "+v"(val)); }
+__device__ __forceinline__ void m3_pin(float4 &c, float4 &val)
+{
+    asm volatile(""
+                 : "+v"(c.x), "+v"(c.y), "+v"(c.z), "+v"(c.w), "+v"(val.x), "+v"(val.y),
+                   "+v"(val.z), "+v"(val.w));
+}
+
+// the work item of a wavefront: its first lane's cell and its t segment
+struct M3Item {
+    int base, t0, t1, item;
+    bool live;
+};
+__device__ __forceinline__ M3Item m3_item(const Dims4 &D, const March3 &M)
+{
+    M3Item w;
+    const int per = (int)gridDim.x / FLOF_NXCD;  // the grid is a multiple of 8
+    const int L = ((int)blockIdx.x % FLOF_NXCD) * per + (int)blockIdx.x / FLOF_NXCD;
+    const int seg = L / M.nwg;
+    const int wv = (L - seg * M.nwg) * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    w.live = L < M.total && wv < M.nw;
+    w.base = M3_OUT * wv - 1;
+    w.t0 = seg * M.seglen;
+    w.t1 = min(w.t0 + M.seglen, D.T);
+    w.item = seg * M.nw + wv;
+    return w;
+}
+
+// lanes whose cell a pass may write and that is interior in x, y and z
+__device__ __forceinline__ bool m3_inner(const Dims4 &D, const M3Item &w, int lane)
+{
+    const int c3 = w.base + lane;
+    if (lane < 1 || lane > M3_OUT || c3 >= (int)D.st) return false;
+    const int i = c3 % D.X, j = (c3 / D.X) % D.Y, k = c3 / (int)D.sz;
+    return i >= 1 && j >= 1 && k >= 1 && i < D.X - 1 && j < D.Y - 1 && k < D.Z - 1;
+}
+
+// The cells the box passes compute (interior, marker 0), and the copy of all
+// others into the second buffer of the alternating passes.
+__global__ void __launch_bounds__(256)
+k_box_mask(const float4 *__restrict__ a, float4 *__restrict__ out,
+           const float *__restrict__ marker, unsigned long long *__restrict__ mask, Dims4 D,
+           March3 M)
+{
+    const M3Item w = m3_item(D, M);
+    if (!w.live) return;
+    const int lane = threadIdx.x & 63;
+    const int c3 = w.base + lane;
+    const bool own = lane >= 1 && lane <= M3_OUT && c3 < (int)D.st;
+    const bool inner = m3_inner(D, w, lane);
+    for (int t = w.t0; t < w.t1; ++t) {
+        const int64_t c = c3 + D.st * t;
+        bool need = inner && t >= 1 && t < D.T - 1;
+        if (need) need = marker[c] == 0.f;
+        if (own && !need) out[c] = a[c];
+        const unsigned long long m = __ballot(need);
+        if (lane == 0) mask[(int64_t)w.item * M.seglen + (t - w.t0)] = m;
     }
 }
 
-// per_cu: workgroups per CU that the t segments aim at
-static BoxMarch make_boxmarch(flof_ctx *ctx, const Dims4 &D, int per_cu = 6)
+// the 9 rows (z, then y) around the lane's cell in plane p; rel: the lane's
+// cell after wb, both kept where every row lies in the plane (the cells of
+// interior cells' rows always do; the others' values are never used)
+template <class T>
+__device__ __forceinline__ void m3_load(T (&R)[9], const T *__restrict__ a, const Dims4 &D,
+                                        int p, int wb, unsigned rel)
 {
-    BoxMarch B;
-    // 32-wide tiles where they cover the x extent with 10% fewer lanes
-    const int w64 = (D.X + 63) / 64 * 64, w32 = (D.X + 31) / 32 * 32;
-    B.tx = 10 * w32 < 9 * w64 ? 32 : 64;
-    const int ty = B.tx == 64 ? BoxTile<64>::Y : BoxTile<32>::Y;
-    B.ntx = (D.X + B.tx - 1) / B.tx;
-    B.nty = (D.Y + ty - 1) / ty;
-    B.ntz = (D.Z + 1) / 2;
-    B.ntile = B.ntx * B.nty * B.ntz;
-    // the default 6: twice the workgroups per CU that LDS admits at once for
-    // 64-wide Vec4 tiles (three of 50 KB)
-    const int target = ctx->num_cu * per_cu;
-    int nseg = (target + B.ntile - 1) / B.ntile;
-    nseg = std::max(1, std::min(nseg, D.T));
-    B.seglen = (D.T + nseg - 1) / nseg;
-    B.nseg = (D.T + B.seglen - 1) / B.seglen;
-    return B;
+    p = max(0, min(p, D.T - 1));
+    const T *b = a + D.st * p + wb;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        const T *row = b + D.sz * (r / 3 - 1) + (int64_t)D.X * (r % 3 - 1);
+        R[r] = *(const T *)((const char *)row + rel * (unsigned)sizeof(T));
+    }
+}
+
+// adds the 27 cells of a plane's rows to val, in order; vt: plane - output (-1, 0, 1)
+template <class T, int OP>
+__device__ __forceinline__ void m3_add(T &val, T (&R)[9], const Blur3W &W, int vt)
+{
+    typedef VOps<T> O;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        m3_pin(R[r], val);
+        if (OP == MARCH_BOX81) {
+            val = O::add(val, lane_below(R[r]));
+            val = O::add(val, R[r]);
+            val = O::add(val, lane_above(R[r]));
+        } else {
+            const int d = (vt != 0) + (r / 3 != 1) + (r % 3 != 1);
+            const T side = O::muls(R[r], W.w[d + 1]);
+            val = O::add(val, lane_below(side));
+            val = O::add(val, O::muls(R[r], W.w[d]));
+            val = O::add(val, lane_above(side));
+        }
+    }
 }
 
 template <class T, int OP>
-static void launch_march3(flof_ctx *ctx, const BoxMarch &B, const T *src, T *dst,
-                          const float *aux, const Dims4 &D, float eps)
+__global__ void __launch_bounds__(256)
+k_march3(const T *__restrict__ a, T *__restrict__ out,
+         const unsigned long long *__restrict__ mask, Dims4 D, March3 M, Blur3W W, float eps)
 {
-    const dim3 grid(B.ntile * B.nseg);
-    if (B.tx == 32)
-        hipLaunchKernelGGL((k_march3_lds<T, OP, 32>), grid, dim3(256), 0, ctx->stream, src, dst,
-                           aux, D, B, eps);
-    else
-        hipLaunchKernelGGL((k_march3_lds<T, OP, 64>), grid, dim3(256), 0, ctx->stream, src, dst,
-                           aux, D, B, eps);
+    typedef VOps<T> O;
+    const M3Item w = m3_item(D, M);
+    if (!w.live) return;
+    const int lane = threadIdx.x & 63;
+    // per t step the lanes that compute: box: lane s holds step s's mask
+    unsigned mlo = 0, mhi = 0;
+    unsigned long long sp = 0;
+    if (OP == MARCH_BOX81) {
+        if (lane < w.t1 - w.t0) {
+            const unsigned long long m = mask[(int64_t)w.item * M.seglen + lane];
+            mlo = (unsigned)m;
+            mhi = (unsigned)(m >> 32);
+        }
+        if (__ballot((mlo | mhi) != 0) == 0) return;
+    } else {
+        sp = __ballot(m3_inner(D, w, lane));
+        if (sp == 0) return;
+    }
+    // lanes of output t (none outside the segment)
+    auto lanes_of = [&](int t) -> unsigned long long {
+        if (t < w.t0 || t >= w.t1) return 0;
+        if (OP == MARCH_BOX81)
+            return (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)mlo, t - w.t0) |
+                   (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)mhi, t - w.t0)
+                       << 32;
+        return t >= 1 && t < D.T - 1 ? sp : 0;
+    };
+    // interior cells exist, so lo <= hi
+    const int lo = D.X * D.Y + D.X, hi = (int)D.st - 1 - lo;
+    const int wb = max(lo, min(w.base, hi));
+    const unsigned rel = (unsigned)(max(lo, min(w.base + lane, hi)) - wb);
+    // sums of the outputs p - 1, p, p + 1 while plane p is added
+    T s0 = O::zero(), s1 = O::zero(), s2 = O::zero();
+    T centre = O::zero();  // the lane's own cell in plane p - 1
+    unsigned long long m0 = 0, m1 = 0, m2 = lanes_of(w.t0);
+    T A[2][9];
+    m3_load(A[0], a, D, w.t0 - 1, wb, rel);
+    for (int pb = w.t0 - 1; pb <= w.t1; pb += 2) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int p = pb + q;
+            if (p > w.t1) break;
+            if (p < w.t1) m3_load(A[q ^ 1], a, D, p + 1, wb, rel);
+            // every lane sums (a lane's neighbours must be active)
+            if (m0) m3_add<T, OP>(s0, A[q], W, 1);
+            if (m1) m3_add<T, OP>(s1, A[q], W, 0);
+            if (m2) m3_add<T, OP>(s2, A[q], W, -1);
+            if ((m0 >> lane) & 1) {
+                const int64_t c = w.base + lane + D.st * (p - 1);
+                if constexpr (OP == MARCH_BOX81) {
+                    const double f = 1. / 81.0;
+                    out[c] = make_float4((float)(s0.x * f), (float)(s0.y * f),
+                                         (float)(s0.z * f), (float)(s0.w * f));
+                } else if constexpr (sizeof(T) == 16) {
+                    out[c] = W.sum > eps ? make_float4(s0.x / W.sum, s0.y / W.sum,
+                                                       s0.z / W.sum, s0.w / W.sum)
+                                         : centre;
+                } else {
+                    out[c] = W.sum > eps ? s0 / W.sum : centre;
+                }
+            }
+            if (OP == MARCH_BLUR1) centre = A[q][4];
+            s0 = s1;
+            s1 = s2;
+            s2 = O::zero();
+            m0 = m1;
+            m1 = m2;
+            m2 = lanes_of(p + 2);
+        }
+    }
+}
+
+// The t segments: a CU runs one workgroup per 4 wavefronts of a segment, and
+// its VALUs are what bounds the pass, so the length is the one that gives the
+// busiest CU the fewest steps, counting 0.7 step per segment for its start
+// (32^3 x 48: 7 steps, 64^4: 16).
+static March3 make_march3(const flof_ctx *ctx, const Dims4 &D)
+{
+    March3 M;
+    M.nw = (int)((D.st + 1 + M3_OUT - 1) / M3_OUT);
+    M.nwg = (M.nw + 3) / 4;
+    double best = 1e300;
+    for (int len = std::min(64, D.T); len >= 1; --len) {
+        const int nseg = (D.T + len - 1) / len;
+        const int64_t rounds = ((int64_t)M.nwg * nseg + ctx->num_cu - 1) / ctx->num_cu;
+        const double cost = (double)rounds * (len + 0.7);
+        if (cost < best) {
+            best = cost;
+            M.seglen = len;
+            M.nseg = nseg;
+        }
+    }
+    M.total = M.nwg * M.nseg;
+    return M;
+}
+static inline dim3 march3_grid(const March3 &M)
+{
+    return dim3((M.total + FLOF_NXCD - 1) / FLOF_NXCD * FLOF_NXCD);
 }
 
 // Gaussian blur (optflow4d.cpp:127-174): every interior cell sums the
@@ -1611,8 +1688,8 @@ static void launch_march3(flof_ctx *ctx, const BoxMarch &B, const T *src, T *dst
 // the weight sum.  The weight of a squared distance d is
 // (float)exp(-d / (2 sigma^2)) evaluated in double on the host, one table
 // entry per d in [0, 4 s^2], so the device uses the host's exp.  This
-// gathering form serves windows of s >= 3; s = 1 and s = 2 run as the LDS
-// marches k_march3_lds and k_blur5_lds with the same sums.
+// gathering form serves windows of s >= 3; s = 1 and s = 2 run as the
+// marches k_march3 and k_march5 with the same sums.
 template <class T>
 __global__ void __launch_bounds__(256)
 k_blur4d(const T *__restrict__ src, T *__restrict__ dst, Dims4 D, Coord4 C, int s,
@@ -1652,111 +1729,231 @@ k_blur4d(const T *__restrict__ src, T *__restrict__ dst, Dims4 D, Coord4 C, int 
     }
 }
 
-// The same blur for windows of s = 2 (5^4 taps) with LDS-staged planes.  A
-// workgroup owns a TX x TY x 2 column of cells of one component (the four
-// components of a Vec4 grid are four independent sums, one workgroup each)
-// and marches it through a t segment, keeping the planes t-2 .. t+2 with a
-// two-cell halo ((TX+4) x (TY+4) x 6 values) in a ring of five LDS slots, so
-// the 625 reads per cell hit LDS instead of the vector caches.  Window
-// positions outside the grid hold +0: the reference skips them, and adding
-// w * (+0) = +0 to a sum that started at +0 changes no bit (such a sum is
-// never -0).  The weight sum of a clipped window depends only on how far
-// the faces clip it: `wsum` holds it for each of the 4^4 clipping patterns
-// (per dimension the window of an interior cell is [-1, 2], [-2, 1], [-2, 2]
-// or [-1, 1]), summed on the host in the reference's order.
+// The same blur for windows of s = 2 (5^4 taps).  Lane l of a wavefront owns
+// one component of position 60 w - 2 + l of the t-planes, positions numbered
+// with one zero column after each row of X cells (so that a row's clipped
+// taps x - 2 and x + 2 fall on that column and the shifts by one and two lanes
+// serve every row); lanes 2 .. 61 are written.  The four wavefronts of a
+// workgroup are the four components of the same cells (Vec4 grids) or four
+// neighbouring stretches (Real grids).  A plane's 25 (z, y) rows are loaded
+// once, one step ahead, and added to the sums of the five outputs t-2 .. t+2
+// that use it.  A value's product with the weight of a squared distance is the
+// same in all of them, so a row takes 6 products and 25 additions for the 25
+// taps (and 6 moves for the shifts by two): about 37 operations where a sum
+// on its own takes 50, and no LDS reads.
+// Window positions outside the grid hold +0: the reference skips them, and
+// adding w * (+0) = +0 to a sum that started at +0 changes no bit (such a sum
+// is never -0).  Rows outside in z lie outside the plane's buffer, whose loads
+// then return 0; rows outside in y get such an address.  The weight sum of a
+// clipped window depends only on how far the faces clip it: `wsum` holds it
+// for each of the 4^4 clipping patterns (per dimension the window of an
+// interior cell is [-1, 2], [-2, 1], [-2, 2] or [-1, 1]), summed on the host
+// in the reference's order.
 struct Blur5W {
     float w[17];  // weight by squared distance 0..16
 };
+constexpr int M5_OUT = 60;  // positions a wavefront writes per t step
 __device__ __forceinline__ int blur5_pattern(int i, int n)
 {
     return (min(2, i) - 1) * 2 + (min(2, n - 1 - i) - 1);
 }
-template <int TX>
-__global__ void __launch_bounds__(256)
-k_blur5_lds(const float *__restrict__ src, float *__restrict__ dst, int cstride, Dims4 D,
-            BoxMarch B, Blur5W W, const float *__restrict__ wsum, float eps)
+// One row (z, y at squared distance s) into the sums v[0 .. 4] of the outputs
+// at t distance -2 .. 2: c times the weights of s + {0, 1, 2, 4, 5, 8}, then
+// the taps x - 2 .. x + 2 in order, each into all five sums.  Written out so
+// that every shift is an operand of its addition (the compiler shares a shift
+// between the two sums that use it, which costs a move more than it saves);
+// a lane shift reads a register at least two instructions after its write.
+__device__ __forceinline__ void m5_row(float c, float (&v)[5], const Blur5W &W, int s)
 {
-    typedef BoxTile<TX> BT;
-    constexpr int HX = BT::X + 4, HY = BT::Y + 4, HZ = BT::Z + 4;
-    constexpr int PLANE = HX * HY * HZ;  // 2448 / 1728 values
-    constexpr int LOADS = (PLANE + 255) / 256;
-    __shared__ float pl[5][PLANE];
-    const int per = B.ntile * B.nseg;
-    const int comp = blockIdx.x / per;
-    const int rem = blockIdx.x - comp * per;
-    const int tile = rem % B.ntile, seg = rem / B.ntile;
-    const int bx = tile % B.ntx, by = (tile / B.ntx) % B.nty, bz = tile / (B.ntx * B.nty);
-    const int x0 = bx * BT::X, y0 = by * BT::Y, z0 = bz * BT::Z;
-    const int t0 = seg * B.seglen;
-    const int t1 = min(t0 + B.seglen, D.T);
-    const int tx = threadIdx.x % BT::X, ty = (threadIdx.x / BT::X) % BT::Y,
-              tz = threadIdx.x / (BT::X * BT::Y);
-    const int gx = x0 + tx, gy = y0 + ty, gz = z0 + tz;
-    const bool own = gx < D.X && gy < D.Y && gz < D.Z;
-    src += comp;  // value of cell c at [c * cstride]
+    float p0, p1, p2, p4, p5, p8, a, b, e;
+#define M5_SHR " wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define M5_SHL " wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+    asm volatile("v_mul_f32 %[p4], %[w4], %[c]\n"
+                 "v_mul_f32 %[p5], %[w5], %[c]\n"
+                 "v_mul_f32 %[p8], %[w8], %[c]\n"
+                 "v_mov_b32_dpp %[a], %[p4]" M5_SHR
+                 "v_mov_b32_dpp %[b], %[p5]" M5_SHR
+                 "v_mov_b32_dpp %[e], %[p8]" M5_SHR
+                 "v_mul_f32 %[p1], %[w1], %[c]\n"
+                 "v_add_f32_dpp %[v2], %[a], %[v2]" M5_SHR
+                 "v_add_f32_dpp %[v1], %[b], %[v1]" M5_SHR
+                 "v_add_f32_dpp %[v3], %[b], %[v3]" M5_SHR
+                 "v_mul_f32 %[p2], %[w2], %[c]\n"
+                 "v_add_f32_dpp %[v0], %[e], %[v0]" M5_SHR
+                 "v_add_f32_dpp %[v4], %[e], %[v4]" M5_SHR
+                 "v_add_f32_dpp %[v2], %[p1], %[v2]" M5_SHR
+                 "v_add_f32_dpp %[v1], %[p2], %[v1]" M5_SHR
+                 "v_add_f32_dpp %[v3], %[p2], %[v3]" M5_SHR
+                 "v_mul_f32 %[p0], %[w0], %[c]\n"
+                 "v_add_f32_dpp %[v0], %[p5], %[v0]" M5_SHR
+                 "v_add_f32_dpp %[v4], %[p5], %[v4]" M5_SHR
+                 "v_mov_b32_dpp %[a], %[p4]" M5_SHL
+                 "v_mov_b32_dpp %[b], %[p5]" M5_SHL
+                 "v_mov_b32_dpp %[e], %[p8]" M5_SHL
+                 "v_add_f32 %[v2], %[p0], %[v2]\n"
+                 "v_add_f32 %[v1], %[p1], %[v1]\n"
+                 "v_add_f32 %[v3], %[p1], %[v3]\n"
+                 "v_add_f32 %[v0], %[p4], %[v0]\n"
+                 "v_add_f32 %[v4], %[p4], %[v4]\n"
+                 "v_add_f32_dpp %[v2], %[p1], %[v2]" M5_SHL
+                 "v_add_f32_dpp %[v1], %[p2], %[v1]" M5_SHL
+                 "v_add_f32_dpp %[v3], %[p2], %[v3]" M5_SHL
+                 "v_add_f32_dpp %[v0], %[p5], %[v0]" M5_SHL
+                 "v_add_f32_dpp %[v4], %[p5], %[v4]" M5_SHL
+                 "v_add_f32_dpp %[v2], %[a], %[v2]" M5_SHL
+                 "v_add_f32_dpp %[v1], %[b], %[v1]" M5_SHL
+                 "v_add_f32_dpp %[v3], %[b], %[v3]" M5_SHL
+                 "v_add_f32_dpp %[v0], %[e], %[v0]" M5_SHL
+                 "v_add_f32_dpp %[v4], %[e], %[v4]" M5_SHL
+                 : [v0] "+v"(v[0]), [v1] "+v"(v[1]), [v2] "+v"(v[2]), [v3] "+v"(v[3]),
+                   [v4] "+v"(v[4]), [p0] "=&v"(p0), [p1] "=&v"(p1), [p2] "=&v"(p2),
+                   [p4] "=&v"(p4), [p5] "=&v"(p5), [p8] "=&v"(p8), [a] "=&v"(a),
+                   [b] "=&v"(b), [e] "=&v"(e)
+                 : [c] "v"(c), [w0] "s"(W.w[s]), [w1] "s"(W.w[s + 1]), [w2] "s"(W.w[s + 2]),
+                   [w4] "s"(W.w[s + 4]), [w5] "s"(W.w[s + 5]), [w8] "s"(W.w[s + 8]));
+#undef M5_SHR
+#undef M5_SHL
+}
+
+// the rows of plane p: off is the lane's byte offset in the plane (beyond it
+// for the zero column), ym / yp the lanes whose rows y - 2 / y + 2 lie outside
+__device__ __forceinline__ void m5_load(float (&R)[25], const float *__restrict__ src,
+                                        const Dims4 &D, int p, unsigned es, unsigned off,
+                                        bool ym, bool yp)
+{
+    const unsigned bytes = (unsigned)D.st * es;  // < 2^32 (checked by the host)
+    const bool in = p >= 0 && p < D.T;
+    const char *b = (const char *)src + (in ? (int64_t)D.st * p * es : 0);
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void *)b, 0, in ? (int)bytes : 0, 0x00020000);
+#pragma unroll
+    for (int r = 0; r < 25; ++r) {
+        const int dz = r / 5 - 2, dy = r % 5 - 2;
+        const unsigned row = (unsigned)((int)(D.sz * dz + D.X * dy) * (int)es);
+        // the zero column's offset stays beyond the plane whatever the row
+        unsigned o = off == 0xffffffffu ? off : off + row;
+        if (dy == -2 && ym) o = 0xffffffffu;
+        if (dy == 2 && yp) o = 0xffffffffu;
+        R[r] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)o, 0, 0));
+    }
+}
+
+__global__ void __launch_bounds__(256, 4)
+k_march5(const float *__restrict__ src, float *__restrict__ dst, int ncomp, Dims4 D, March3 M,
+         Blur5W W, const float *__restrict__ wt, const float *__restrict__ wsum, float eps)
+{
+    const int per = (int)gridDim.x / FLOF_NXCD;  // the grid is a multiple of 8
+    const int L = ((int)blockIdx.x % FLOF_NXCD) * per + (int)blockIdx.x / FLOF_NXCD;
+    if (L >= M.total) return;
+    const int seg = L / M.nwg;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int wg = L - seg * M.nwg;
+    const int wv = ncomp == 4 ? wg : wg * 4 + wave;
+    if (wv >= M.nw) return;
+    const int comp = ncomp == 4 ? wave : 0;
+    const int t0 = seg * M.seglen, t1 = min(t0 + M.seglen, D.T);
+    const int lane = threadIdx.x & 63;
+    const int pos = M5_OUT * wv - 2 + lane;  // padded position
+    const int pitch = D.X + 1;
+    const int rows = D.Y * D.Z;
+    const int jr = pos >= 0 ? pos / pitch : 0;
+    const int i = pos >= 0 ? pos - jr * pitch : D.X;
+    const bool cell = i < D.X && jr < rows;
+    const int j = jr % D.Y, k = jr / D.Y;
+    const unsigned es = 4u * ncomp;
+    const unsigned off = cell ? (unsigned)(i + D.X * jr) * es : 0xffffffffu;
+    const bool inner = lane >= 2 && lane < 2 + M5_OUT && cell && i >= 1 && j >= 1 && k >= 1 &&
+                       i < D.X - 1 && j < D.Y - 1 && k < D.Z - 1;
+    if (__ballot(inner) == 0) return;
+    const bool ym = j < 2, yp = j + 2 >= D.Y;
+    src += comp;
     dst += comp;
-    // window cells this thread stages: e = threadIdx.x + 256 m
-    int64_t hoff[LOADS];  // cell offset inside a t-plane, -1: outside the grid
+    const int pxyz = inner ? (blur5_pattern(k, D.Z) * 4 + blur5_pattern(j, D.Y)) * 4 +
+                                 blur5_pattern(i, D.X)
+                           : 0;
+    // sums of the outputs p - 2 .. p + 2 while plane p is added
+    float v[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    float c0 = 0.f, c1 = 0.f;  // the lane's own cell in planes p - 2, p - 1
+    const int lo = max(t0, 1), hi = min(t1, D.T - 1);  // outputs [lo, hi)
+    float A[2][25];
+    m5_load(A[0], src, D, lo - 2, es, off, ym, yp);
+    for (int pb = lo - 2; pb <= hi + 1; pb += 2) {
 #pragma unroll
-    for (int m = 0; m < LOADS; ++m) {
-        const int e = threadIdx.x + 256 * m;
-        hoff[m] = -1;
-        if (e < PLANE) {
-            const int hx = e % HX, hy = (e / HX) % HY, hz = e / (HX * HY);
-            const int x = x0 + hx - 2, y = y0 + hy - 2, z = z0 + hz - 2;
-            if (x >= 0 && x < D.X && y >= 0 && y < D.Y && z >= 0 && z < D.Z)
-                hoff[m] = x + (int64_t)D.X * y + D.sz * z;
+        for (int q = 0; q < 2; ++q) {
+            const int p = pb + q;
+            if (p > hi + 1) break;
+            if (p <= hi) m5_load(A[q ^ 1], src, D, p + 1, es, off, ym, yp);
+            if (p - 2 >= lo && p + 2 < hi) {
+                // all five outputs
+#pragma unroll
+                for (int r = 0; r < 25; ++r)
+                    m5_row(A[q][r], v,
+                           W, (r / 5 - 2) * (r / 5 - 2) + (r % 5 - 2) * (r % 5 - 2));
+            } else if (p >= 0 && p < D.T) {
+                // the ends of the segment: each output on its own, in v[0]
+                // while the sums go round once
+#pragma unroll 1
+                for (int k5 = 0; k5 < 5; ++k5) {
+                    const int t = p - 2 + k5;
+                    if (t >= lo && t < hi) {
+                        const float *w = wt + (k5 - 2) * (k5 - 2);
+#pragma unroll
+                        for (int r = 0; r < 25; ++r) {
+                            const int s = (r / 5 - 2) * (r / 5 - 2) + (r % 5 - 2) * (r % 5 - 2);
+                            m3_pin(A[q][r], v[0]);
+                            const float c = A[q][r];
+                            const float far = c * w[s + 4], near = c * w[s + 1];
+                            v[0] = v[0] + lane_below(lane_below(far));
+                            v[0] = v[0] + lane_below(near);
+                            v[0] = v[0] + c * w[s];
+                            v[0] = v[0] + lane_above(near);
+                            v[0] = v[0] + lane_above(lane_above(far));
+                        }
+                    }
+                    const float first = v[0];
+                    v[0] = v[1];
+                    v[1] = v[2];
+                    v[2] = v[3];
+                    v[3] = v[4];
+                    v[4] = first;
+                }
+            }
+            const int t = p - 2;
+            if (inner && t >= lo) {
+                const float weight = wsum[blur5_pattern(t, D.T) * 64 + pxyz];
+                const int64_t c = i + (int64_t)D.X * jr + D.st * t;
+                dst[c * ncomp] = weight > eps ? v[0] / weight : c0;
+            }
+            c0 = c1;
+            c1 = A[q][12];
+#pragma unroll
+            for (int k5 = 0; k5 < 4; ++k5) v[k5] = v[k5 + 1];
+            v[4] = 0.f;
         }
     }
-    float stv[LOADS];
-    auto fetch = [&](int p) {
-#pragma unroll
-        for (int m = 0; m < LOADS; ++m)
-            stv[m] = (p >= 0 && p < D.T && hoff[m] >= 0) ? src[(hoff[m] + D.st * p) * cstride]
-                                                         : 0.f;
-    };
-    auto stash = [&](int p) {
-        float *sl = pl[(p + 10) % 5];
-#pragma unroll
-        for (int m = 0; m < LOADS; ++m) {
-            const int e = threadIdx.x + 256 * m;
-            if (e < PLANE) sl[e] = stv[m];
+}
+
+// The t segments of k_march5, as make_march3 picks them; a segment's two ends
+// cost about 2.5 steps (their planes serve fewer outputs)
+static March3 make_march5(const flof_ctx *ctx, const Dims4 &D, int ncomp)
+{
+    March3 M;
+    const int64_t pos = (int64_t)(D.X + 1) * D.Y * D.Z + 2;
+    M.nw = (int)((pos + M5_OUT - 1) / M5_OUT);
+    M.nwg = ncomp == 4 ? M.nw : (M.nw + 3) / 4;
+    double best = 1e300;
+    for (int len = D.T; len >= 1; --len) {
+        const int nseg = (D.T + len - 1) / len;
+        const int64_t rounds = ((int64_t)M.nwg * nseg + ctx->num_cu - 1) / ctx->num_cu;
+        const double cost = (double)rounds * (len + 2.5);
+        if (cost < best) {
+            best = cost;
+            M.seglen = len;
+            M.nseg = nseg;
         }
-    };
-    // planes t0-2 .. t0+1 (those outside the grid hold +0)
-    for (int p = t0 - 2; p <= t0 + 1; ++p) {
-        fetch(p);
-        stash(p);
     }
-    const int cl = (tx + 2) + HX * ((ty + 2) + HY * (tz + 2));
-    const bool own_in = own && gx >= 1 && gy >= 1 && gz >= 1 && gx < D.X - 1 &&
-                        gy < D.Y - 1 && gz < D.Z - 1;
-    const int pxyz = (blur5_pattern(gz, D.Z) * 4 + blur5_pattern(gy, D.Y)) * 4 +
-                     blur5_pattern(gx, D.X);
-    for (int t = t0; t < t1; ++t) {
-        fetch(t + 2);
-        __syncthreads();  // every wave is done with plane t-3's slot
-        stash(t + 2);
-        __syncthreads();
-        if (!own_in || t < 1 || t >= D.T - 1) continue;
-        // the reference's order: t, z, y, x from low to high
-        float val = 0.f;
-#pragma unroll
-        for (int vt = -2; vt <= 2; ++vt) {
-            const float *sl = pl[(t + vt + 10) % 5] + cl;
-#pragma unroll
-            for (int zk = -2; zk <= 2; ++zk)
-#pragma unroll
-                for (int yj = -2; yj <= 2; ++yj)
-#pragma unroll
-                    for (int xi = -2; xi <= 2; ++xi)
-                        val = val + sl[xi + HX * (yj + HY * zk)] *
-                                        W.w[vt * vt + zk * zk + yj * yj + xi * xi];
-        }
-        const float weight = wsum[blur5_pattern(t, D.T) * 64 + pxyz];
-        const int64_t c = gx + (int64_t)D.X * gy + D.sz * gz + D.st * t;
-        dst[c * cstride] = weight > eps ? val / weight : pl[t % 5][cl];
-    }
+    M.total = M.nwg * M.nseg;
+    return M;
 }
 
 void gaussian_blur(flof_ctx *ctx, void *a, const Dims4 &D, bool vec4, float sigma,
@@ -1780,13 +1977,24 @@ void gaussian_blur(flof_ctx *ctx, void *a, const Dims4 &D, bool vec4, float sigm
     Coord4 C = make_coord4(D);
     const int nb = grid_blocks_xcd(ctx, n);
     const float eps = 1e-6f;  // VECTOR_EPSILON of FP32 builds
-    const BoxMarch BM = make_boxmarch(ctx, D);
+    const March3 M3 = make_march3(ctx, D);
+    // s = 1: the weight of each squared distance and the sum of the 81 in the
+    // reference's order (no window of an interior cell is clipped)
+    Blur3W w3{};
+    if (s == 1) {
+        for (int d = 0; d < 5; ++d) w3.w[d] = wh[d];
+        for (int q = 0; q < 81; ++q)
+            w3.sum = w3.sum + wh[(q / 27 != 1) + (q / 9 % 3 != 1) + (q / 3 % 3 != 1) +
+                                 (q % 3 != 1)];
+    }
     // s = 2: the weight of each squared distance and the weight sums of the
     // 4^4 clipping patterns (summed in the reference's order)
     Blur5W w5{};
     Tmp wsum5;
-    BoxMarch BM5{};
-    if (s == 2) {
+    March3 M5{};
+    // (grids whose t-plane does not fit a 32-bit buffer take the gathering form)
+    const bool march5 = s == 2 && D.st * (vec4 ? 16 : 4) < (1ll << 32) - 64;
+    if (march5) {
         for (int d = 0; d < 17; ++d) w5.w[d] = wh[d];
         std::vector<float> ws(256);
         for (int pt = 0; pt < 4; ++pt)
@@ -1812,32 +2020,29 @@ void gaussian_blur(flof_ctx *ctx, void *a, const Dims4 &D, bool vec4, float sigm
         FLOF_HIP(hipMemcpyAsync(wsum5.p, ws.data(), 256 * sizeof(float),
                                 hipMemcpyHostToDevice, ctx->stream));
         FLOF_HIP(hipStreamSynchronize(ctx->stream));  // ws lives on the stack
-        BM5 = make_boxmarch(ctx, D, vec4 ? 2 : 6);
+        M5 = make_march5(ctx, D, vec4 ? 4 : 1);
     }
     auto pass = [&](const void *src, void *dst) {
-        if (s == 2) {
-            const int ncomp = vec4 ? 4 : 1;
-            const dim3 grid(BM5.ntile * BM5.nseg * ncomp);
-            if (BM5.tx == 32)
-                hipLaunchKernelGGL(k_blur5_lds<32>, grid, dim3(256), 0, ctx->stream,
-                                   (const float *)src, (float *)dst, ncomp, D, BM5, w5,
-                                   (const float *)wsum5.as<float>(), eps);
-            else
-                hipLaunchKernelGGL(k_blur5_lds<64>, grid, dim3(256), 0, ctx->stream,
-                                   (const float *)src, (float *)dst, ncomp, D, BM5, w5,
-                                   (const float *)wsum5.as<float>(), eps);
-            check_launch("k_blur5_lds");
+        if (march5) {
+            if (D.X < 3 || D.Y < 3 || D.Z < 3 || D.T < 3) return;  // no interior cell
+            hipLaunchKernelGGL(k_march5, march3_grid(M5), dim3(256), 0, ctx->stream,
+                               (const float *)src, (float *)dst, vec4 ? 4 : 1, D, M5, w5,
+                               (const float *)wdev.as<float>(), (const float *)wsum5.as<float>(), eps);
+            check_launch("k_march5");
             return;
         }
         if (s == 1) {
-            // the LDS-tiled form of the same sums (identical results)
+            // the marching form of the same sums (identical results)
+            if (D.X < 3 || D.Y < 3 || D.Z < 3 || D.T < 3) return;  // no interior cell
             if (vec4)
-                launch_march3<float4, MARCH_BLUR1>(ctx, BM, (const float4 *)src, (float4 *)dst,
-                                                   (const float *)wdev.as<float>(), D, eps);
+                hipLaunchKernelGGL((k_march3<float4, MARCH_BLUR1>), march3_grid(M3), dim3(256),
+                                   0, ctx->stream, (const float4 *)src, (float4 *)dst, nullptr,
+                                   D, M3, w3, eps);
             else
-                launch_march3<float, MARCH_BLUR1>(ctx, BM, (const float *)src, (float *)dst,
-                                                  (const float *)wdev.as<float>(), D, eps);
-            check_launch("k_march3_lds<blur1>");
+                hipLaunchKernelGGL((k_march3<float, MARCH_BLUR1>), march3_grid(M3), dim3(256),
+                                   0, ctx->stream, (const float *)src, (float *)dst, nullptr, D,
+                                   M3, w3, eps);
+            check_launch("k_march3<blur1>");
             return;
         }
         if (vec4)
@@ -1971,7 +2176,9 @@ void corr_vels_of(flof_ctx *ctx, float4 *dst, float4 *vel, const float *phiOrg,
     const int64_t n = (int64_t)D.st * D.T;
     const float blurThreshold = 0.98f;
     const int doCvExtrapol = (int)(host_max_norm_vec4(ctx, vel, n) + 4);
-    Tmp marker(ctx, (size_t)n * 4), tmp(ctx, (size_t)n * 16);
+    const March3 M3 = make_march3(ctx, D);
+    Tmp marker(ctx, (size_t)n * 4), tmp(ctx, (size_t)n * 16),
+        mask(ctx, (size_t)M3.nw * M3.nseg * M3.seglen * sizeof(unsigned long long));
     Coord4 C = make_coord4(D);
     const int nb = grid_blocks(ctx, n);
     int singleStep = 0;
@@ -1983,14 +2190,19 @@ void corr_vels_of(flof_ctx *ctx, float4 *dst, float4 *vel, const float *phiOrg,
                            phiOrg, phiTarget, marker.as<float>(), D, C, threshPhi, maxIter,
                            dt);
         check_launch("k_project_cells");
-        // the passes alternate between dst and tmp (every pass writes every
-        // cell); one copy at the end if the last pass wrote tmp
+        // the passes alternate between dst and tmp; one copy at the end if
+        // the last pass wrote tmp
         float4 *cur = dst, *nxt = tmp.as<float4>();
-        const BoxMarch BM = make_boxmarch(ctx, D);
+        hipLaunchKernelGGL(k_box_mask, march3_grid(M3), dim3(256), 0, ctx->stream,
+                           (const float4 *)cur, nxt, (const float *)marker.as<float>(),
+                           mask.as<unsigned long long>(), D, M3);
+        check_launch("k_box_mask");
         for (int it = 0; it < doCvExtrapol; ++it) {
-            launch_march3<float4, MARCH_BOX81>(ctx, BM, (const float4 *)cur, nxt,
-                                               (const float *)marker.as<float>(), D, 0.f);
-            check_launch("k_march3_lds<box81>");
+            hipLaunchKernelGGL((k_march3<float4, MARCH_BOX81>), march3_grid(M3), dim3(256), 0,
+                               ctx->stream, (const float4 *)cur, nxt,
+                               (const unsigned long long *)mask.as<unsigned long long>(), D, M3,
+                               Blur3W{}, 0.f);
+            check_launch("k_march3<box81>");
             std::swap(cur, nxt);
         }
         if (cur != dst)

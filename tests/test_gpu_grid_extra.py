@@ -299,3 +299,39 @@ def test_corr_vels_of4d_two_x_tiles_bit_exact(vx, X):
     assert np.abs(rd).max() > 0.5
     assert np.array_equal(dst.to_numpy(), rd)
     assert np.array_equal(vel.to_numpy(), rv)
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 3, 3), (61, 4, 5, 9), (62, 3, 4, 18), (63, 5, 3, 7),
+                                   (31, 6, 7, 33), (7, 30, 3, 70)])
+def test_marches_at_wavefront_and_segment_edges_bit_exact(shape):
+    """The blur marches (3^4 and 5^4 windows) and the box passes where a
+    wavefront's stretch of 62 cells (60 positions for the 5^4 window) ends at,
+    just before and just after a row's end, with one interior cell, and with t
+    extents that one, two and several t segments cover, infinities and NaN
+    among the values: equal to the oracle bit for bit."""
+    X, Y, Z, T = shape
+    rng = np.random.default_rng(15)
+    s = M.Solver(gridSize=M.vec3(X, Y, Z), fourthDim=T)
+    a4 = rng.standard_normal((T, Z, Y, X, 4)).astype(np.float32)
+    a4[T // 2, Z // 2, Y // 2, X // 2] = [np.inf, -np.inf, np.nan, -0.0]
+    say("marches", shape)
+    for sigma in (1.0, 2.0):
+        for vec in (True, False):
+            a = a4 if vec else np.ascontiguousarray(a4[..., 0])
+            g = s.create(M.Grid4Vec4 if vec else M.Grid4Real)
+            g.from_numpy(a)
+            M.gaussianBlur4d(g, sigma, 1)
+            assert np.array_equal(g.to_numpy(), O.gaussian_blur(a, sigma, 1), equal_nan=True)
+    x = np.arange(X, dtype=np.float64) + 0.5
+    phiOrg = (x - 0.45 * X + 0.3 * rng.standard_normal((T, Z, Y, X))).astype(np.float32)
+    phiTgt = (phiOrg - 1.0 + 0.3 * rng.standard_normal((T, Z, Y, X))).astype(np.float32)
+    vel0 = rng.standard_normal((T, Z, Y, X, 4)).astype(np.float32)
+    dst, vel = s.create(M.Grid4Vec4), s.create(M.Grid4Vec4)
+    vel.from_numpy(vel0)
+    po, pt = s.create(M.Grid4Real), s.create(M.Grid4Real)
+    po.from_numpy(phiOrg)
+    pt.from_numpy(phiTgt)
+    M.corrVelsOf4d(dst, vel, po, po, pt, threshPhi=1.5, postVelBlur=0.0, maxIter=40)
+    rd, rv = O.corr_vels_of4d(vel0, phiOrg, phiTgt, threshPhi=1.5, postVelBlur=0.0, maxIter=40)
+    assert np.array_equal(dst.to_numpy(), rd)
+    assert np.array_equal(vel.to_numpy(), rv)
