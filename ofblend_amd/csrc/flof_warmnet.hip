@@ -7,26 +7,27 @@
 // to the finest level and handed to the solve as its warm start (the solve
 // keeps it only where its residual is not larger than the zero start's).
 //
-// Network (C = 16 channels, activations FP32 channels-last [cell][16]):
-//   h0 = lift(i0/4, i1/4)                       pointwise 2 -> 16
+// Network (C = 16 channels, activations channels-last [cell][16]):
+//   h0 = lift(i0/4, i1/4)                       pointwise 2 -> 16 (not stored)
 //   4 blocks:  s = Ws * h + bs                  3x3x3 space conv 16 -> 16
 //              a = relu(s)
 //              h = h + (Wt * a + bt)            3-tap time conv 16 -> 16
 //   block b spaces its taps 2^b cells apart (dilation 1, 2, 4, 8), so the
 //   network sees 31 cells in x, y, z and t: as far as the flows reach
 //   flow = head(h)                              pointwise 16 -> 4
-// The convolutions run on the matrix cores: v_mfma_f32_16x16x32_bf16 with
-// BF16 weights and BF16-rounded activations, FP32 accumulation.  A wavefront
-// computes out^T (16 channels x 16 cells) for two taps per instruction:
+// The convolutions run on the matrix cores with BF16 weights and BF16-rounded
+// inputs, FP32 accumulation.  A value that only feeds convolutions (a, and
+// the copies of h, dh and ds that they read) is stored in BF16, rounded once
+// as the convolutions would round it; the residual chain h and its gradient
+// stay FP32.  A wavefront computes out^T (16 channels x 16 cells), in the
+// space convolutions for two taps per instruction (16x16x32):
 //   A (16 x 32) = weights   lane l: out channel l%16, k = 8*(l/16) .. +7
 //   B (32 x 16) = inputs    lane l: cell l%16,        k = 8*(l/16) .. +7
 //   D (16 x 16) = out^T     lane l: cell l%16, out channels 4*(l/16) .. +3
-// with k = 16*(tap - 2*pair) + input channel, so every lane loads 8
-// consecutive channels (32 B) of one neighbour and stores 4 consecutive
-// output channels (16 B) of one cell.  The backward data pass is the same
-// kernel with mirrored taps and transposed weights; the weight gradient uses
-// the same instruction with the cells as the reduction dimension.  Training
-// is Adam on FP32 master weights.
+// with k = 16*(tap - 2*pair) + input channel, in the time convolutions for one
+// (16x16x16, 4 channels per lane).  The backward data pass is the same kernel
+// with mirrored taps and transposed weights; the weight gradients have the
+// cells as the reduction dimension.  Training is Adam on FP32 master weights.
 
 #include <algorithm>
 #include <cmath>
@@ -44,7 +45,6 @@ constexpr int NB = 4;       // residual blocks
 constexpr int NS = 27;      // space taps
 constexpr int NTT = 3;      // time taps
 constexpr int PAIRS_S = 14; // ceil(27 / 2)
-constexpr int PAIRS_T = 2;  // ceil(3 / 2)
 
 // parameter layout (FP32, flat)
 constexpr int OFF_WL = 0;                   // [2][16]
@@ -60,15 +60,17 @@ constexpr int OFF_BH = OFF_WH + C * 4;      // [4]
 constexpr int NPARAM = OFF_BH + 4;          // 30964
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// round to nearest even (v_cvt_pk_bf16_f32)
 __device__ __forceinline__ unsigned short to_bf16(float f)
 {
-    unsigned u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
+    return __builtin_bit_cast(unsigned short, (__bf16)f);
 }
 
 __device__ __forceinline__ bf16x8 pack8(const float4 &a, const float4 &b)
@@ -84,6 +86,13 @@ __device__ __forceinline__ bf16x8 pack8(const float4 &a, const float4 &b)
     u[7] = to_bf16(b.w);
     return __builtin_bit_cast(bf16x8, u);
 }
+__device__ __forceinline__ u16x4 pack4(const f32x4 &v)
+{
+    u16x4 u;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = to_bf16(v[r]);
+    return u;
+}
 
 struct Geo {
     int X, Y, Z, T;
@@ -91,102 +100,399 @@ struct Geo {
     int dil;  // tap spacing of the convolutions
 };
 
-__device__ __forceinline__ void cell_coords(const Geo &g, int c, int &i, int &j, int &k, int &t)
+// Where a convolution's input comes from: a BF16 tensor [cell][16], or (block
+// 0) the lift of the two level sets, formed where it is needed: 8 bytes per
+// cell instead of 32 (BF16) or 64 (FP32 residual).
+struct In {
+    const unsigned short *b;
+    const float *i0, *i1, *P;
+};
+// channel o of the lift
+__device__ __forceinline__ float lift(const float *__restrict__ P, int o, float x0, float x1)
 {
-    i = c % g.X;
-    int r = c / g.X;
-    j = r % g.Y;
-    r /= g.Y;
-    k = r % g.Z;
-    t = r / g.Z;
+    return P[OFF_WL + o] * x0 + P[OFF_WL + C + o] * x1 + P[OFF_BL + o];
 }
 
-// tap m of a kind: space taps (dz, dy, dx) in {-1,0,1}^3 with dx fastest;
-// time taps dt in {-1, 0, 1}
-__device__ __forceinline__ void tap_offset(bool space, int m, int &dx, int &dy, int &dz, int &dt)
+// ---------------------------------------------------------------------------
+// The 3x3x3 space convolution.  Taps are d cells apart, so cells with equal
+// (y mod d, z mod d) form planes of their own; a workgroup owns TY = 8 such
+// rows of up to 64 x cells of one t step (`XW` wide, d columns of halo on each
+// side, zero outside the grid) and marches through the planes of its z class,
+// keeping three haloed planes in LDS as BF16 (the two 8-channel halves apart,
+// so that the 16 lanes of an operand read 256 contiguous bytes).  Every input
+// value is loaded about 1.25 times from memory and read 27 times from LDS;
+// the form that gathered the taps from memory read 27 x 64 bytes per cell
+// through the vector caches and rounded each value 27 times.
+// A wavefront computes 16-cell tiles of the XW x 8 outputs (positions are
+// numbered row by row, so ragged widths fill the tiles), 14 MFMA each, with
+// the weights in registers.
+struct SpaceGeo {
+    int X, Y, Z, T, d;
+    int nxt, XW;      // x tiles and their width
+    int nyt, nzs;     // y tiles per y class, z segments per z class
+    int zlen;         // planes per z segment
+    int pitch;        // XW + 2 d
+    int total;        // work items
+};
+constexpr int SP_W = 64, SP_DMAX = 8;
+template <int TY> struct SpLds {
+    static constexpr int ROWS = TY + 2;
+    static constexpr int HALF = ROWS * (SP_W + 2 * SP_DMAX) + 8;  // 16-byte slots of a half
+    static constexpr int LOADS = (2 * ROWS * (SP_W + 2 * SP_DMAX) + 255) / 256;
+};
+
+struct SpItem {
+    int x0, y0, ry, z0, z1, rz, t;  // first sub row y0 (rows ry + d yy), planes z0 .. z1 - 1
+};
+template <int TY>
+__device__ __forceinline__ bool sp_item(const SpaceGeo &S, int L, SpItem &w)
 {
-    if (space) {
-        dx = m % 3 - 1;
-        dy = (m / 3) % 3 - 1;
-        dz = m / 9 - 1;
-        dt = 0;
-    } else {
-        dx = dy = dz = 0;
-        dt = m - 1;
-    }
+    int r = L;
+    const int yt = r % S.nyt;
+    r /= S.nyt;
+    w.ry = r % S.d;
+    r /= S.d;
+    const int zs = r % S.nzs;
+    r /= S.nzs;
+    w.rz = r % S.d;
+    r /= S.d;
+    const int xt = r % S.nxt;
+    w.t = r / S.nxt;
+    w.x0 = xt * S.XW;
+    w.y0 = yt * TY;
+    w.z0 = zs * S.zlen;
+    const int zc = (S.Z - w.rz + S.d - 1) / S.d;  // planes of the class
+    w.z1 = min(w.z0 + S.zlen, zc);
+    return w.ry + S.d * w.y0 < S.Y && w.rz < S.Z && w.z0 < w.z1;
 }
 
-enum { EP_BIAS = 1, EP_RELU = 2, EP_MASK = 4, EP_RES = 8 };
-
-// out[c][o] = ep( sum_tap sum_i W[tap][i][o] in[c + sgn*off(tap)][i] )
-// with zero padding outside the grid; ep: (+ bias[o]) (relu) (* (mask > 0))
-// (+ res); out_relu (optional) receives max(out, 0) as well.  wf: packed A
-// fragments [pairs][64 lanes] (16 B each).
-template <bool SPACE>
-__global__ void __launch_bounds__(256)
-k_conv(const float *__restrict__ in, float *__restrict__ out, float *__restrict__ out_relu,
-       const bf16x8 *__restrict__ wf, const float *__restrict__ bias,
-       const float *__restrict__ mask, const float *__restrict__ res, Geo g, int sgn,
-       int flags)
+enum { SP_FWD = 0, SP_BWD = 1 };
+// SP_FWD: out_b = bf16(relu(conv + bias)) (a positive value never rounds to
+// zero, so its sign serves as the mask of the backward pass).
+// SP_BWD: out_f = res + conv, out_b = bf16(out_f), and the workgroup's column
+// sums of out_f (the gradient of the previous block's time bias).
+// NT: tiles per wavefront (the 8 rows hold up to 32 tiles of 16 positions)
+template <bool LIFT, int MODE, int NT>
+__global__ void __launch_bounds__(256, 2)
+k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
+        const float *__restrict__ i1, const float *__restrict__ P,
+        const bf16x8 *__restrict__ wf, const float *__restrict__ bias,
+        const float *__restrict__ res, float *__restrict__ out_f,
+        unsigned short *__restrict__ out_b, float *__restrict__ colsum, SpaceGeo S)
 {
-    constexpr int NT = SPACE ? NS : NTT;
-    const int dil = g.dil;
-    constexpr int NP = (NT + 1) / 2;
-    const int lane = threadIdx.x & 63;
-    const int grp = lane >> 4;       // 0..3
-    const int sub = grp >> 1;        // tap of the pair
-    const int half = grp & 1;        // input channels 8*half .. +7
-    const int waves = gridDim.x * (blockDim.x >> 6);
-    const int ntiles = (g.n + 15) >> 4;
-    for (int tile = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); tile < ntiles;
-         tile += waves) {
-        const int c = tile * 16 + (lane & 15);
-        const bool live = c < g.n;
-        int i = 0, j = 0, k = 0, t = 0;
-        if (live) cell_coords(g, c, i, j, k, t);
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-        for (int p = 0; p < NP; ++p) {
-            const int m = 2 * p + sub;
-            float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
-            if (live && m < NT) {
-                int dx, dy, dz, dt;
-                tap_offset(SPACE, m, dx, dy, dz, dt);
-                const int sd = sgn * dil;
-                const int ni = i + sd * dx, nj = j + sd * dy, nk = k + sd * dz,
-                          nt = t + sd * dt;
-                if (ni >= 0 && nj >= 0 && nk >= 0 && nt >= 0 && ni < g.X && nj < g.Y &&
-                    nk < g.Z && nt < g.T) {
-                    const int nc = ni + g.X * (nj + g.Y * (nk + g.Z * nt));
-                    const float4 *src = (const float4 *)(in + (int64_t)nc * C + 8 * half);
-                    lo = src[0];
-                    hi = src[1];
+    constexpr int TY = 8;
+    typedef SpLds<TY> L_;
+    __shared__ bf16x8 lds[3][2][L_::HALF];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int grp = lane >> 4, sub = grp >> 1, half = grp & 1;
+    const int per = (int)gridDim.x / FLOF_NXCD;  // the grid is a multiple of 8
+    const int L = ((int)blockIdx.x % FLOF_NXCD) * per + (int)blockIdx.x / FLOF_NXCD;
+    f32x4 cs = {0.f, 0.f, 0.f, 0.f};
+    SpItem w;
+    if (L < S.total && sp_item<TY>(S, L, w)) {  // uniform over the workgroup
+        const int d = S.d, pitch = S.pitch, X = S.X;
+        const int64_t plane = (int64_t)X * S.Y;
+        const int64_t tb = plane * S.Z * w.t;
+        bf16x8 wr[PAIRS_S];
+#pragma unroll
+        for (int p = 0; p < PAIRS_S; ++p) wr[p] = wf[p * 64 + lane];
+        // staged elements of this thread: 16-byte half sh of halo cells e; the
+        // two halves of a cell by neighbouring lanes, or (the lift, whose
+        // weights are then scalars of one half) by wavefronts
+        const int sh = LIFT ? __builtin_amdgcn_readfirstlane(wave >> 1) : tid & 1;
+        const int e0 = LIFT ? tid & 127 : tid >> 1;
+        int off[L_::LOADS];
+#pragma unroll
+        for (int m = 0; m < L_::LOADS; ++m) {
+            const int e = e0 + 128 * m;
+            const int row = e / pitch, x = w.x0 - d + (e - row * pitch);
+            const int y = w.ry + d * (w.y0 - 1 + row);
+            off[m] = row < L_::ROWS && x >= 0 && x < X && y >= 0 && y < S.Y ? x + X * y : -1;
+        }
+        const int nst = L_::ROWS * pitch;
+        bf16x8 st[L_::LOADS];
+        bool st_ok = false;
+        // loads are unconditional (cell 0 of the t step where the element lies
+        // outside the grid, replaced by zero when it is written to LDS)
+        auto fetch = [&](int zz) {
+            const int z = w.rz + d * zz;
+            const bool zok = zz >= 0 && z < S.Z;
+            const int64_t zb = tb + (zok ? plane * z : 0);
+            if (LIFT) {
+                float x0[L_::LOADS], x1[L_::LOADS];
+#pragma unroll
+                for (int m = 0; m < L_::LOADS; ++m) {
+                    const int o = max(off[m], 0);
+                    x0[m] = i0[zb + o] * 0.25f;
+                    x1[m] = i1[zb + o] * 0.25f;
+                }
+#pragma unroll
+                for (int m = 0; m < L_::LOADS; ++m) {
+                    float v[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) v[q] = lift(P, 8 * sh + q, x0[m], x1[m]);
+                    st[m] = pack8(make_float4(v[0], v[1], v[2], v[3]),
+                                  make_float4(v[4], v[5], v[6], v[7]));
+                }
+            } else {
+#pragma unroll
+                for (int m = 0; m < L_::LOADS; ++m)
+                    st[m] = __builtin_bit_cast(
+                        bf16x8,
+                        *(const u32x4 *)(inb + (zb + max(off[m], 0)) * C + 8 * sh));
+            }
+            st_ok = zok;
+        };
+        auto stash = [&](int zz) {
+            bf16x8 *s = lds[(zz + 3) % 3][sh];
+#pragma unroll
+            for (int m = 0; m < L_::LOADS; ++m) {
+                const int e = e0 + 128 * m;
+                if (e < nst) s[e] = st_ok && off[m] >= 0 ? st[m] : bf16x8{};
+            }
+        };
+        // the tiles of this wavefront: LDS slot of the lane's cell in a plane,
+        // and its offset in a grid plane (-1: not an output)
+        const int npos = TY * S.XW;
+        int base[NT], cell[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const int pos = (wave + 4 * j) * 16 + (lane & 15);
+            const int row = pos / S.XW, x = pos - row * S.XW;
+            const int y = w.ry + d * (w.y0 + row);
+            const bool ok = pos < npos && w.x0 + x < X && y < S.Y;
+            base[j] = (pos < npos ? (row + 1) * pitch + x + d : pitch + d) + half * L_::HALF;
+            cell[j] = ok ? w.x0 + x + X * y : -1;
+        }
+        fetch(w.z0 - 1);
+        stash(w.z0 - 1);
+        fetch(w.z0);
+        stash(w.z0);
+        fetch(w.z0 + 1);
+        const bf16x8 *flat = &lds[0][0][0];
+        for (int zz = w.z0; zz < w.z1; ++zz) {
+            __syncthreads();  // every wave is done with plane zz - 2's slot
+            stash(zz + 1);
+            __syncthreads();
+            if (zz + 1 < w.z1) fetch(zz + 2);
+            f32x4 acc[NT];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const int s0 = ((zz + 2) % 3) * 2 * L_::HALF, s1 = (zz % 3) * 2 * L_::HALF,
+                      s2 = ((zz + 1) % 3) * 2 * L_::HALF;
+#pragma unroll
+            for (int p = 0; p < PAIRS_S; ++p) {
+                auto tap = [&](int m) {
+                    return (m / 9 == 0 ? s0 : m / 9 == 1 ? s1 : s2) +
+                           (m / 3 % 3 - 1) * pitch + (m % 3 - 1) * d;
+                };
+                const int o = sub ? tap(2 * p + 1 < NS ? 2 * p + 1 : 2 * p) : tap(2 * p);
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    bf16x8 b = flat[base[j] + o];
+                    if (2 * p + 1 >= NS && sub) b = bf16x8{};  // the pair's missing tap
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[p], b, acc[j], 0, 0, 0);
                 }
             }
-            const bf16x8 b = pack8(lo, hi);
-            const bf16x8 a = wf[p * 64 + lane];
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-        }
-        if (!live) continue;
-        const int o0 = 4 * grp;
-        float v[4] = {acc[0], acc[1], acc[2], acc[3]};
-        const int64_t base = (int64_t)c * C + o0;
+            const int64_t zb = tb + plane * (w.rz + d * zz);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (flags & EP_BIAS) v[r] += bias[o0 + r];
-            if (flags & EP_RELU) v[r] = fmaxf(v[r], 0.f);
-            if (flags & EP_MASK) v[r] = mask[base + r] > 0.f ? v[r] : 0.f;
-            if (flags & EP_RES) v[r] += res[base + r];
+            for (int j = 0; j < NT; ++j) {
+                if (cell[j] < 0) continue;
+                const int64_t o = (zb + cell[j]) * C + 4 * grp;
+                f32x4 v = acc[j];
+                if (MODE == SP_FWD) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] += bias[4 * grp + r];
+                    u16x4 u;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        u[r] = to_bf16(fmaxf(v[r], 0.f));
+                        if (v[r] > 0.f && u[r] == 0) u[r] = 1;
+                    }
+                    *(u16x4 *)(out_b + o) = u;
+                } else {
+                    const f32x4 rs = *(const f32x4 *)(res + o);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        v[r] += rs[r];
+                        cs[r] += v[r];
+                    }
+                    *(f32x4 *)(out_f + o) = v;
+                    *(u16x4 *)(out_b + o) = pack4(v);
+                }
+            }
         }
-        *(float4 *)(out + base) = make_float4(v[0], v[1], v[2], v[3]);
-        if (out_relu)
-            *(float4 *)(out_relu + base) = make_float4(fmaxf(v[0], 0.f), fmaxf(v[1], 0.f),
-                                                       fmaxf(v[2], 0.f), fmaxf(v[3], 0.f));
+    }
+    if (MODE == SP_BWD) {
+        __shared__ float sh[4][C];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            for (int m = 8; m >= 1; m >>= 1) cs[r] += __shfl_xor(cs[r], m, 64);
+        if ((lane & 15) == 0)
+            for (int r = 0; r < 4; ++r) sh[wave][4 * grp + r] = cs[r];
+        __syncthreads();
+        if (tid < C)
+            colsum[(int64_t)blockIdx.x * C + tid] =
+                sh[0][tid] + sh[1][tid] + sh[2][tid] + sh[3][tid];
     }
 }
 
-// A fragments of a conv from W[tap][in][out] (FP32).  transpose: the
-// backward data pass, whose "out" channel is W's input channel.
+// ---------------------------------------------------------------------------
+// The 3-tap time convolution.  A wavefront owns 64 consecutive cells of the 3D
+// grid (four tiles of 16) and marches through the t steps of one class mod d,
+// the BF16 inputs at t - d, t, t + d in registers and the next one requested a
+// step ahead, so every input is read once.  MFMA 16x16x16, one tap each: a
+// lane's operand (4 channels of one cell) has the layout of the result, so
+// loads, residual and stores are all 8 or 16 bytes per lane of one contiguous
+// stretch.  Bound by memory: forward 32 + 64 bytes read and 64 + 32 written
+// per cell (64^4: 0.52 ms, 6.2 TB/s; 1.03 ms before, reading each input three
+// times in FP32).
+// TM_FWD: v = res + (conv + bias); out_f (optional) = v, out_b (optional) =
+// bf16(v); flow (optional) = the head of v, FP32 on the matrix cores
+// (16x16x4: the head's 4 outputs are rows 0..3 of the result).
+// TM_BWD: v = conv where the mask tensor is positive, else 0; out_b = bf16(v),
+// and the workgroup's column sums of v (the space bias gradient).
+enum { TM_FWD = 0, TM_BWD = 1 };
+struct TimeGeo {
+    int64_t n3;
+    int T, d;
+    int nch;         // stretches of 64 cells
+    int klen, nseg;  // steps of a class per segment, segments
+    int total;       // workgroups of 4 stretches: ceil(nch / 4) * d * nseg
+};
+template <bool LIFT, int MODE>
+__global__ void __launch_bounds__(256)
+k_time(const unsigned short *__restrict__ in, const s16x4 *__restrict__ wf,
+       const float *__restrict__ bias, const float *__restrict__ res, In lin,
+       const unsigned short *__restrict__ mask, float *__restrict__ out_f,
+       unsigned short *__restrict__ out_b, const float *__restrict__ P,
+       float4 *__restrict__ flow, float *__restrict__ colsum, TimeGeo G)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = lane >> 4;
+    const int nwg = (G.nch + 3) / 4;
+    int r_ = blockIdx.x;
+    const int ch = (r_ % nwg) * 4 + wave;
+    r_ /= nwg;
+    const int rt = r_ % G.d, seg = r_ / G.d;
+    f32x4 cs = {0.f, 0.f, 0.f, 0.f};
+    const int kc = (G.T - rt + G.d - 1) / G.d;  // steps of the class
+    const int k0 = seg * G.klen, k1 = min(k0 + G.klen, kc);
+    if (ch < G.nch && rt < G.T && k0 < k1) {
+        const s16x4 w0 = wf[lane], w1 = wf[64 + lane], w2 = wf[128 + lane];
+        f32x4 bs = {0.f, 0.f, 0.f, 0.f};
+        if (MODE == TM_FWD)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) bs[r] = bias[4 * grp + r];
+        float wh[4];
+        f32x4 bh = {0.f, 0.f, 0.f, 0.f};
+        if (flow) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                wh[r] = (lane & 15) < 4 ? P[OFF_WH + (4 * grp + r) * 4 + (lane & 15)] : 0.f;
+                bh[r] = grp == 0 ? P[OFF_BH + r] : 0.f;
+            }
+        }
+        float l0[4], l1[4], lb[4];
+        if (LIFT) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                l0[r] = P[OFF_WL + 4 * grp + r];
+                l1[r] = P[OFF_WL + C + 4 * grp + r];
+                lb[r] = P[OFF_BL + 4 * grp + r];
+            }
+        }
+        int64_t c3[4];
+        bool ok[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            c3[j] = (int64_t)ch * 64 + 16 * j + (lane & 15);
+            ok[j] = c3[j] < G.n3;
+            if (!ok[j]) c3[j] = 0;
+        }
+        s16x4 am[4], ac[4], ap[4];
+        auto load = [&](s16x4 (&a)[4], int k) {
+            const int t = rt + G.d * k;
+            const bool in_t = k >= 0 && t < G.T;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                a[j] = s16x4{0, 0, 0, 0};
+                if (in_t) a[j] = *(const s16x4 *)(in + (c3[j] + G.n3 * t) * C + 4 * grp);
+            }
+        };
+        load(am, k0 - 1);
+        load(ac, k0);
+        load(ap, k0 + 1);
+        for (int k = k0; k < k1; ++k) {
+            const int t = rt + G.d * k;
+            s16x4 an[4];
+            if (k + 1 < k1) load(an, k + 2);
+            f32x4 rs[4];
+            s16x4 mk[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t c = c3[j] + G.n3 * t;
+                if (MODE == TM_BWD) {
+                    mk[j] = *(const s16x4 *)(mask + c * C + 4 * grp);
+                } else if (LIFT) {
+                    const float x0 = lin.i0[c] * 0.25f, x1 = lin.i1[c] * 0.25f;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) rs[j][r] = l0[r] * x0 + l1[r] * x1 + lb[r];
+                } else {
+                    rs[j] = *(const f32x4 *)(res + c * C + 4 * grp);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                f32x4 v = {0.f, 0.f, 0.f, 0.f};
+                v = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w0, am[j], v, 0, 0, 0);
+                v = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w1, ac[j], v, 0, 0, 0);
+                v = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w2, ap[j], v, 0, 0, 0);
+                const int64_t c = c3[j] + G.n3 * t;
+                if (MODE == TM_FWD) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = (v[r] + bs[r]) + rs[j][r];
+                    if (ok[j]) {
+                        if (out_f) *(f32x4 *)(out_f + c * C + 4 * grp) = v;
+                        if (out_b) *(u16x4 *)(out_b + c * C + 4 * grp) = pack4(v);
+                    }
+                    if (flow) {
+                        f32x4 f = bh;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            f = __builtin_amdgcn_mfma_f32_16x16x4f32(wh[r], v[r], f, 0, 0, 0);
+                        if (ok[j] && grp == 0) flow[c] = make_float4(f[0], f[1], f[2], f[3]);
+                    }
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        if (!(mk[j][r] > 0)) v[r] = 0.f;  // bf16 sign and zero as int16
+                        if (ok[j]) cs[r] += v[r];
+                    }
+                    if (ok[j]) *(u16x4 *)(out_b + c * C + 4 * grp) = pack4(v);
+                }
+                am[j] = ac[j];
+                ac[j] = ap[j];
+                ap[j] = an[j];
+            }
+        }
+    }
+    if (MODE == TM_BWD) {
+        __shared__ float sh[4][C];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            for (int m = 8; m >= 1; m >>= 1) cs[r] += __shfl_xor(cs[r], m, 64);
+        if ((lane & 15) == 0)
+            for (int r = 0; r < 4; ++r) sh[wave][4 * grp + r] = cs[r];
+        __syncthreads();
+        if (tid < C)
+            colsum[(int64_t)blockIdx.x * C + tid] =
+                sh[0][tid] + sh[1][tid] + sh[2][tid] + sh[3][tid];
+    }
+}
+
+// A fragments of a space conv (16x16x32, two taps) from W[tap][in][out]
+// (FP32).  transpose: the backward data pass, whose "out" channel is W's
+// input channel and whose taps are mirrored.
 __global__ void k_pack_frag(const float *__restrict__ W, bf16x8 *__restrict__ wf, int ntaps,
                             int npairs, int transpose)
 {
@@ -199,145 +505,314 @@ __global__ void k_pack_frag(const float *__restrict__ W, bf16x8 *__restrict__ wf
     for (int q = 0; q < 8; ++q) {
         const int ii = 8 * (grp & 1) + q;
         float w = 0.f;
-        if (m < ntaps) w = transpose ? W[(m * C + o) * C + ii] : W[(m * C + ii) * C + o];
+        if (m < ntaps)
+            w = transpose ? W[((ntaps - 1 - m) * C + o) * C + ii] : W[(m * C + ii) * C + o];
         v[q] = w;
     }
     wf[idx] = pack8(make_float4(v[0], v[1], v[2], v[3]), make_float4(v[4], v[5], v[6], v[7]));
 }
-
-// weight gradient of a forward conv (sgn +1):
-//   dW[tap][i][o] = sum_c bf16(in[c + off(tap)][i]) * bf16(dout[c][o])
-// D = A B with A (16 x 32) = in^T over 32 cells, B (32 x 16) = dout over the
-// same cells; each wavefront accumulates taps M0 .. M0+NT-1 over its cells
-// and writes one partial [tap][16][16] (taps of one launch: at most 9, so
-// the accumulators stay in registers).
-template <bool SPACE, int M0, int NT>
-__global__ void __launch_bounds__(256)
-k_conv_wgrad(const float *__restrict__ in, const float *__restrict__ dout,
-             float *__restrict__ part, Geo g)
+// the same for the time conv (16x16x16, one tap)
+__global__ void k_pack_frag_t(const float *__restrict__ W, s16x4 *__restrict__ wf, int transpose)
 {
-    const int lane = threadIdx.x & 63;
-    const int grp = lane >> 4;
-    const int ch = lane & 15;
-    const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int waves = gridDim.x * (blockDim.x >> 6);
-    f32x4 acc[NT];
+    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= NTT * 64) return;
+    const int m = idx >> 6, lane = idx & 63;
+    const int o = lane & 15, grp = lane >> 4;
+    u16x4 u;
+    for (int q = 0; q < 4; ++q) {
+        const int ii = 4 * grp + q;
+        u[q] = to_bf16(transpose ? W[((NTT - 1 - m) * C + o) * C + ii] : W[(m * C + ii) * C + o]);
+    }
+    wf[idx] = __builtin_bit_cast(s16x4, u);
+}
+
+// ---------------------------------------------------------------------------
+// Weight gradients, dW[tap][i][o] = sum_c in[c + off(tap)][i] dout[c][o] with
+// the cells as the reduction dimension of MFMA 16x16x16: an operand is 4
+// consecutive x cells of one channel, so the tiles are staged channel by
+// channel in LDS.
+// Space: tiles, classes and march of k_space with TY = 4 rows; the 27
+// accumulators of a wavefront (108 registers) live through all of its work
+// items, and the lanes' quads of x cells give three taps at once where their
+// ranges overlap (d = 1: 12 bytes, d = 2: 16 bytes instead of 24).  At
+// 50x46x44x40: 0.19-0.24 ms per convolution, where gathering every operand
+// value from memory in three launches of 9 taps took 2.95 ms.
+template <int TY> struct WgLds {
+    static constexpr int ROWS = TY + 2;
+    static constexpr int PITCH = SP_W + 2 * SP_DMAX + 4;
+    // bytes of one channel; odd multiples of 32 spread the 16 channels over the banks
+    static constexpr int CH = (3 * ROWS * PITCH * 2 + 31) / 64 * 64 + 32;
+    static constexpr int DCH = (TY * SP_W * 2) / 64 * 64 + 32;
+};
+template <bool LIFT, int D>
+__global__ void __launch_bounds__(256)
+k_wgrad_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
+              const float *__restrict__ i1, const float *__restrict__ P,
+              const unsigned short *__restrict__ dout, float *__restrict__ part, SpaceGeo S)
+{
+    constexpr int TY = 4;
+    typedef WgLds<TY> L_;
+    constexpr int LOADS = (2 * L_::ROWS * (SP_W + 2 * SP_DMAX) + 255) / 256;
+    constexpr int DLOADS = (2 * TY * SP_W + 255) / 256;
+    static_assert(3 * L_::ROWS * L_::PITCH * 2 <= L_::CH && TY * SP_W * 2 <= L_::DCH, "");
+    __shared__ __attribute__((aligned(16))) char li[C * L_::CH];
+    __shared__ __attribute__((aligned(16))) char ld[C * L_::DCH];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int grp = lane >> 4, ch = lane & 15;
+    const int d = D > 0 ? D : S.d, X = S.X;
+    // a multiple of 4 columns: the quads' reads stay 8-byte aligned
+    const int pitch = (S.XW + 3) / 4 * 4 + max(4, 2 * d);
+    const int64_t plane = (int64_t)X * S.Y;
+    f32x4 acc[NS];
 #pragma unroll
-    for (int m = 0; m < NT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int nchunks = (g.n + 31) >> 5;
-    for (int chunk = wave; chunk < nchunks; chunk += waves) {
-        int ci[8], cj[8], ck[8], ct[8];
-        bool live[8];
-        float bo[8];
+    for (int m = 0; m < NS; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int qx = (S.XW + 3) / 4;  // quads per row
+    const int nq = TY * qx;
+    for (int L = blockIdx.x; L < S.total; L += gridDim.x) {
+        SpItem w;
+        if (!sp_item<TY>(S, L, w)) continue;  // uniform over the workgroup
+        const int64_t tb = plane * S.Z * w.t;
+        const int sh = LIFT ? __builtin_amdgcn_readfirstlane(wave >> 1) : tid & 1;
+        const int e0 = LIFT ? tid & 127 : tid >> 1;
+        int off[LOADS], dof[DLOADS];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int c = chunk * 32 + 8 * grp + q;
-            live[q] = c < g.n;
-            ci[q] = cj[q] = ck[q] = ct[q] = 0;
-            if (live[q]) cell_coords(g, c, ci[q], cj[q], ck[q], ct[q]);
-            bo[q] = live[q] ? dout[(int64_t)c * C + ch] : 0.f;
+        for (int m = 0; m < LOADS; ++m) {
+            const int e = e0 + 128 * m;
+            const int row = e / pitch, x = w.x0 - d + (e - row * pitch);
+            const int y = w.ry + d * (w.y0 - 1 + row);
+            off[m] = row < L_::ROWS && x >= 0 && x < X && y >= 0 && y < S.Y ? x + X * y : -1;
         }
-        const bf16x8 b = pack8(make_float4(bo[0], bo[1], bo[2], bo[3]),
-                               make_float4(bo[4], bo[5], bo[6], bo[7]));
 #pragma unroll
-        for (int m = 0; m < NT; ++m) {
-            int dx, dy, dz, dt;
-            tap_offset(SPACE, M0 + m, dx, dy, dz, dt);
-            float av[8];
+        for (int m = 0; m < DLOADS; ++m) {
+            const int e = (tid + 256 * m) >> 1;
+            const int row = e / (4 * qx), x = e - row * (4 * qx);
+            const int y = w.ry + d * (w.y0 + row);
+            dof[m] = row < TY && x < S.XW && w.x0 + x < X && y < S.Y ? w.x0 + x + X * y : -1;
+        }
+        const int nst = L_::ROWS * pitch, ndst = 2 * TY * 4 * qx;
+        u16x8 st[LOADS], sd[DLOADS];
+        bool st_ok = false;
+        auto fetch = [&](int zz) {
+            const int z = w.rz + d * zz;
+            st_ok = zz >= 0 && z < S.Z;
+            const int64_t zb = tb + (st_ok ? plane * z : 0);
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int ni = ci[q] + g.dil * dx, nj = cj[q] + g.dil * dy,
-                          nk = ck[q] + g.dil * dz, nt = ct[q] + g.dil * dt;
-                av[q] = (live[q] && ni >= 0 && nj >= 0 && nk >= 0 && nt >= 0 && ni < g.X &&
-                         nj < g.Y && nk < g.Z && nt < g.T)
-                            ? in[(int64_t)(ni + g.X * (nj + g.Y * (nk + g.Z * nt))) * C + ch]
-                            : 0.f;
+            for (int m = 0; m < LOADS; ++m) {
+                const int64_t c = zb + max(off[m], 0);
+                if (LIFT) {
+                    const float x0 = i0[c] * 0.25f, x1 = i1[c] * 0.25f;
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) st[m][q] = to_bf16(lift(P, 8 * sh + q, x0, x1));
+                } else {
+                    st[m] = *(const u16x8 *)(inb + c * C + 8 * sh);
+                }
             }
-            const bf16x8 a = pack8(make_float4(av[0], av[1], av[2], av[3]),
-                                   make_float4(av[4], av[5], av[6], av[7]));
-            acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[m], 0, 0, 0);
+        };
+        auto fetch_d = [&](int zz) {
+            const int64_t zb = tb + plane * (w.rz + d * zz);
+#pragma unroll
+            for (int m = 0; m < DLOADS; ++m)
+                sd[m] = *(const u16x8 *)(dout + (zb + max(dof[m], 0)) * C + 8 * (tid & 1));
+        };
+        auto stash = [&](int zz) {
+            const int so = ((zz + 3) % 3) * L_::ROWS * pitch;
+#pragma unroll
+            for (int m = 0; m < LOADS; ++m) {
+                const int e = e0 + 128 * m;
+                if (!(st_ok && off[m] >= 0)) st[m] = u16x8{};
+                if (e < nst) {
+                    char *p = li + 8 * sh * L_::CH + (so + e) * 2;
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) *(unsigned short *)(p + q * L_::CH) = st[m][q];
+                }
+            }
+        };
+        auto stash_d = [&]() {
+#pragma unroll
+            for (int m = 0; m < DLOADS; ++m) {
+                const int e = tid + 256 * m;
+                if (dof[m] < 0) sd[m] = u16x8{};
+                if (e < ndst) {
+                    char *p = ld + 8 * (tid & 1) * L_::DCH + (e >> 1) * 2;
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) *(unsigned short *)(p + q * L_::DCH) = sd[m][q];
+                }
+            }
+        };
+        __syncthreads();  // the previous item's last step has been read
+        fetch(w.z0 - 1);
+        stash(w.z0 - 1);
+        fetch(w.z0);
+        stash(w.z0);
+        fetch(w.z0 + 1);
+        fetch_d(w.z0);
+        for (int zz = w.z0; zz < w.z1; ++zz) {
+            if (zz > w.z0) __syncthreads();  // every wave is done with the last step
+            stash(zz + 1);
+            stash_d();
+            __syncthreads();
+            if (zz + 1 < w.z1) {
+                fetch(zz + 2);
+                fetch_d(zz + 1);
+            }
+            for (int q0 = wave * 4; q0 < nq; q0 += 16) {
+                const int q = q0 + grp;
+                const bool ok = q < nq;
+                const int row = ok ? q / qx : 0, x = ok ? 4 * (q - row * qx) : 0;
+                s16x4 b = *(const s16x4 *)(ld + ch * L_::DCH + (row * 4 * qx + x) * 2);
+                if (!ok) b = s16x4{0, 0, 0, 0};
+#pragma unroll
+                for (int r = 0; r < 9; ++r) {
+                    const int slot = (zz + r / 3 + 2) % 3;
+                    const char *p = li + ch * L_::CH +
+                                    ((slot * L_::ROWS + row + r % 3) * pitch + x) * 2;
+                    s16x4 a0, a1, a2;
+                    if (D == 1) {
+                        const uint2 u = *(const uint2 *)p;
+                        const unsigned v = *(const unsigned *)(p + 8);
+                        a0 = __builtin_bit_cast(s16x4, u);
+                        a1 = __builtin_bit_cast(
+                            s16x4, make_uint2(__builtin_amdgcn_alignbit(u.y, u.x, 16),
+                                              __builtin_amdgcn_alignbit(v, u.y, 16)));
+                        a2 = __builtin_bit_cast(s16x4, make_uint2(u.y, v));
+                    } else if (D == 2) {
+                        const uint2 u = *(const uint2 *)p, v = *(const uint2 *)(p + 8);
+                        a0 = __builtin_bit_cast(s16x4, u);
+                        a1 = __builtin_bit_cast(s16x4, make_uint2(u.y, v.x));
+                        a2 = __builtin_bit_cast(s16x4, v);
+                    } else {
+                        a0 = *(const s16x4 *)p;
+                        a1 = *(const s16x4 *)(p + 2 * d);
+                        a2 = *(const s16x4 *)(p + 4 * d);
+                    }
+                    acc[3 * r] =
+                        __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, b, acc[3 * r], 0, 0, 0);
+                    acc[3 * r + 1] =
+                        __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, b, acc[3 * r + 1], 0, 0, 0);
+                    acc[3 * r + 2] =
+                        __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a2, b, acc[3 * r + 2], 0, 0, 0);
+                }
+            }
         }
     }
-    // D[i][o]: lane holds i = 4*grp + r, o = lane % 16
-    float *dst = part + (int64_t)wave * NT * C * C;
+    // D[i][o]: lane holds i = 4 grp + r, o = lane % 16
+    float *dst = part + ((int64_t)blockIdx.x * 4 + wave) * NS * C * C;
 #pragma unroll
-    for (int m = 0; m < NT; ++m)
+    for (int m = 0; m < NS; ++m)
 #pragma unroll
         for (int r = 0; r < 4; ++r) dst[(m * C + 4 * grp + r) * C + ch] = acc[m][r];
 }
 
-// rows x cols partial sums -> one row (sum over rows), one thread per column
-__global__ void k_sum_rows(const float *__restrict__ part, int rows, int cols,
-                           float *__restrict__ dst, int accumulate)
-{
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= cols) return;
-    double s = 0.;
-    for (int r = 0; r < rows; ++r) s += (double)part[(int64_t)r * cols + col];
-    dst[col] = accumulate ? dst[col] + (float)s : (float)s;
-}
-
-// per-block column sums of a [n][cols] tensor (bias gradients etc.)
+// Time: a wavefront takes the stretches and t classes of k_time in turn; a
+// step's input (t + d) and dout (t) go channel by channel through its own
+// LDS rows (read back by the same wavefront), the inputs at t - d and t stay
+// in registers.
+constexpr int WT_ROW = 64 * 2 + 16;  // bytes of one channel's 64 cells
 __global__ void __launch_bounds__(256)
-k_col_partials(const float *__restrict__ a, int n, int cols, float *__restrict__ part)
+k_wgrad_time(const unsigned short *__restrict__ in, const unsigned short *__restrict__ dout,
+             float *__restrict__ part, TimeGeo G)
 {
-    // blockDim 256 = 16 rows x 16 columns; cols <= 16
-    const int col = threadIdx.x & 15;
-    const int row0 = threadIdx.x >> 4;
-    float s = 0.f;
-    if (col < cols)
-        for (int r = blockIdx.x * 16 + row0; r < n; r += gridDim.x * 16)
-            s += a[(int64_t)r * cols + col];
-    __shared__ float sh[256];
-    sh[threadIdx.x] = s;
+    __shared__ __attribute__((aligned(16))) char lds[4][2][C * WT_ROW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int grp = lane >> 4, ch = lane & 15;
+    f32x4 acc[NTT];
+#pragma unroll
+    for (int m = 0; m < NTT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int items = G.nch * G.d * G.nseg;
+    for (int it = blockIdx.x * 4 + wave; it < items; it += gridDim.x * 4) {
+        int r_ = it;
+        const int chn = r_ % G.nch;
+        r_ /= G.nch;
+        const int rt = r_ % G.d, seg = r_ / G.d;
+        const int kc = (G.T - rt + G.d - 1) / G.d;
+        const int k0 = seg * G.klen, k1 = min(k0 + G.klen, kc);
+        if (rt >= G.T || k0 >= k1) continue;
+        // cells of this lane's two 16-byte halves: lane >> 1 and 32 + (lane >> 1)
+        const int64_t cb = (int64_t)chn * 64;
+        auto load = [&](const unsigned short *src, u16x8 (&v)[2], int k) {
+            const int t = rt + G.d * k;
+            const bool in_t = k >= 0 && t < G.T;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int64_t c = cb + 32 * j + (lane >> 1);
+                v[j] = u16x8{};
+                if (in_t && c < G.n3)
+                    v[j] = *(const u16x8 *)(src + (c + G.n3 * t) * C + 8 * (lane & 1));
+            }
+        };
+        // through the wavefront's own rows (its lanes run in step; the waits
+        // on LDS order the writes and the reads)
+        auto turn = [&](const u16x8 (&v)[2], s16x4 (&o)[4], int slot) {
+            char *p = lds[wave][slot];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    *(unsigned short *)(p + (8 * (lane & 1) + q) * WT_ROW +
+                                        (32 * j + (lane >> 1)) * 2) = v[j][q];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                o[j] = *(const s16x4 *)(p + ch * WT_ROW + (16 * j + 4 * grp) * 2);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        };
+        u16x8 raw[2], rawd[2];
+        s16x4 am[4], ac[4], ap[4], b[4];
+        load(in, raw, k0 - 1);
+        turn(raw, am, 0);
+        load(in, raw, k0);
+        turn(raw, ac, 0);
+        load(in, raw, k0 + 1);
+        load(dout, rawd, k0);
+        for (int k = k0; k < k1; ++k) {
+            turn(raw, ap, 0);
+            turn(rawd, b, 1);
+            if (k + 1 < k1) {
+                load(in, raw, k + 2);
+                load(dout, rawd, k + 1);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                acc[0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(am[j], b[j], acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ac[j], b[j], acc[1], 0, 0, 0);
+                acc[2] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ap[j], b[j], acc[2], 0, 0, 0);
+                am[j] = ac[j];
+                ac[j] = ap[j];
+            }
+        }
+    }
+    float *dst = part + ((int64_t)blockIdx.x * 4 + wave) * NTT * C * C;
+#pragma unroll
+    for (int m = 0; m < NTT; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dst[(m * C + 4 * grp + r) * C + ch] = acc[m][r];
+}
+
+// rows x cols partial sums -> one row (FP64 sum over rows): a workgroup takes
+// 16 columns with 16 row lanes each, so that few columns of many rows do not
+// run as one serial chain (one thread per column took 355 us per call on
+// average in a training step, this takes 12)
+__global__ void __launch_bounds__(256)
+k_sum_rows(const float *__restrict__ part, int rows, int cols, float *__restrict__ dst)
+{
+    __shared__ double sh[16][17];
+    const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4;
+    const int col = blockIdx.x * 16 + cl;
+    double s = 0.;
+    if (col < cols) {
+#pragma unroll 8
+        for (int r = rl; r < rows; r += 16) s += (double)part[(int64_t)r * cols + col];
+    }
+    sh[rl][cl] = s;
     __syncthreads();
-    if (threadIdx.x < 16) {
-        float t = 0.f;
-        for (int q = 0; q < 16; ++q) t += sh[q * 16 + threadIdx.x];
-        if (threadIdx.x < cols) part[(int64_t)blockIdx.x * cols + threadIdx.x] = t;
-    }
-}
-
-// h0[c][o] = Wl[0][o] * i0/4 + Wl[1][o] * i1/4 + bl[o]
-__global__ void k_lift(const float *__restrict__ i0, const float *__restrict__ i1,
-                       const float *__restrict__ P, float *__restrict__ h, int n)
-{
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
-        const float x0 = i0[c] * 0.25f, x1 = i1[c] * 0.25f;
-        float v[C];
-#pragma unroll
-        for (int o = 0; o < C; ++o)
-            v[o] = P[OFF_WL + o] * x0 + P[OFF_WL + C + o] * x1 + P[OFF_BL + o];
-        float4 *d = (float4 *)(h + (int64_t)c * C);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) d[q] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
-    }
-}
-
-// flow[c][d] = sum_i Wh[i][d] h[c][i] + bh[d]
-__global__ void k_head(const float *__restrict__ h, const float *__restrict__ P,
-                       float4 *__restrict__ flow, int n)
-{
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
-        const float4 *s = (const float4 *)(h + (int64_t)c * C);
-        float hv[C];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 t = s[q];
-            hv[4 * q] = t.x;
-            hv[4 * q + 1] = t.y;
-            hv[4 * q + 2] = t.z;
-            hv[4 * q + 3] = t.w;
-        }
-        float o[4];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            float a = P[OFF_BH + d];
-#pragma unroll
-            for (int i = 0; i < C; ++i) a += P[OFF_WH + i * 4 + d] * hv[i];
-            o[d] = a;
-        }
-        flow[c] = make_float4(o[0], o[1], o[2], o[3]);
+    if (rl == 0 && col < cols) {
+        double t = 0.;
+        for (int q = 0; q < 16; ++q) t += sh[q][cl];
+        dst[col] = (float)t;
     }
 }
 
@@ -365,47 +840,63 @@ k_loss(const float4 *__restrict__ flow, const float4 *__restrict__ tgt,
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-// head backward: dh[c][i] = sum_d Wh[i][d] dy[c][d]; per-block partials of
-// dWh[i][d] = sum_c h[c][i] dy[c][d] (64) and dbh[d] = sum_c dy[c][d] (4)
+// sums of the workgroup's v[0 .. N-1], one row of N partials (lane sums by
+// shuffles, then the four wavefronts through LDS)
+template <int N> __device__ __forceinline__ void block_cols(float (&v)[N], float *dst)
+{
+    __shared__ float sh[4][N];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        for (int m = 32; m >= 1; m >>= 1) v[q] += __shfl_xor(v[q], m, 64);
+        if (lane == 0) sh[wave][q] = v[q];
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < N; q += blockDim.x)
+        dst[q] = sh[0][q] + sh[1][q] + sh[2][q] + sh[3][q];
+}
+
+// head backward: dh[c][i] = sum_d Wh[i][d] dy[c][d], FP32 and BF16; per-block
+// partials of dWh[i][d] = sum_c h[c][i] dy[c][d] (64), dbh[d] = sum_c dy[c][d]
+// (4) and sum_c dh[c][i] (16, the last block's time bias)
+constexpr int HEAD_COLS = C * 4 + 4 + C;
 __global__ void __launch_bounds__(256)
 k_head_bwd(const float *__restrict__ h, const float4 *__restrict__ dy,
-           const float *__restrict__ P, float *__restrict__ dh, int n,
-           float *__restrict__ part)
+           const float *__restrict__ P, float *__restrict__ dh,
+           unsigned short *__restrict__ dhb, int n, float *__restrict__ part)
 {
-    float gw[C * 4], gb[4];
+    float g[HEAD_COLS];
 #pragma unroll
-    for (int q = 0; q < C * 4; ++q) gw[q] = 0.f;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) gb[d] = 0.f;
+    for (int q = 0; q < HEAD_COLS; ++q) g[q] = 0.f;
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
         const float4 e = dy[c];
         const float ev[4] = {e.x, e.y, e.z, e.w};
-        const float *hc = h + (int64_t)c * C;
-        float *dc = dh + (int64_t)c * C;
+        const f32x4 *hc = (const f32x4 *)(h + (int64_t)c * C);
+        f32x4 *dc = (f32x4 *)(dh + (int64_t)c * C);
+        u16x4 *db = (u16x4 *)(dhb + (int64_t)c * C);
 #pragma unroll
-        for (int i = 0; i < C; ++i) {
-            float a = 0.f;
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 hv = hc[q];
+            f32x4 o;
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                a += P[OFF_WH + i * 4 + d] * ev[d];
-                gw[i * 4 + d] += hc[i] * ev[d];
+            for (int r = 0; r < 4; ++r) {
+                const int i = 4 * q + r;
+                float a = 0.f;
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    a += P[OFF_WH + i * 4 + d] * ev[d];
+                    g[i * 4 + d] += hv[r] * ev[d];
+                }
+                o[r] = a;
+                g[C * 4 + 4 + i] += a;
             }
-            dc[i] = a;
+            dc[q] = o;
+            db[q] = pack4(o);
         }
 #pragma unroll
-        for (int d = 0; d < 4; ++d) gb[d] += ev[d];
+        for (int d = 0; d < 4; ++d) g[C * 4 + d] += ev[d];
     }
-    __shared__ float sh[256];
-    for (int q = 0; q < C * 4 + 4; ++q) {
-        sh[threadIdx.x] = q < C * 4 ? gw[q] : gb[q - C * 4];
-        __syncthreads();
-        for (int w = 128; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) part[(int64_t)blockIdx.x * (C * 4 + 4) + q] = sh[0];
-        __syncthreads();
-    }
+    block_cols<HEAD_COLS>(g, part + (int64_t)blockIdx.x * HEAD_COLS);
 }
 
 // lift backward: per-block partials of dWl[k][o] = sum_c x_k[c] dh0[c][o]
@@ -414,32 +905,25 @@ __global__ void __launch_bounds__(256)
 k_lift_bwd(const float *__restrict__ i0, const float *__restrict__ i1,
            const float *__restrict__ dh, int n, float *__restrict__ part)
 {
-    float gw[2 * C], gb[C];
+    float g[3 * C];
 #pragma unroll
-    for (int q = 0; q < 2 * C; ++q) gw[q] = 0.f;
-#pragma unroll
-    for (int q = 0; q < C; ++q) gb[q] = 0.f;
+    for (int q = 0; q < 3 * C; ++q) g[q] = 0.f;
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
         const float x0 = i0[c] * 0.25f, x1 = i1[c] * 0.25f;
-        const float *d = dh + (int64_t)c * C;
+        const f32x4 *d = (const f32x4 *)(dh + (int64_t)c * C);
 #pragma unroll
-        for (int o = 0; o < C; ++o) {
-            gw[o] += x0 * d[o];
-            gw[C + o] += x1 * d[o];
-            gb[o] += d[o];
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 v = d[q];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int o = 4 * q + r;
+                g[o] += x0 * v[r];
+                g[C + o] += x1 * v[r];
+                g[2 * C + o] += v[r];
+            }
         }
     }
-    __shared__ float sh[256];
-    for (int q = 0; q < 3 * C; ++q) {
-        sh[threadIdx.x] = q < 2 * C ? gw[q] : gb[q - 2 * C];
-        __syncthreads();
-        for (int w = 128; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) part[(int64_t)blockIdx.x * (3 * C) + q] = sh[0];
-        __syncthreads();
-    }
+    block_cols<3 * C>(g, part + (int64_t)blockIdx.x * 3 * C);
 }
 
 __global__ void k_adam(float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m,
@@ -474,8 +958,9 @@ struct flof_warmnet {
 
 namespace {
 
-constexpr int FRAG_S = PAIRS_S * 64, FRAG_T = PAIRS_T * 64;
-// fragment slots per block: space fwd, space bwd, time fwd, time bwd
+// 16-byte fragment slots per block: space fwd, space bwd, time fwd, time bwd
+// (the time fragments are 8 bytes per lane)
+constexpr int FRAG_S = PAIRS_S * 64, FRAG_T = NTT * 64 / 2;
 constexpr int FRAG_BLK = 2 * FRAG_S + 2 * FRAG_T;
 
 void pack_all(flof_warmnet *net)
@@ -488,10 +973,10 @@ void pack_all(flof_warmnet *net)
                            blk + BLK_WS, f, NS, PAIRS_S, 0);
         hipLaunchKernelGGL(k_pack_frag, dim3((FRAG_S + 255) / 256), dim3(256), 0, ctx->stream,
                            blk + BLK_WS, f + FRAG_S, NS, PAIRS_S, 1);
-        hipLaunchKernelGGL(k_pack_frag, dim3(1), dim3(256), 0, ctx->stream, blk + BLK_WT,
-                           f + 2 * FRAG_S, NTT, PAIRS_T, 0);
-        hipLaunchKernelGGL(k_pack_frag, dim3(1), dim3(256), 0, ctx->stream, blk + BLK_WT,
-                           f + 2 * FRAG_S + FRAG_T, NTT, PAIRS_T, 1);
+        hipLaunchKernelGGL(k_pack_frag_t, dim3(1), dim3(256), 0, ctx->stream, blk + BLK_WT,
+                           (s16x4 *)(f + 2 * FRAG_S), 0);
+        hipLaunchKernelGGL(k_pack_frag_t, dim3(1), dim3(256), 0, ctx->stream, blk + BLK_WT,
+                           (s16x4 *)(f + 2 * FRAG_S + FRAG_T), 1);
     }
     check_launch("k_pack_frag");
     net->frag_ok = true;
@@ -503,55 +988,130 @@ Geo geo_of(const flof_grid4d *g)
     return Geo{g->X, g->Y, g->Z, g->T, (int)g->n(), 1};
 }
 
-int conv_blocks(flof_ctx *ctx, int n)
+// tiles of a space conv with ty rows per workgroup; z segments of at least 4
+// planes, as many as give the chip about `want` workgroups
+SpaceGeo space_geo(const Geo &g, int ty, int want)
 {
-    const int tiles = (n + 15) / 16;
-    return std::max(1, std::min((tiles + 3) / 4, ctx->num_cu * 8));
+    SpaceGeo S;
+    S.X = g.X;
+    S.Y = g.Y;
+    S.Z = g.Z;
+    S.T = g.T;
+    S.d = g.dil;
+    S.nxt = (g.X + SP_W - 1) / SP_W;
+    S.XW = (g.X + S.nxt - 1) / S.nxt;
+    S.nyt = ((g.Y + g.dil - 1) / g.dil + ty - 1) / ty;
+    const int zc = (g.Z + g.dil - 1) / g.dil;
+    const int64_t cols = (int64_t)g.T * S.nxt * S.nyt * g.dil * g.dil;
+    const int most = std::max(1, zc / 4);
+    S.nzs = (int)std::max<int64_t>(1, std::min<int64_t>(most, (want + cols - 1) / cols));
+    S.zlen = (zc + S.nzs - 1) / S.nzs;
+    S.nzs = (zc + S.zlen - 1) / S.zlen;
+    S.pitch = S.XW + 2 * g.dil;
+    FLOF_REQUIRE(cols * S.nzs < (1ll << 31), FLOF_ERR_DIM, "warm-start net: grid too large");
+    S.total = (int)(cols * S.nzs);
+    return S;
+}
+int space_blocks(const SpaceGeo &S)
+{
+    return (S.total + FLOF_NXCD - 1) / FLOF_NXCD * FLOF_NXCD;
+}
+// stretches and t classes of a time conv; segments of at least 4 steps, as
+// many as give the chip about 8192 wavefronts
+TimeGeo time_geo(const Geo &g)
+{
+    TimeGeo G;
+    G.n3 = (int64_t)g.X * g.Y * g.Z;
+    G.T = g.T;
+    G.d = g.dil;
+    G.nch = (int)((G.n3 + 63) / 64);
+    const int kc = (g.T + g.dil - 1) / g.dil;
+    const int64_t cols = (int64_t)G.nch * g.dil;
+    G.nseg = (int)std::max<int64_t>(
+        1, std::min<int64_t>(std::max(1, kc / 4), (8192 + cols - 1) / cols));
+    G.klen = (kc + G.nseg - 1) / G.nseg;
+    G.nseg = (kc + G.klen - 1) / G.klen;
+    G.total = (G.nch + 3) / 4 * g.dil * G.nseg;
+    return G;
 }
 
-template <bool SPACE>
-void conv(flof_ctx *ctx, const float *in, float *out, float *out_relu, const bf16x8 *wf,
-          const float *bias, const float *mask, const float *res, const Geo &g, int sgn,
-          int flags)
+size_t bf_bytes(const Geo &g) { return (size_t)g.n * C * 2; }
+size_t f_bytes(const Geo &g) { return (size_t)g.n * C * 4; }
+unsigned short *u16p(const Tmp &t) { return t.as<unsigned short>(); }
+
+template <bool LIFT, int MODE>
+void launch_space(flof_ctx *ctx, const In &in, const bf16x8 *wf, const float *bias,
+                  const float *res, float *out_f, unsigned short *out_b, float *colsum,
+                  const SpaceGeo &S)
 {
-    hipLaunchKernelGGL(k_conv<SPACE>, dim3(conv_blocks(ctx, g.n)), dim3(256), 0, ctx->stream,
-                       in, out, out_relu, wf, bias, mask, res, g, sgn, flags);
-    check_launch("k_conv");
+    // 16-position tiles per wavefront; two, four, six and eight are built
+    const int nt = (8 * S.XW + 63) / 64;
+    auto k = nt <= 2   ? k_space<LIFT, MODE, 2>
+             : nt <= 4 ? k_space<LIFT, MODE, 4>
+             : nt <= 6 ? k_space<LIFT, MODE, 6>
+                       : k_space<LIFT, MODE, 8>;
+    hipLaunchKernelGGL(k, dim3(space_blocks(S)), dim3(256), 0, ctx->stream, in.b, in.i0, in.i1,
+                       in.P, wf, bias, res, out_f, out_b, colsum, S);
+    check_launch("k_space");
 }
 
-// activations of one forward pass, kept for the backward pass
+// a = relu(space conv of hb (block 0: of the lift) + bias), BF16
+void space_fwd(flof_ctx *ctx, const In &in, bool first, const bf16x8 *wf, const float *bias,
+               unsigned short *out, const Geo &g)
+{
+    if (first)
+        launch_space<true, SP_FWD>(ctx, in, wf, bias, nullptr, nullptr, out, nullptr,
+                                   space_geo(g, 8, 2048));
+    else
+        launch_space<false, SP_FWD>(ctx, in, wf, bias, nullptr, nullptr, out, nullptr,
+                                    space_geo(g, 8, 2048));
+}
+
+// h' = res + (time conv of a + bias): FP32 and / or BF16, or its head
+void time_fwd(flof_ctx *ctx, const unsigned short *a, const bf16x8 *wf, const float *bias,
+              const float *res, const In &lin, float *hf, unsigned short *hb, const float *P,
+              float4 *flow, const Geo &g)
+{
+    const TimeGeo G = time_geo(g);
+    auto k = res ? k_time<false, TM_FWD> : k_time<true, TM_FWD>;
+    hipLaunchKernelGGL(k, dim3(G.total), dim3(256), 0, ctx->stream, a, (const s16x4 *)wf, bias,
+                       res, lin, nullptr, hf, hb, P, flow, nullptr, G);
+    check_launch("k_time");
+}
+
+// what a backward pass needs of a forward one: the BF16 conv inputs and the
+// last block's FP32 output
 struct Acts {
-    Tmp h[NB + 1], s[NB], a[NB];
+    Tmp hb[NB], ab[NB], h;
 };
 
-void forward(flof_warmnet *net, const float *i0, const float *i1, const Geo &g0, Acts &A,
-             float4 *flow)
+// the network's flow; with A its activations are kept
+void forward(flof_ctx *ctx, flof_warmnet *net, const float *i0, const float *i1, const Geo &g0,
+             Acts *A, float4 *flow)
 {
-    const Geo &g = g0;
-    flof_ctx *ctx = net->ctx;
     if (!net->frag_ok) pack_all(net);
-    const size_t ab = (size_t)g.n * C * 4;
-    for (int b = 0; b <= NB; ++b) A.h[b] = Tmp(ctx, ab);
+    Tmp hf[2], hbt[2], abt;
+    if (!A) abt = Tmp(ctx, bf_bytes(g0));
+    const In lin{nullptr, i0, i1, net->P};
     for (int b = 0; b < NB; ++b) {
-        A.s[b] = Tmp(ctx, ab);
-        A.a[b] = Tmp(ctx, ab);
-    }
-    hipLaunchKernelGGL(k_lift, dim3(grid_blocks(ctx, g.n)), dim3(256), 0, ctx->stream, i0, i1,
-                       (const float *)net->P, A.h[0].as<float>(), g.n);
-    check_launch("k_lift");
-    for (int b = 0; b < NB; ++b) {
+        const bool last = b == NB - 1;
         const float *blk = net->P + OFF_BLK + b * BLK_SIZE;
         const bf16x8 *f = net->frag + (size_t)b * FRAG_BLK;
         Geo g = g0;
         g.dil = 1 << b;
-        conv<true>(ctx, A.h[b].as<float>(), A.s[b].as<float>(), A.a[b].as<float>(), f,
-                   blk + BLK_BS, nullptr, nullptr, g, 1, EP_BIAS);
-        conv<false>(ctx, A.a[b].as<float>(), A.h[b + 1].as<float>(), nullptr, f + 2 * FRAG_S,
-                    blk + BLK_BT, nullptr, A.h[b].as<float>(), g, 1, EP_BIAS | EP_RES);
+        In in = lin;
+        if (b) in.b = u16p(A ? A->hb[b] : hbt[b & 1]);
+        if (A) A->ab[b] = Tmp(ctx, bf_bytes(g));
+        unsigned short *a = u16p(A ? A->ab[b] : abt);
+        space_fwd(ctx, in, b == 0, f, blk + BLK_BS, a, g);
+        Tmp &hn = last && A ? A->h : hf[(b + 1) & 1];
+        if (!hn.p && (!last || A)) hn = Tmp(ctx, f_bytes(g));
+        Tmp *hbn = last ? nullptr : A ? &A->hb[b + 1] : &hbt[(b + 1) & 1];
+        if (hbn && !hbn->p) *hbn = Tmp(ctx, bf_bytes(g));
+        time_fwd(ctx, a, f + 2 * FRAG_S, blk + BLK_BT, b ? hf[b & 1].as<float>() : nullptr, lin,
+                 last && !A ? nullptr : hn.as<float>(), hbn ? u16p(*hbn) : nullptr, net->P,
+                 last ? flow : nullptr, g);
     }
-    hipLaunchKernelGGL(k_head, dim3(grid_blocks(ctx, g.n)), dim3(256), 0, ctx->stream,
-                       (const float *)A.h[NB].as<float>(), (const float *)net->P, flow, g.n);
-    check_launch("k_head");
 }
 
 }  // namespace
@@ -565,132 +1125,131 @@ void flof::warmnet_infer(flof_ctx *ctx, flof_warmnet *net, const float *i0, cons
     FLOF_REQUIRE(n >= 1 && n < (1ll << 30), FLOF_ERR_DIM,
                  "warm-start net: 1 to 2^30 cells");
     const Geo g0{D.X, D.Y, D.Z, D.T, (int)n, 1};
-    if (!net->frag_ok) pack_all(net);
-    const size_t ab = (size_t)n * C * 4;
-    Tmp h(ctx, ab), h2(ctx, ab), s(ctx, ab), a(ctx, ab);
-    hipLaunchKernelGGL(k_lift, dim3(grid_blocks(ctx, n)), dim3(256), 0, ctx->stream, i0, i1,
-                       (const float *)net->P, h.as<float>(), (int)n);
-    check_launch("k_lift");
-    for (int b = 0; b < NB; ++b) {
-        const float *blk = net->P + OFF_BLK + b * BLK_SIZE;
-        const bf16x8 *f = net->frag + (size_t)b * FRAG_BLK;
-        Geo g = g0;
-        g.dil = 1 << b;
-        conv<true>(ctx, h.as<float>(), s.as<float>(), a.as<float>(), f, blk + BLK_BS, nullptr,
-                   nullptr, g, 1, EP_BIAS);
-        conv<false>(ctx, a.as<float>(), h2.as<float>(), nullptr, f + 2 * FRAG_S, blk + BLK_BT,
-                    nullptr, h.as<float>(), g, 1, EP_BIAS | EP_RES);
-        std::swap(h, h2);
-    }
-    hipLaunchKernelGGL(k_head, dim3(grid_blocks(ctx, n)), dim3(256), 0, ctx->stream,
-                       (const float *)h.as<float>(), (const float *)net->P, flow, (int)n);
-    check_launch("k_head");
+    forward(ctx, net, i0, i1, g0, nullptr, flow);
 }
 
 
 namespace {
 
-int wgrad_blocks(flof_ctx *ctx, int n)
+// sum of `rows` rows of partials into dst, in FP64
+void sum_rows(flof_ctx *ctx, const float *part, int rows, int cols, float *dst)
 {
-    const int chunks = (n + 31) / 32;
-    return std::max(1, std::min((chunks + 3) / 4, ctx->num_cu * 2));
-}
-
-// dW (and db) of one conv: partials per wavefront, then a column sum
-template <bool SPACE, int M0, int NT>
-void wgrad_taps(flof_ctx *ctx, const float *in, const float *dout, const Geo &g, float *dW)
-{
-    const int nbk = wgrad_blocks(ctx, g.n);
-    const int waves = nbk * 4;
-    Tmp part(ctx, (size_t)waves * NT * C * C * 4);
-    hipLaunchKernelGGL((k_conv_wgrad<SPACE, M0, NT>), dim3(nbk), dim3(256), 0, ctx->stream, in,
-                       dout, part.as<float>(), g);
-    check_launch("k_conv_wgrad");
-    hipLaunchKernelGGL(k_sum_rows, dim3((NT * C * C + 255) / 256), dim3(256), 0, ctx->stream,
-                       (const float *)part.as<float>(), waves, NT * C * C, dW + M0 * C * C, 0);
+    hipLaunchKernelGGL(k_sum_rows, dim3((cols + 15) / 16), dim3(256), 0, ctx->stream, part, rows,
+                       cols, dst);
     check_launch("k_sum_rows");
 }
 
-template <bool SPACE>
-void conv_wgrad(flof_ctx *ctx, const float *in, const float *dout, const Geo &g, float *dW,
-                float *db)
+// two workgroups of the weight-gradient kernels per CU, as LDS admits
+int wgrad_blocks(flof_ctx *ctx, int items)
 {
-    if (SPACE) {
-        wgrad_taps<true, 0, 9>(ctx, in, dout, g, dW);
-        wgrad_taps<true, 9, 9>(ctx, in, dout, g, dW);
-        wgrad_taps<true, 18, 9>(ctx, in, dout, g, dW);
-    } else {
-        wgrad_taps<false, 0, NTT>(ctx, in, dout, g, dW);
-    }
-    const int cb = grid_blocks(ctx, (g.n + 15) / 16, 1, 4);
-    Tmp bp(ctx, (size_t)cb * C * 4);
-    hipLaunchKernelGGL(k_col_partials, dim3(cb), dim3(256), 0, ctx->stream, dout, g.n, C,
-                       bp.as<float>());
-    hipLaunchKernelGGL(k_sum_rows, dim3(1), dim3(256), 0, ctx->stream,
-                       (const float *)bp.as<float>(), cb, C, db, 0);
-    check_launch("k_col_partials");
+    return std::max(1, std::min(items, ctx->num_cu * 2));
+}
+
+void wgrad_space(flof_ctx *ctx, const In &in, bool first, const unsigned short *dout,
+                 const Geo &g, float *dW)
+{
+    const SpaceGeo S = space_geo(g, 4, 2048);
+    const int nbk = wgrad_blocks(ctx, S.total);
+    Tmp part(ctx, (size_t)nbk * 4 * NS * C * C * 4);
+    auto k = first ? k_wgrad_space<true, 1>
+                   : g.dil == 1 ? k_wgrad_space<false, 1>
+                                : g.dil == 2 ? k_wgrad_space<false, 2> : k_wgrad_space<false, 0>;
+    hipLaunchKernelGGL(k, dim3(nbk), dim3(256), 0, ctx->stream, in.b, in.i0, in.i1, in.P, dout,
+                       part.as<float>(), S);
+    check_launch("k_wgrad_space");
+    sum_rows(ctx, part.as<float>(), nbk * 4, NS * C * C, dW);
+}
+
+void wgrad_time(flof_ctx *ctx, const unsigned short *in, const unsigned short *dout, const Geo &g,
+                float *dW)
+{
+    const TimeGeo G = time_geo(g);
+    const int nbk = wgrad_blocks(ctx, (G.nch * G.d * G.nseg + 3) / 4);
+    Tmp part(ctx, (size_t)nbk * 4 * NTT * C * C * 4);
+    hipLaunchKernelGGL(k_wgrad_time, dim3(nbk), dim3(256), 0, ctx->stream, in, dout,
+                       part.as<float>(), G);
+    check_launch("k_wgrad_time");
+    sum_rows(ctx, part.as<float>(), nbk * 4, NTT * C * C, dW);
 }
 
 // forward + loss + backward; gradients into net->G, returns the loss
 double loss_grad(flof_warmnet *net, const float *i0, const float *i1, const float4 *tgt,
                  const Geo &g0)
 {
-    const Geo &g = g0;
     flof_ctx *ctx = net->ctx;
+    const int n = g0.n;
     Acts A;
-    Tmp flow(ctx, (size_t)g.n * 16), dy(ctx, (size_t)g.n * 16);
-    forward(net, i0, i1, g, A, flow.as<float4>());
-    const int lb = grid_blocks(ctx, g.n, 256, 4);
+    Tmp flow(ctx, (size_t)n * 16), dy(ctx, (size_t)n * 16);
+    forward(ctx, net, i0, i1, g0, &A, flow.as<float4>());
+    const int lb = grid_blocks(ctx, n, 256, 4);
     Tmp lp(ctx, (size_t)lb * 8);
     hipLaunchKernelGGL(k_loss, dim3(lb), dim3(256), 0, ctx->stream,
-                       (const float4 *)flow.as<float4>(), tgt, dy.as<float4>(), g.n,
+                       (const float4 *)flow.as<float4>(), tgt, dy.as<float4>(), n,
                        lp.as<double>());
     check_launch("k_loss");
-    const size_t ab = (size_t)g.n * C * 4;
-    Tmp dh(ctx, ab), dh2(ctx, ab), ds(ctx, ab);
-    const int hb = grid_blocks(ctx, g.n, 256, 2);
-    Tmp hp(ctx, (size_t)hb * (C * 4 + 4) * 4);
+    Tmp dh(ctx, f_bytes(g0)), dh2(ctx, f_bytes(g0)), dhb(ctx, bf_bytes(g0)),
+        dhb2(ctx, bf_bytes(g0)), dsb(ctx, bf_bytes(g0));
+    const int hb = grid_blocks(ctx, n, 256, 4);
+    Tmp hp(ctx, (size_t)hb * HEAD_COLS * 4), hs(ctx, HEAD_COLS * 4);
     hipLaunchKernelGGL(k_head_bwd, dim3(hb), dim3(256), 0, ctx->stream,
-                       (const float *)A.h[NB].as<float>(), (const float4 *)dy.as<float4>(),
-                       (const float *)net->P, dh.as<float>(), g.n, hp.as<float>());
+                       (const float *)A.h.as<float>(), (const float4 *)dy.as<float4>(),
+                       (const float *)net->P, dh.as<float>(), u16p(dhb), n, hp.as<float>());
     check_launch("k_head_bwd");
-    hipLaunchKernelGGL(k_sum_rows, dim3(1), dim3(256), 0, ctx->stream,
-                       (const float *)hp.as<float>(), hb, C * 4 + 4, net->G + OFF_WH, 0);
+    sum_rows(ctx, hp.as<float>(), hb, HEAD_COLS, hs.as<float>());
+    FLOF_HIP(hipMemcpyAsync(net->G + OFF_WH, hs.p, (C * 4 + 4) * 4, hipMemcpyDeviceToDevice,
+                            ctx->stream));
+    FLOF_HIP(hipMemcpyAsync(net->G + OFF_BLK + (NB - 1) * BLK_SIZE + BLK_BT,
+                            hs.as<float>() + C * 4 + 4, C * 4, hipMemcpyDeviceToDevice,
+                            ctx->stream));
+    const In lin{nullptr, i0, i1, net->P};
     for (int b = NB - 1; b >= 0; --b) {
         Geo g = g0;
         g.dil = 1 << b;
         float *gb = net->G + OFF_BLK + b * BLK_SIZE;
-        const float *blk = net->P + OFF_BLK + b * BLK_SIZE;
         const bf16x8 *f = net->frag + (size_t)b * FRAG_BLK;
-        (void)blk;
         // h_{b+1} = h_b + Wt * a + bt
-        conv_wgrad<false>(ctx, A.a[b].as<float>(), dh.as<float>(), g, gb + BLK_WT,
-                          gb + BLK_BT);
-        // ds = (Wt^T * dh) masked by s > 0
-        conv<false>(ctx, dh.as<float>(), ds.as<float>(), nullptr, f + 2 * FRAG_S + FRAG_T,
-                    nullptr, A.s[b].as<float>(), nullptr, g, -1, EP_MASK);
-        conv_wgrad<true>(ctx, A.h[b].as<float>(), ds.as<float>(), g, gb + BLK_WS,
-                         gb + BLK_BS);
-        // dh_b = dh_{b+1} + Ws^T * ds
-        conv<true>(ctx, ds.as<float>(), dh2.as<float>(), nullptr, f + FRAG_S, nullptr,
-                   nullptr, dh.as<float>(), g, -1, EP_RES);
+        wgrad_time(ctx, u16p(A.ab[b]), u16p(dhb), g, gb + BLK_WT);
+        // ds = (Wt^T * dh) where a > 0; its sum is the space bias' gradient
+        {
+            const TimeGeo G = time_geo(g);
+            Tmp cp(ctx, (size_t)G.total * C * 4);
+            hipLaunchKernelGGL((k_time<false, TM_BWD>), dim3(G.total), dim3(256), 0, ctx->stream,
+                               u16p(dhb), (const s16x4 *)(f + 2 * FRAG_S + FRAG_T), nullptr,
+                               nullptr, lin, u16p(A.ab[b]), nullptr, u16p(dsb), nullptr, nullptr,
+                               cp.as<float>(), G);
+            check_launch("k_time (backward)");
+            sum_rows(ctx, cp.as<float>(), G.total, C, gb + BLK_BS);
+        }
+        In in = lin;
+        in.b = b ? u16p(A.hb[b]) : nullptr;
+        wgrad_space(ctx, in, b == 0, u16p(dsb), g, gb + BLK_WS);
+        // dh_b = dh_{b+1} + Ws^T * ds; its sum is block b - 1's time bias' gradient
+        {
+            const SpaceGeo S = space_geo(g, 8, 2048);
+            const int nbk = space_blocks(S);
+            Tmp cp(ctx, (size_t)nbk * C * 4);
+            In ds = lin;
+            ds.b = u16p(dsb);
+            launch_space<false, SP_BWD>(ctx, ds, f + FRAG_S, nullptr, dh.as<float>(),
+                                        dh2.as<float>(), u16p(dhb2), cp.as<float>(), S);
+            if (b) sum_rows(ctx, cp.as<float>(), nbk, C, gb - BLK_SIZE + BLK_BT);
+        }
         std::swap(dh, dh2);
+        std::swap(dhb, dhb2);
     }
-    const int fb = grid_blocks(ctx, g.n, 256, 2);
+    const int fb = grid_blocks(ctx, n, 256, 4);
     Tmp fp(ctx, (size_t)fb * 3 * C * 4);
     hipLaunchKernelGGL(k_lift_bwd, dim3(fb), dim3(256), 0, ctx->stream, i0, i1,
-                       (const float *)dh.as<float>(), g.n, fp.as<float>());
+                       (const float *)dh.as<float>(), n, fp.as<float>());
     check_launch("k_lift_bwd");
-    hipLaunchKernelGGL(k_sum_rows, dim3(1), dim3(256), 0, ctx->stream,
-                       (const float *)fp.as<float>(), fb, 3 * C, net->G + OFF_WL, 0);
-    check_launch("k_sum_rows");
+    sum_rows(ctx, fp.as<float>(), fb, 3 * C, net->G + OFF_WL);
     std::vector<double> h(lb);
     FLOF_HIP(hipMemcpyAsync(h.data(), lp.p, (size_t)lb * 8, hipMemcpyDeviceToHost,
                             ctx->stream));
     FLOF_HIP(hipStreamSynchronize(ctx->stream));
     double s = 0.;
     for (double v : h) s += v;
-    return s / (4.0 * (double)g.n);
+    return s / (4.0 * (double)n);
 }
 
 void need_pair(const flof_grid4d *i0, const flof_grid4d *i1, const flof_grid4d *v,
@@ -823,8 +1382,8 @@ int flof_warmnet_forward(flof_warmnet *net, flof_grid4d *i0, flof_grid4d *i1,
     FLOF_REQUIRE(net, FLOF_ERR_ARG, "warmnet_forward: null net");
     need_pair(i0, i1, flow, "warmnet_forward");
     const Geo g = geo_of(i0);
-    Acts A;
-    forward(net, (const float *)i0->data, (const float *)i1->data, g, A, (float4 *)flow->data);
+    forward(ctx, net, (const float *)i0->data, (const float *)i1->data, g, nullptr,
+            (float4 *)flow->data);
     FLOF_HIP(hipStreamSynchronize(ctx->stream));
     API_CATCH(ctx)
 }
@@ -898,10 +1457,7 @@ int flof_warmnet_warm_start(flof_warmnet *net, flof_grid4d *i0, flof_grid4d *i1,
         v[L - 1] = Tmp(ctx, (size_t)g.n * 16);
         out = v[L - 1].as<float4>();
     }
-    {
-        Acts A;
-        forward(net, ca, cb, g, A, out);
-    }
+    forward(ctx, net, ca, cb, g, nullptr, out);
     for (size_t l = L - 1; l >= 1; --l) {
         void *dst = l == 1 ? warm->data : nullptr;
         if (l > 1) {

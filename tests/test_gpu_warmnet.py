@@ -73,6 +73,33 @@ def test_gradients_match_oracle():
         assert rel < 3e-2, name
 
 
+@pytest.mark.parametrize("shape", [(3, 5, 9, 17), (9, 18, 3, 65), (17, 2, 33, 5), (1, 9, 8, 48)])
+def test_network_tile_edges_match_oracle(shape):
+    """Forward pass and gradients on grids whose rows fill the 16-cell tiles
+    unevenly (17, 48 and 5 wide), span two x tiles (65), have fewer rows,
+    planes or t steps than the widest tap spacing (8), or end a stretch of 64
+    cells early: the bounds of the two tests above."""
+    say("warmnet tile edges", shape)
+    s, a, b, g0, g1 = _case(shape)
+    net = WS.WarmNet(seed=9)
+    P = (RNG.standard_normal(WS.num_params()) * 0.2).astype(np.float32)
+    net.set_params(P)
+    flow = s.create(M.Grid4Vec4)
+    net.forward(g0, g1, flow)
+    y = flow.to_numpy()
+    ref = W.forward(P.astype(np.float64), a, b, rnd=True)
+    assert np.abs(y - ref).max() < 2e-2 * np.abs(ref).max()
+    assert np.sqrt(((y - ref) ** 2).mean()) < 3e-3 * np.abs(ref).max()
+    tgt = RNG.standard_normal(a.shape + (4,)).astype(np.float32)
+    tg = s.create(M.Grid4Vec4)
+    tg.from_numpy(tgt)
+    loss = net.loss_grad(g0, g1, tg)
+    g = net.get_grads().astype(np.float64)
+    rl, rg = W.loss_grad(P.astype(np.float64), a, b, tgt, rnd=True)
+    assert abs(loss - rl) <= 1e-3 * rl
+    assert np.linalg.norm(g - rg) < 3e-2 * np.linalg.norm(rg)
+
+
 def test_training_lowers_loss_and_warm_start_is_used():
     """Train on plain-solve flows of 16^4 drop pairs, then warm-start unseen
     pairs: the loss falls, the warm start is kept on the finest level, the
