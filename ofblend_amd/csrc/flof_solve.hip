@@ -40,6 +40,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "flof_cg.h"
 #include "flof_internal.h"
 
 // unroll factor of the t-marching loops
@@ -60,38 +61,6 @@
 #endif
 
 namespace flof {
-
-struct CgState {
-    double sigma;
-    double alpha;
-    double alpha_prev;  // alpha of the previous iteration (deferred x update)
-    double beta;
-    double acc;      // stopping threshold cgAccuracy * resIni
-    double resIni;   // signed max of the initial residual
-    double resRel;   // (float)(residual / resIni), as ret_residual
-    double r2, b2;   // warm-start residual check
-    double bb, rr;   // ||b||^2 of the rhs and ||r||^2 of the final residual
-    double gamma;    // warm-start scale
-    int iters;
-    int done;
-    int status;  // 0 converged, 1 not converged, 2 sigma 0/NaN, 3 tiny rhs
-    int maxIter;
-    int warm;    // warm start kept
-    int zero;    // result must be zeroed (failed solve)
-    int dir_mode;  // k_cg_dir: 0 skip, 1 x and p update, 2 x update only
-    int fast_rcp;  // set-up: every interior g_d^2 + diag in rcp_newton's range
-};
-
-struct LevelGeom {
-    Dims4 D;
-    Coord4 C;
-    float offd;   // -wSmooth (times mDx2Inv = 1)
-    float diag;   // 8*wSmooth + wEnergy, formed as the reference does
-    int use_offd; // offd != 0
-    float eps;    // VECTOR_EPSILON of FP32 builds
-    int fast_rcp; // every interior diagonal entry g_d^2 + diag of the level
-                  // lies in the range of rcp_newton (set after the set-up)
-};
 
 __device__ __forceinline__ bool interior(const Dims4 &D, int i, int j, int k, int t)
 {
@@ -146,14 +115,6 @@ __device__ __forceinline__ float4 apply_I(const float4 &pc)
         out[d] = v;
     }
     return make_float4(out[0], out[1], out[2], out[3]);
-}
-
-__device__ __forceinline__ void dd_add4(DD &a, const float4 &u, const float4 &v)
-{
-    dd_add(a, (double)(u.x * v.x));
-    dd_add(a, (double)(u.y * v.y));
-    dd_add(a, (double)(u.z * v.z));
-    dd_add(a, (double)(u.w * v.w));
 }
 
 __device__ __forceinline__ float4 prec_of(const float4 &g, float diag)
@@ -1024,14 +985,6 @@ k_cg_update_tm(float4 *__restrict__ r, const typename PS::T *__restrict__ p,
 // two roundings in the same order, so x is the same while it is read and
 // written every other iteration only.  dir_mode 2 (the last iteration)
 // applies the pending updates and leaves p.
-__device__ __forceinline__ float4 x_plus(const float4 &x, double a, const float4 &p)
-{
-    return make_float4((float)((double)x.x + a * (double)p.x),
-                       (float)((double)x.y + a * (double)p.y),
-                       (float)((double)x.z + a * (double)p.z),
-                       (float)((double)x.w + a * (double)p.w));
-}
-
 template <class PS, bool ODD, class IM>
 __device__ __forceinline__ void
 cg_dir_tm_body(int bid, int nblk, const typename PS::T *__restrict__ p, typename PS::T *pn,
@@ -2774,15 +2727,58 @@ static void level_iterate(flof_ctx *ctx, LevelCg &L, int maxIter)
     L.hs = hs;
 }
 
+// The resident form (flof_resident.hip) takes the levels whose vectors fit the
+// chip: FP32 direction storage, stencil form not forced, no timing of the
+// iteration's kernels (it has none of its own).  Measured per iteration against
+// the launches of level_iterate: @RESTABLE@
+static ResPlan resident_level_plan(const flof_ctx *ctx, const LevelCg &L, int budget,
+                                   bool fewest = false)
+{
+    for (int k : {FLOF_KT_CG_APPLY, FLOF_KT_CG_UPDATE, FLOF_KT_CG_DIR})
+        if (ctx->timers[k].on) return ResPlan{};
+    if (!ctx->use_tmarch || ctx->stencil != FLOF_STENCIL_AUTO || L.pstore != FLOF_PSTORE_F32 ||
+        L.hs.done)
+        return ResPlan{};
+    return resident_plan(L.D, budget, fewest);
+}
+
+// iterates the levels side by side; false: set them up again and use another form
+static bool resident_levels(flof_ctx *ctx, const std::vector<LevelCg *> &Ls,
+                            const std::vector<ResPlan> &plans)
+{
+    std::vector<ResLevel> lv;
+    for (LevelCg *L : Ls) {
+        LevelWork &W = L->W;
+        lv.push_back(ResLevel{L->D, L->G.offd, L->G.diag, L->G.use_offd, W.g.as<float4>(),
+                              W.prec.as<float4>(), W.x.as<float4>(), W.r.as<float4>(),
+                              W.p.as<float4>(), W.q.as<float4>(), L->st()});
+    }
+    if (!resident_iterate(ctx, lv, plans)) return false;
+    for (LevelCg *L : Ls)
+        FLOF_HIP(hipMemcpyAsync(&L->hs, L->st(), sizeof(CgState), hipMemcpyDeviceToHost,
+                                ctx->stream));
+    FLOF_HIP(hipStreamSynchronize(ctx->stream));
+    return true;
+}
+
 SolveOut solve_level(flof_ctx *ctx, const void *i0, const void *i1, const float4 *vin,
                      float *rhsT, const Dims4 &D, float wSmooth, float wEnergy,
                      float cgAccuracy, float dt, int maxIter, const float4 *warm,
                      const float4 *warm_base, float4 *out, bool accumulate)
 {
     LevelCg L(ctx, D);
-    level_setup(ctx, L, i0, i1, vin, rhsT, wSmooth, wEnergy, cgAccuracy, dt, maxIter, warm,
-                warm_base, false);
-    level_iterate(ctx, L, maxIter);
+    auto setup = [&]() {
+        level_setup(ctx, L, i0, i1, vin, rhsT, wSmooth, wEnergy, cgAccuracy, dt, maxIter, warm,
+                    warm_base, false);
+    };
+    setup();
+    bool done = false;
+    const ResPlan plan = resident_level_plan(ctx, L, ctx->num_cu);
+    if (plan.nwg > 0) {
+        done = resident_levels(ctx, {&L}, {plan});
+        if (!done) setup();
+    }
+    if (!done) level_iterate(ctx, L, maxIter);
     return level_finish(ctx, L, out, accumulate);
 }
 
@@ -3330,6 +3326,7 @@ static void multiscale_fused(flof_ctx *ctx, int np, float4 *const *vel_top,
         for (int j = 0; j < np; ++j)
             if ((int)pr[j].D.size() > l) act.push_back(j);
         std::vector<std::unique_ptr<LevelCg>> Ls;
+        std::vector<std::function<void()>> setups;
         std::vector<Tmp> warped;
         for (int j : act) {
             Prob &q = pr[j];
@@ -3350,15 +3347,53 @@ static void multiscale_fused(flof_ctx *ctx, int np, float4 *const *vel_top,
             // is the problem's own solve, bit for bit.
             Ls.emplace_back(new LevelCg(ctx, D));
             const bool may_solo = n >= SOLO_MIN_CELLS;
-            level_setup(ctx, *Ls.back(), w, q.i1[l], nullptr, nullptr, P.wSmooth, P.wEnergy,
-                        P.cgAccuracy, dt, P.cgMaxIter, nullptr, nullptr, !may_solo);
+            LevelCg *Lc = Ls.back().get();
+            const void *i1l = q.i1[l];
+            setups.push_back([=]() {
+                level_setup(ctx, *Lc, w, i1l, nullptr, nullptr, P.wSmooth, P.wEnergy,
+                            P.cgAccuracy, dt, P.cgMaxIter, nullptr, nullptr, !may_solo);
+            });
+            setups.back()();
+        }
+        // levels that fit the chip's registers and LDS run resident, as many
+        // side by side as their smallest plans allow (a level on few
+        // workgroups takes longer per iteration, but by less than the number
+        // of levels that share the launch); the rest share launches per kernel
+        std::vector<size_t> res;
+        std::vector<int> need(Ls.size(), 0);
+        for (size_t a = 0; a < Ls.size(); ++a) {
+            need[a] = resident_level_plan(ctx, *Ls[a], ctx->num_cu, true).nwg;
+            if (need[a] > 0) res.push_back(a);
+        }
+        std::stable_sort(res.begin(), res.end(),
+                         [&](size_t a, size_t b) { return Ls[a]->n > Ls[b]->n; });
+        for (size_t at = 0; at < res.size();) {
+            int sum = 0;
+            size_t end = at;
+            while (end < res.size() && sum + need[res[end]] <= ctx->num_cu)
+                sum += need[res[end++]];
+            std::vector<LevelCg *> group;
+            std::vector<ResPlan> plans;
+            for (size_t a = at; a < end; ++a) {
+                group.push_back(Ls[res[a]].get());
+                plans.push_back(resident_level_plan(
+                    ctx, *group.back(),
+                    (int)((int64_t)need[res[a]] * ctx->num_cu / sum)));
+            }
+            if (!resident_levels(ctx, group, plans))
+                for (size_t a = at; a < end; ++a) {
+                    setups[res[a]]();
+                    need[res[a]] = 0;
+                }
+            at = end;
         }
         std::vector<LevelCg *> raw;
-        for (auto &L : Ls) {
-            if (L->W.lds)
-                level_iterate(ctx, *L, P.cgMaxIter);
+        for (size_t a = 0; a < Ls.size(); ++a) {
+            if (need[a] > 0) continue;
+            if (Ls[a]->W.lds)
+                level_iterate(ctx, *Ls[a], P.cgMaxIter);
             else
-                raw.push_back(L.get());
+                raw.push_back(Ls[a].get());
         }
         fused_iterations(ctx, raw);
         for (size_t a = 0; a < act.size(); ++a) {
