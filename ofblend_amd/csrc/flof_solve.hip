@@ -2729,8 +2729,10 @@ static void level_iterate(flof_ctx *ctx, LevelCg &L, int maxIter)
 
 // The resident form (flof_resident.hip) takes the levels whose vectors fit the
 // chip: FP32 direction storage, stencil form not forced, no timing of the
-// iteration's kernels (it has none of its own).  Measured per iteration against
-// the launches of level_iterate: @RESTABLE@
+// iteration's kernels (it has none of its own).  Per iteration, launches of
+// level_iterate against the resident form: 8^4 14.8 and 5.5 us, 16^4 16.8 and
+// 7.9, 24^4 29.4 and 13.5, 32^4 50.7 and 18.8, 32^3 x 48 65.4 and 26.3: it is
+// the better one wherever it fits, up to 256 boxes of 11 cells per thread.
 static ResPlan resident_level_plan(const flof_ctx *ctx, const LevelCg &L, int budget,
                                    bool fewest = false)
 {

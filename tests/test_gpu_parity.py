@@ -592,3 +592,45 @@ def test_non_finite_image_gives_the_references_zero_flow(where, bad):
     assert np.isfinite(got).all()
     assert lv["status"] == [st] and st == 2
     assert lv["iters"] == [it] == [0]
+
+
+@pytest.mark.parametrize("shape,smooth", [
+    ((3, 3, 3, 4), 0.1), ((5, 4, 3, 9), 0.1), ((16, 30, 4, 36), 0.1), ((100, 8, 8, 12), 0.1),
+    ((9, 23, 4, 6), 0.0), ((24, 23, 25, 22), 0.1), ((30, 27, 26, 29), 0.1),
+    ((29, 28, 29, 29), 0.1), ((32, 31, 30, 33), 0.1), ((31, 33, 30, 47), 0.1)])
+def test_resident_pcg_matches_launched_pcg(shape, smooth):
+    """The resident PCG (one launch per level) on levels of one workgroup, of
+    one-row and one-plane boxes, of boxes with 1 to 11 cells per thread and
+    with x rows of 1 to 98 cells, with and without neighbour terms, from an
+    incoming flow, to convergence and to caps after an odd and an even
+    iteration: the flow, the iterations and the residuals are those of the
+    t-marching launches bit for bit (which the oracle pins above); the small
+    ones are compared with the oracle directly."""
+    from ofblend_amd import _lib
+    from ofblend_amd.abi import FLOF_STENCIL_AUTO, FLOF_STENCIL_TMARCH
+    X, Y, Z, T = shape
+    a, b = O.drop_sdf(X, Y, Z, T, seed=81), O.drop_sdf(X, Y, Z, T, seed=82)
+    vin = (np.random.default_rng(83).standard_normal((T, Z, Y, X, 4)) * 0.5).astype(np.float32)
+    s = solver(X, Y, Z, T)
+    ga, gb = real(s, a), real(s, b)
+    L, ctx = _lib.lib(), M.context()
+    for cap in (1, 2, 150):
+        res = []
+        for code in (FLOF_STENCIL_AUTO, FLOF_STENCIL_TMARCH):
+            say("resident pcg", shape, "cap", cap, "stencil", code)
+            try:
+                assert L.flof_ctx_set_stencil(ctx, code) == 0
+                vel = vec4(s, vin)
+                M.opticalFlow4d(vel, ga, gb, wSmooth=smooth, wEnergy=1e-4, cgAccuracy=1e-5,
+                                cgMaxIter=cap)
+            finally:
+                L.flof_ctx_set_stencil(ctx, FLOF_STENCIL_AUTO)
+            res.append((vel.to_numpy(), M.getLastSolveInfo().summary()["levels"][0]))
+        assert res[0][1] == res[1][1]
+        assert np.array_equal(res[0][0], res[1][0])
+    if X * Y * Z * T < 40000:
+        p = default_params(wSmooth=smooth, wEnergy=1e-4, cgAccuracy=1e-5, cgMaxIter=150)
+        with O.sum_mode(1):
+            ref, it, _, st = O.optical_flow4d(vin, a, b, p)
+        assert res[0][1]["iters"] == [it] and res[0][1]["status"] == [st]
+        assert np.array_equal(res[0][0], ref)
