@@ -2,6 +2,7 @@
 (repeatFrame4d, extrap4dLsSimple, shiftForwGrid4d, Grid4d save/load,
 loadPlaceGrid4d from .uni files, loadAdvectTimeSlice_OptInit/OptRun/Finish)
 against the CPU oracle, through the C-ABI.  All results are bit-exact."""
+import ctypes as C
 import gzip
 import struct
 
@@ -9,6 +10,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
+from ofblend_amd import _lib
 from ofblend_amd import manta as M
 
 pytestmark = pytest.mark.gpu
@@ -58,6 +60,28 @@ def test_extrap_ls_simple_bit_exact(inside):
     g = real(solver(N, N, N, T), a)
     M.extrap4dLsSimple(g, distance=4, inside=inside)
     assert np.array_equal(g.to_numpy(), O.extrap4d_ls_simple(a, 4, inside))
+
+
+@pytest.mark.parametrize("shape,marks,distance", [
+    ((3, 3, 3, 3), 1, 4), ((2, 5, 5, 5), 0, 4), ((7, 5, 6, 9), 0, 3), ((66, 4, 5, 19), 2, 40),
+    ((131, 5, 3, 20), 3, 60), ((64, 7, 4, 5), 2, 1), ((65, 3, 4, 5), 2, 0), ((129, 6, 3, 3), 1, -3),
+    ((300, 4, 4, 5), 1, 254), ((300, 4, 4, 5), 1, 255), ((7, 4, 290, 5), 1, 1000)])
+def test_extrap_layers_at_distance_and_row_edges_bit_exact(shape, marks, distance):
+    """Rows of one to five wavefronts of cells, no, one and a few marked cells,
+    distances of 0 to beyond the grid and around the largest that a byte holds,
+    NaN among the values: the oracle's layers bit for bit, both ways round."""
+    X, Y, Z, T = shape
+    rng = np.random.default_rng(sum(shape) + distance)
+    a = rng.uniform(0.5, 9.0, (T, Z, Y, X)).astype(np.float32)
+    a.reshape(-1)[::37] = np.nan
+    for _ in range(marks):
+        a[tuple(rng.integers(1, max(2, n - 1)) for n in (T, Z, Y, X))] = -1.5
+    for inside, phi in ((False, a), (True, -a)):
+        say("extrap4dLsSimple", shape, "marks", marks, "distance", distance, "inside", inside)
+        g = real(solver(X, Y, Z, T), phi)
+        M.extrap4dLsSimple(g, distance=distance, inside=inside)
+        ref = O.extrap4d_ls_simple(phi, distance, inside)
+        assert np.array_equal(g.to_numpy(), ref, equal_nan=True)
 
 
 def test_shift_forw_grid():
