@@ -572,7 +572,7 @@ void check_launch(const char *what);
 float host_max_norm_vec4(flof_ctx *ctx, const float4 *v, int64_t n);
 double host_ls_diff(flof_ctx *ctx, const float *a, const float *b, float *out,
                     const Dims4 &D, float corr, int bnd);
-void place_frames(flof_grid4d *phi, int sx, int sy, int sz,
+void place_frames(flof_grid4d *phi, int sx, int sy, int sz, const float *stack,
                   const std::function<const float *(int)> &frame_of, const float offset[4],
                   const float scale[4], int fileIdxStart, int fileIdxEnd, int debugSkipLoad,
                   float spread, const float overrideSize[4], float overrideTimeOff,

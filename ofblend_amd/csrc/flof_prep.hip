@@ -522,7 +522,7 @@ int flof_load_place_grid4d_uni(const char *fname, flof_grid4d *phi, const float 
     std::vector<float> host(fsz);
     Tmp dev(ctx, fsz * 4);
     place_frames(
-        phi, dims[0], dims[1], dims[2],
+        phi, dims[0], dims[1], dims[2], nullptr,
         [&](int f) -> const float * {
             // kernels of the previous frame may still read the buffer
             FLOF_HIP(hipStreamSynchronize(ctx->stream));

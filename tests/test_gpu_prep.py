@@ -152,6 +152,64 @@ def test_load_place_grid4d_from_files(tmp_path):
         M.loadPlaceGrid4d(pat, phi, M.Vec4(0.), M.Vec4(1.), fileIdxStart=0, fileIdxEnd=F)
 
 
+@pytest.mark.parametrize("shape,frame,F,kw", [
+    ((20, 18, 17, 9), (11, 9, 8), 6, {}),
+    ((9, 8, 3, 70), (23, 21, 19), 70, dict(spread=1.7)),
+    ((17, 16, 33, 5), (17, 16, 33), 400, dict(spread=2.0)),
+    ((12, 11, 10, 12), (24, 22, 20), 12, dict(rescaleSdfValues=True, sdfIsoOff=0.25)),
+    ((12, 11, 10, 12), (12, 11, 10), 7, dict(overrideGoodRegion=5, repeatStartFrame=0.3)),
+    ((2, 5, 5, 4), (5, 5, 5), 4, {}),
+    ((13, 12, 11, 8), (9, 9, 9), 8, dict(offset=(1.5, -2.0, 0.5, 1.0), scale=(0.7, 0.8, 0.9, 0.6)))])
+def test_place_runs_at_edges_bit_exact(shape, frame, F, kw, tmp_path):
+    """Placement of frames on the device: more slices and more frames per slice
+    than one launch takes, planes that are no multiple of a thread's run, frames
+    finer and coarser than the grid, the level-set fix-up, a kept region, no
+    interior; the oracle's values bit for bit, outer cells included.  The same
+    frames from files take the position-by-position launches."""
+    X, Y, Z, T = shape
+    sx, sy, sz = frame
+    rng = np.random.default_rng(91)
+    frames = rng.standard_normal((F, sz, sy, sx)).astype(np.float32)
+    old = rng.standard_normal((T, Z, Y, X)).astype(np.float32)
+    say("place", shape, "frames", F, frame, kw)
+    ref = O.place_frames((T, Z, Y, X), frames, fileIdxStart=0, fileIdxEnd=F, phi=old, **kw)
+    mk = dict(kw)
+    off, sc = M.Vec4(*mk.pop("offset", (0.,) * 4)), M.Vec4(*mk.pop("scale", (1.,) * 4))
+    phi = real(solver(X, Y, Z, T), old)
+    M.loadPlaceGrid4dFrames(M.DeviceArray.from_numpy(frames), phi, off, sc, fileIdxStart=0,
+                            fileIdxEnd=F, **mk)
+    assert np.array_equal(phi.to_numpy(), ref)
+    if F <= 12:
+        for f in range(F):
+            write_mnt2(tmp_path / ("e_%04d.uni" % f), frames[f])
+        phi = real(solver(X, Y, Z, T), old)
+        M.loadPlaceGrid4d(str(tmp_path / "e_%04d.uni"), phi, off, sc, fileIdxStart=0,
+                          fileIdxEnd=F, **mk)
+        assert np.array_equal(phi.to_numpy(), ref)
+
+
+def test_warp_of_more_frames_than_a_launch_takes():
+    """130 frames warped by one call are those of one call per frame."""
+    N, T, NF = 24, 6, 130
+    rng = np.random.default_rng(92)
+    s = solver(N, N, N, T)
+    phi = real(s, rng.standard_normal((T, N, N, N)).astype(np.float32))
+    defo = solver(8, 8, 8, T).create(M.Grid4Vec4)
+    defo.from_numpy(rng.standard_normal((T, 8, 8, 8, 4)).astype(np.float32))
+    out = M.DeviceArray.from_numpy(np.zeros((NF, N, N, N), np.float32))
+    f4 = lambda *c: (C.c_float * 4)(*c)
+    say("warp", NF, "frames in one call")
+    _lib.check(_lib.lib().flof_advect_time_slices_opt(
+        defo.h, out.ptr, N, N, N, NF, 0.0, 1.0 / 32, phi.h, 0.5, 1.0, f4(0, 0, 0, 0),
+        f4(1, 1, 1, 1), f4(2, 2, 2, 1), 1, 1.0), phi.ctx)
+    got = out.to_numpy()
+    for f in (0, 63, 64, 100, 127, 128, 129):
+        dst = M.DeviceArray.from_numpy(np.zeros((N, N, N), np.float32))
+        M.loadAdvectTimeSliceFromDefo(defo, dst, phi, f / 32, 0.5, defoFactor=M.Vec4(2, 2, 2, 1))
+        assert np.array_equal(got[f], dst.to_numpy())
+        assert got[f].any()
+
+
 def test_advect_time_slice_from_file(tmp_path):
     """OptInit reads the M4T2 deformation; OptRun equals the oracle warp."""
     say("loadAdvectTimeSlice_OptInit/OptRun/Finish")
