@@ -81,6 +81,58 @@ def test_advect_cfl_bit_exact(cfl):
     assert np.array_equal(gg.to_numpy(), ref)
 
 
+@pytest.mark.parametrize("shape", [(2, 2, 2, 2), (3, 4, 3, 5), (130, 3, 5, 4), (33, 7, 6, 9)])
+def test_advect_columns_at_edges_bit_exact(shape):
+    """Odd and even numbers of planes, grids without an interior, flows that
+    leave the grid, infinities and NaN in the outer layer's flow (which is not
+    used): the oracle's advected scalars and Vec4 values bit for bit, in two
+    (the result is back in the grid) and three substeps as well."""
+    X, Y, Z, T = shape
+    rng = np.random.default_rng(31)
+    vel = (rng.standard_normal((T, Z, Y, X, 4)) * 3.0).astype(np.float32)
+    a = rng.standard_normal((T, Z, Y, X)).astype(np.float32)
+    av = rng.standard_normal((T, Z, Y, X, 4)).astype(np.float32)
+    s = M.Solver(gridSize=M.vec3(X, Y, Z), fourthDim=T)
+    gv, gg, g4 = s.create(M.Grid4Vec4), s.create(M.Grid4Real), s.create(M.Grid4Vec4)
+    say("advect", shape)
+    fast = np.sqrt((vel ** 2).sum(-1).max())
+    for steps in (2, 3):
+        gv.from_numpy(vel)
+        gg.from_numpy(a)
+        cfl = float(fast / (steps - 0.5))
+        _lib.check(_lib.lib().flof_advect_cfl4d(gv.h, gg.h, cfl, 1.0, 1.0), gv.ctx)
+        assert np.array_equal(gg.to_numpy(), O.advect_cfl4d(vel, a, cfl=cfl))
+    vel[0, 0, 0, 0] = (np.inf, -np.inf, np.nan, 1.0)
+    vel[-1, -1, -1, -1] = np.nan
+    gv.from_numpy(vel)
+    for g, ref in ((gg, a), (g4, av)):
+        g.from_numpy(ref)
+        M.advect4d(gv, g, dtFac=0.6)
+        assert np.array_equal(g.to_numpy(), O.advect4d(vel, ref, dtFac=0.6))
+
+
+@pytest.mark.parametrize("src,dst", [((7, 6, 5, 9), (90, 91, 70, 8)), ((7, 6, 5, 3), (90, 91, 70, 8)),
+                                     ((7, 6, 5, 9), (90, 91, 70, 3)), ((20, 3, 2, 17), (21, 40, 3, 35)),
+                                     ((5, 4, 3, 2), (2, 3, 2, 40))])
+def test_resample_marches_in_t_bit_exact(src, dst):
+    """Grids of one t segment and of one per slice, up to 13 outputs per source
+    slice and several source slices per output: the oracle's values bit for
+    bit, scalars and Vec4, with an offset that leaves the grid."""
+    rng = np.random.default_rng(32)
+    a = rng.standard_normal(src[::-1]).astype(np.float32)
+    av = rng.standard_normal(src[::-1] + (4,)).astype(np.float32)
+    say("resample", src, dst)
+    ss = M.Solver(gridSize=M.vec3(*src[:3]), fourthDim=src[3])
+    sd = M.Solver(gridSize=M.vec3(*dst[:3]), fourthDim=dst[3])
+    for cls, x, f in ((M.Grid4Real, a, M.interpolateGrid4d), (M.Grid4Vec4, av, M.interpolateGrid4dVec)):
+        g, t = ss.create(cls), sd.create(cls)
+        g.from_numpy(x)
+        f(t, g, offset=M.Vec4(0.3, -0.2, 0.1, 1.0), scale=M.Vec4(1.1, 0.9, 1.0, 1.2))
+        ref = O.interpolate_grid4d(dst[::-1], x, offset=(0.3, -0.2, 0.1, 1.0),
+                                   scale=(1.1, 0.9, 1.0, 1.2))
+        assert np.array_equal(t.to_numpy(), ref)
+
+
 @pytest.mark.parametrize("thresh,maxIter", [(4.0, 40), (1.5, 60), (4.0, 0), (1.0, 7),
                                             (0.3, 45)])
 def test_corr_vels_of4d_far_cells_bit_exact(thresh, maxIter):
