@@ -44,7 +44,7 @@ constexpr int C = 16;       // channels
 constexpr int NB = 4;       // residual blocks
 constexpr int NS = 27;      // space taps
 constexpr int NTT = 3;      // time taps
-constexpr int PAIRS_S = 14; // ceil(27 / 2)
+constexpr int PAIRS_S = 5;  // the nine (z, x) taps by two, each with its three y taps
 
 // parameter layout (FP32, flat)
 constexpr int OFF_WL = 0;                   // [2][16]
@@ -120,12 +120,15 @@ __device__ __forceinline__ float lift(const float *__restrict__ P, int o, float 
 // side, zero outside the grid) and marches through the planes of its z class,
 // keeping three haloed planes in LDS as BF16 (the two 8-channel halves apart,
 // so that the 16 lanes of an operand read 256 contiguous bytes).  Every input
-// value is loaded about 1.25 times from memory and read 27 times from LDS;
+// value is loaded about 1.25 times from memory and read 11 to 18 times from LDS;
 // the form that gathered the taps from memory read 27 x 64 bytes per cell
 // through the vector caches and rounded each value 27 times.
-// A wavefront computes 16-cell tiles of the XW x 8 outputs (positions are
-// numbered row by row, so ragged widths fill the tiles), 14 MFMA each, with
-// the weights in registers.
+// A wavefront computes rows of a block of 16 x cells, with the weights in
+// registers.  An operand is a row's 16 cells under two of the nine (z, x) taps,
+// and serves the three output rows that see this row under their three y taps:
+// 50 LDS reads and 120 MFMA for eight rows instead of 112 of each.  64^4: 449
+// -> 409 us (167 at the rate of memory; what is left is instruction issue, and
+// the two barriers per plane with two workgroups per CU to cover them).
 struct SpaceGeo {
     int X, Y, Z, T, d;
     int nxt, XW;      // x tiles and their width
@@ -171,8 +174,9 @@ enum { SP_FWD = 0, SP_BWD = 1 };
 // zero, so its sign serves as the mask of the backward pass).
 // SP_BWD: out_f = res + conv, out_b = bf16(out_f), and the workgroup's column
 // sums of out_f (the gradient of the previous block's time bias).
-// NT: tiles per wavefront (the 8 rows hold up to 32 tiles of 16 positions)
-template <bool LIFT, int MODE, int NT>
+// NR rows of NB blocks of 16 x cells per wavefront: of four blocks one each, of
+// three two rows of each, of two four rows of one, of one two rows.
+template <bool LIFT, int MODE, int NR, int NB>
 __global__ void __launch_bounds__(256, 2)
 k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
         const float *__restrict__ i1, const float *__restrict__ P,
@@ -193,9 +197,11 @@ k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
         const int d = S.d, pitch = S.pitch, X = S.X;
         const int64_t plane = (int64_t)X * S.Y;
         const int64_t tb = plane * S.Z * w.t;
-        bf16x8 wr[PAIRS_S];
+        bf16x8 wr[PAIRS_S][3];
 #pragma unroll
-        for (int p = 0; p < PAIRS_S; ++p) wr[p] = wf[p * 64 + lane];
+        for (int p = 0; p < PAIRS_S; ++p)
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy) wr[p][dy] = wf[(p * 3 + dy) * 64 + lane];
         // staged elements of this thread: 16-byte half sh of halo cells e; the
         // two halves of a cell by neighbouring lanes, or (the lift, whose
         // weights are then scalars of one half) by wavefronts
@@ -251,19 +257,19 @@ k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
                 if (e < nst) s[e] = st_ok && off[m] >= 0 ? st[m] : bf16x8{};
             }
         };
-        // the tiles of this wavefront: LDS slot of the lane's cell in a plane,
-        // and its offset in a grid plane (-1: not an output)
-        const int npos = TY * S.XW;
-        int base[NT], cell[NT];
+        // the rows of this wavefront: LDS slot of the lane's cell one row before
+        // the first, and the cells' offsets in a grid plane (-1: not an output)
+        constexpr int GROUPS = TY / NR;  // of rows per x block
+        const int xt = (NB > 1 ? 0 : wave / GROUPS * 16) + (lane & 15), r0 = wave % GROUPS * NR;
+        const int base = r0 * pitch + xt + d + half * L_::HALF;
+        int cell[NB][NR];
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            const int pos = (wave + 4 * j) * 16 + (lane & 15);
-            const int row = pos / S.XW, x = pos - row * S.XW;
-            const int y = w.ry + d * (w.y0 + row);
-            const bool ok = pos < npos && w.x0 + x < X && y < S.Y;
-            base[j] = (pos < npos ? (row + 1) * pitch + x + d : pitch + d) + half * L_::HALF;
-            cell[j] = ok ? w.x0 + x + X * y : -1;
-        }
+        for (int k = 0; k < NB; ++k)
+#pragma unroll
+            for (int j = 0; j < NR; ++j) {
+                const int x = xt + 16 * k, y = w.ry + d * (w.y0 + r0 + j);
+                cell[k][j] = x < S.XW && w.x0 + x < X && y < S.Y ? w.x0 + x + X * y : -1;
+            }
         fetch(w.z0 - 1);
         stash(w.z0 - 1);
         fetch(w.z0);
@@ -275,31 +281,41 @@ k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
             stash(zz + 1);
             __syncthreads();
             if (zz + 1 < w.z1) fetch(zz + 2);
-            f32x4 acc[NT];
+            f32x4 acc[NB][NR];
 #pragma unroll
-            for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int k = 0; k < NB; ++k)
+#pragma unroll
+                for (int j = 0; j < NR; ++j) acc[k][j] = f32x4{0.f, 0.f, 0.f, 0.f};
             const int s0 = ((zz + 2) % 3) * 2 * L_::HALF, s1 = (zz % 3) * 2 * L_::HALF,
                       s2 = ((zz + 1) % 3) * 2 * L_::HALF;
 #pragma unroll
             for (int p = 0; p < PAIRS_S; ++p) {
                 auto tap = [&](int m) {
-                    return (m / 9 == 0 ? s0 : m / 9 == 1 ? s1 : s2) +
-                           (m / 3 % 3 - 1) * pitch + (m % 3 - 1) * d;
+                    return (m / 3 == 0 ? s0 : m / 3 == 1 ? s1 : s2) + (m % 3 - 1) * d;
                 };
-                const int o = sub ? tap(2 * p + 1 < NS ? 2 * p + 1 : 2 * p) : tap(2 * p);
+                const int o = base + (sub && 2 * p + 1 < 9 ? tap(2 * p + 1) : tap(2 * p));
 #pragma unroll
-                for (int j = 0; j < NT; ++j) {
-                    bf16x8 b = flat[base[j] + o];
-                    if (2 * p + 1 >= NS && sub) b = bf16x8{};  // the pair's missing tap
-                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[p], b, acc[j], 0, 0, 0);
-                }
+                for (int row = 0; row < NR + 2; ++row)
+#pragma unroll
+                    for (int k = 0; k < NB; ++k) {
+                        bf16x8 b = flat[o + row * pitch + 16 * k];
+                        if (2 * p + 1 >= 9 && sub) b = bf16x8{};  // the pair's missing tap
+#pragma unroll
+                        for (int dy = 0; dy < 3; ++dy) {
+                            const int j = row - dy;
+                            if (j < 0 || j >= NR) continue;
+                            f32x4 &a = acc[k][j < 0 ? 0 : j < NR ? j : 0];
+                            a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[p][dy], b, a, 0, 0, 0);
+                        }
+                    }
             }
             const int64_t zb = tb + plane * (w.rz + d * zz);
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                if (cell[j] < 0) continue;
-                const int64_t o = (zb + cell[j]) * C + 4 * grp;
-                f32x4 v = acc[j];
+            for (int j = 0; j < NB * NR; ++j) {
+                const int cl = cell[j / NR][j % NR];
+                if (cl < 0) continue;
+                const int64_t o = (zb + cl) * C + 4 * grp;
+                f32x4 v = acc[j / NR][j % NR];
                 if (MODE == SP_FWD) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v[r] += bias[4 * grp + r];
@@ -493,20 +509,20 @@ k_time(const unsigned short *__restrict__ in, const s16x4 *__restrict__ wf,
 // A fragments of a space conv (16x16x32, two taps) from W[tap][in][out]
 // (FP32).  transpose: the backward data pass, whose "out" channel is W's
 // input channel and whose taps are mirrored.
-__global__ void k_pack_frag(const float *__restrict__ W, bf16x8 *__restrict__ wf, int ntaps,
-                            int npairs, int transpose)
+__global__ void k_pack_frag(const float *__restrict__ W, bf16x8 *__restrict__ wf, int transpose)
 {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= npairs * 64) return;
-    const int p = idx >> 6, lane = idx & 63;
+    if (idx >= PAIRS_S * 3 * 64) return;
+    const int p = idx / 192, dy = idx / 64 % 3, lane = idx & 63;
     const int o = lane & 15, grp = lane >> 4;
-    const int m = 2 * p + (grp >> 1);
+    const int zx = 2 * p + (grp >> 1);  // the (z, x) tap
+    const int m = zx / 3 * 9 + dy * 3 + zx % 3;
     float v[8];
     for (int q = 0; q < 8; ++q) {
         const int ii = 8 * (grp & 1) + q;
         float w = 0.f;
-        if (m < ntaps)
-            w = transpose ? W[((ntaps - 1 - m) * C + o) * C + ii] : W[(m * C + ii) * C + o];
+        if (zx < 9)
+            w = transpose ? W[((NS - 1 - m) * C + o) * C + ii] : W[(m * C + ii) * C + o];
         v[q] = w;
     }
     wf[idx] = pack8(make_float4(v[0], v[1], v[2], v[3]), make_float4(v[4], v[5], v[6], v[7]));
@@ -960,7 +976,7 @@ namespace {
 
 // 16-byte fragment slots per block: space fwd, space bwd, time fwd, time bwd
 // (the time fragments are 8 bytes per lane)
-constexpr int FRAG_S = PAIRS_S * 64, FRAG_T = NTT * 64 / 2;
+constexpr int FRAG_S = PAIRS_S * 3 * 64, FRAG_T = NTT * 64 / 2;
 constexpr int FRAG_BLK = 2 * FRAG_S + 2 * FRAG_T;
 
 void pack_all(flof_warmnet *net)
@@ -970,9 +986,9 @@ void pack_all(flof_warmnet *net)
         const float *blk = net->P + OFF_BLK + b * BLK_SIZE;
         bf16x8 *f = net->frag + (size_t)b * FRAG_BLK;
         hipLaunchKernelGGL(k_pack_frag, dim3((FRAG_S + 255) / 256), dim3(256), 0, ctx->stream,
-                           blk + BLK_WS, f, NS, PAIRS_S, 0);
+                           blk + BLK_WS, f, 0);
         hipLaunchKernelGGL(k_pack_frag, dim3((FRAG_S + 255) / 256), dim3(256), 0, ctx->stream,
-                           blk + BLK_WS, f + FRAG_S, NS, PAIRS_S, 1);
+                           blk + BLK_WS, f + FRAG_S, 1);
         hipLaunchKernelGGL(k_pack_frag_t, dim3(1), dim3(256), 0, ctx->stream, blk + BLK_WT,
                            (s16x4 *)(f + 2 * FRAG_S), 0);
         hipLaunchKernelGGL(k_pack_frag_t, dim3(1), dim3(256), 0, ctx->stream, blk + BLK_WT,
@@ -1044,12 +1060,11 @@ void launch_space(flof_ctx *ctx, const In &in, const bf16x8 *wf, const float *bi
                   const float *res, float *out_f, unsigned short *out_b, float *colsum,
                   const SpaceGeo &S)
 {
-    // 16-position tiles per wavefront; two, four, six and eight are built
-    const int nt = (8 * S.XW + 63) / 64;
-    auto k = nt <= 2   ? k_space<LIFT, MODE, 2>
-             : nt <= 4 ? k_space<LIFT, MODE, 4>
-             : nt <= 6 ? k_space<LIFT, MODE, 6>
-                       : k_space<LIFT, MODE, 8>;
+    // the workgroup's eight rows of x blocks over its four wavefronts
+    auto k = S.XW <= 16   ? k_space<LIFT, MODE, 2, 1>
+             : S.XW <= 32 ? k_space<LIFT, MODE, 4, 1>
+             : S.XW <= 48 ? k_space<LIFT, MODE, 2, 3>
+                          : k_space<LIFT, MODE, 8, 1>;
     hipLaunchKernelGGL(k, dim3(space_blocks(S)), dim3(256), 0, ctx->stream, in.b, in.i0, in.i1,
                        in.P, wf, bias, res, out_f, out_b, colsum, S);
     check_launch("k_space");

@@ -73,7 +73,8 @@ def test_gradients_match_oracle():
         assert rel < 3e-2, name
 
 
-@pytest.mark.parametrize("shape", [(3, 5, 9, 17), (9, 18, 3, 65), (17, 2, 33, 5), (1, 9, 8, 48)])
+@pytest.mark.parametrize("shape", [(3, 5, 9, 17), (9, 18, 3, 65), (17, 2, 33, 5), (1, 9, 8, 48),
+                                   (2, 3, 11, 61)])
 def test_network_tile_edges_match_oracle(shape):
     """Forward pass and gradients on grids whose rows fill the 16-cell tiles
     unevenly (17, 48 and 5 wide), span two x tiles (65), have fewer rows,
