@@ -45,8 +45,9 @@ B_DIR = (B_DIR_EVEN + B_DIR_ODD) / 2  # per iteration
 B_ITER_MIN = 112                 # x,r,p read+written once, g read once
 # kernel names of the PCG launch kinds on the finest level: the library runs
 # the LDS-tiled stencil kernels there (64^4, FP32: long t segments of full
-# tiles) and the t-marching ones on the coarser levels; FLOF_LDS_STENCIL=0
-# selects the t-marching kernels everywhere
+# tiles); the coarser levels run as one resident launch each, or, while their
+# kernels are timed, the t-marching ones; FLOF_LDS_STENCIL=0 selects the
+# t-marching kernels everywhere
 LDS_STENCIL = os.environ.get("FLOF_LDS_STENCIL", "auto")[:1] != "0"
 KN_UPDATE = "k_cg_stencil_lds<update>" if LDS_STENCIL else "k_cg_update_tm"
 KN_APPLY = "k_cg_stencil_lds<pq>" if LDS_STENCIL else "k_cg_pq_tm"
@@ -267,8 +268,9 @@ def main():
         "roofline": roofline,
         "kernels_finest_level": kst0,
         "kernels_all_levels": kst,
-        "kernels_all_levels_note": "per launch kind; the coarser levels run the "
-                                   "t-marching p.Ap and update kernels",
+        "kernels_all_levels_note": "per launch kind; while they are timed the coarser "
+                                   "levels run the t-marching kernels, otherwise "
+                                   "one resident launch each",
         "ms_per_step_with_kernel_events": 1000.0 * float(np.median(t_events)),
     }
 

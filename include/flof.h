@@ -173,8 +173,10 @@ int flof_ctx_tuned_shape(const flof_ctx *ctx, int X, int Y, int Z, int T, int *t
 /* Kernels of the PCG's two stencil passes, p.(A p) and the update (no
  * reference counterpart; results are identical): FLOF_STENCIL_LDS tiles
  * 64x4x4 cells in LDS, FLOF_STENCIL_TMARCH reads the neighbours through the
- * caches, FLOF_STENCIL_AUTO (the default) takes the LDS tiles for levels
- * where they are faster (FP32 direction storage, t segments of 16 or more
+ * caches, FLOF_STENCIL_AUTO (the default) runs all iterations of a level as
+ * one launch where its vectors fit the registers and LDS of the chip (up to
+ * about 1.3 million interior cells, FP32 direction storage, no timing of the
+ * iteration's kernels), takes the LDS tiles for levels where they are faster (FP32 direction storage, t segments of 16 or more
  * steps, X filling 90% of the 64-wide tiles) and the t-marching kernels
  * elsewhere; FLOF_STENCIL_QARRAY is the first GPU form (three streaming
  * kernels that store q = A p and g, 208 B per cell and iteration, FP32
@@ -568,9 +570,9 @@ int flof_warmnet_set_params(flof_warmnet *net, const float *host, int n);
 /* Gradient of the last flof_warmnet_loss_grad call. */
 int flof_warmnet_get_grads(flof_warmnet *net, float *host, int n);
 /* flow (VEC4, cells of the input grid) = net(i0, i1).  The training entries
- * (forward, loss_grad) keep every activation for the backward pass and take
- * grids below 2^31/16 cells; the solver's own inference (the _net solve)
- * takes larger ones. */
+ * (forward, loss_grad) take grids below 2^31/16 cells, loss_grad keeps every
+ * activation for the backward pass; the solver's own inference (the _net
+ * solve) takes larger grids. */
 int flof_warmnet_forward(flof_warmnet *net, flof_grid4d *i0, flof_grid4d *i1,
                          flof_grid4d *flow);
 /* Mean squared error against target (VEC4) and its gradient (kept in the
