@@ -33,7 +33,8 @@
 // outer loop's values right after a divergent loop was seen to be emitted
 // before the execution mask is restored, so that r of some lanes was lost
 // (wrong sums from the second iteration on).  Hence fresh(), the loads
-// without conditions and the vectors declared inside the loop.
+// without conditions and the vectors declared inside the loop; a kernel that
+// was given scratch memory all the same is not launched.
 //
 // The launch is cooperative, so all workgroups are resident together.  A
 // workgroup that still waits after two seconds gives up and says so in a word
@@ -710,6 +711,12 @@ bool resident_iterate(flof_ctx *ctx, const std::vector<ResLevel> &levels,
                     : cpt <= 6 ? (const void *)k_cg_resident<6, false>
                     : cpt <= 8 ? (const void *)k_cg_resident<8, false>
                                : (const void *)k_cg_resident<R_CPT, true>;
+    // no form that a compiler gave scratch memory (see the top of the file)
+    hipFuncAttributes fa;
+    if (hipFuncGetAttributes(&fa, k) != hipSuccess || fa.localSizeBytes != 0) {
+        (void)hipGetLastError();
+        return false;
+    }
     const hipError_t e =
         hipLaunchCooperativeKernel(k, dim3(total), dim3(RT), args, 0, ctx->stream);
     if (e != hipSuccess) {
