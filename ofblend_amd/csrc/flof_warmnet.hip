@@ -16,18 +16,21 @@
 //   network sees 31 cells in x, y, z and t: as far as the flows reach
 //   flow = head(h)                              pointwise 16 -> 4
 // The convolutions run on the matrix cores with BF16 weights and BF16-rounded
-// inputs, FP32 accumulation.  A value that only feeds convolutions (a, and
+// inputs, FP32 accumulation (tap after tap, two per instruction).  A value that only feeds convolutions (a, and
 // the copies of h, dh and ds that they read) is stored in BF16, rounded once
 // as the convolutions would round it; the residual chain h and its gradient
-// stay FP32.  A wavefront computes out^T (16 channels x 16 cells), in the
-// space convolutions for two taps per instruction (16x16x32):
+// stay FP32.  A wavefront computes out^T (16 channels x 16 cells) for two
+// taps per instruction (16x16x32):
 //   A (16 x 32) = weights   lane l: out channel l%16, k = 8*(l/16) .. +7
 //   B (32 x 16) = inputs    lane l: cell l%16,        k = 8*(l/16) .. +7
 //   D (16 x 16) = out^T     lane l: cell l%16, out channels 4*(l/16) .. +3
-// with k = 16*(tap - 2*pair) + input channel, in the time convolutions for one
-// (16x16x16, 4 channels per lane).  The backward data pass is the same kernel
-// with mirrored taps and transposed weights; the weight gradients have the
-// cells as the reduction dimension.  Training is Adam on FP32 master weights.
+// with k = 16*(tap - 2*pair) + input channel.  The order of a sum's taps and
+// their pairing decide its roundings, and through them which BF16 neighbour the
+// next layer reads: they are part of the network's definition here, so that a
+// flow does not change with the kernel that computes it.  The backward data
+// pass is the same kernel with mirrored taps and transposed weights; the weight
+// gradients have the cells as the reduction dimension.  Training is Adam on
+// FP32 master weights.
 
 #include <algorithm>
 #include <cmath>
@@ -44,7 +47,8 @@ constexpr int C = 16;       // channels
 constexpr int NB = 4;       // residual blocks
 constexpr int NS = 27;      // space taps
 constexpr int NTT = 3;      // time taps
-constexpr int PAIRS_S = 5;  // the nine (z, x) taps by two, each with its three y taps
+constexpr int PAIRS_S = 14;  // ceil(27 / 2)
+constexpr int PAIRS_T = 2;   // ceil(3 / 2)
 
 // parameter layout (FP32, flat)
 constexpr int OFF_WL = 0;                   // [2][16]
@@ -120,15 +124,19 @@ __device__ __forceinline__ float lift(const float *__restrict__ P, int o, float 
 // side, zero outside the grid) and marches through the planes of its z class,
 // keeping three haloed planes in LDS as BF16 (the two 8-channel halves apart,
 // so that the 16 lanes of an operand read 256 contiguous bytes).  Every input
-// value is loaded about 1.25 times from memory and read 11 to 18 times from LDS;
+// value is loaded about 1.25 times from memory and read 23 times from LDS;
 // the form that gathered the taps from memory read 27 x 64 bytes per cell
 // through the vector caches and rounded each value 27 times.
 // A wavefront computes rows of a block of 16 x cells, with the weights in
-// registers.  An operand is a row's 16 cells under two of the nine (z, x) taps,
-// and serves the three output rows that see this row under their three y taps:
-// 50 LDS reads and 120 MFMA for eight rows instead of 112 of each.  64^4: 449
-// -> 409 us (167 at the rate of memory; what is left is instruction issue, and
-// the two barriers per plane with two workgroups per CU to cover them).
+// registers.  An operand is a row's 16 cells under the two taps of a pair.  The
+// taps are taken in order, so most pairs' operands serve one output row; in
+// each z plane one pair recurs two rows further on (the first two x taps of the
+// rows y - 1 and y + 1, in the middle plane the last two) and is kept in
+// registers in between: 94 LDS reads and 112 MFMA for eight rows.
+// 64^4: 442 us (167 at the rate of memory); one read per MFMA 449, and taps
+// paired over (z, x), whose operands serve three output rows each, 409, but
+// that order of the sums gives another flow.  What is left is instruction issue,
+// and the two barriers per plane with two workgroups per CU to cover them.
 struct SpaceGeo {
     int X, Y, Z, T, d;
     int nxt, XW;      // x tiles and their width
@@ -197,11 +205,9 @@ k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
         const int d = S.d, pitch = S.pitch, X = S.X;
         const int64_t plane = (int64_t)X * S.Y;
         const int64_t tb = plane * S.Z * w.t;
-        bf16x8 wr[PAIRS_S][3];
+        bf16x8 wr[PAIRS_S];
 #pragma unroll
-        for (int p = 0; p < PAIRS_S; ++p)
-#pragma unroll
-            for (int dy = 0; dy < 3; ++dy) wr[p][dy] = wf[(p * 3 + dy) * 64 + lane];
+        for (int p = 0; p < PAIRS_S; ++p) wr[p] = wf[p * 64 + lane];
         // staged elements of this thread: 16-byte half sh of halo cells e; the
         // two halves of a cell by neighbouring lanes, or (the lift, whose
         // weights are then scalars of one half) by wavefronts
@@ -288,25 +294,31 @@ k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
                 for (int j = 0; j < NR; ++j) acc[k][j] = f32x4{0.f, 0.f, 0.f, 0.f};
             const int s0 = ((zz + 2) % 3) * 2 * L_::HALF, s1 = (zz % 3) * 2 * L_::HALF,
                       s2 = ((zz + 1) % 3) * 2 * L_::HALF;
+            bf16x8 keep[NB][NR + 2];  // operands of the pair that recurs, by row
 #pragma unroll
             for (int p = 0; p < PAIRS_S; ++p) {
                 auto tap = [&](int m) {
-                    return (m / 3 == 0 ? s0 : m / 3 == 1 ? s1 : s2) + (m % 3 - 1) * d;
+                    return (m / 9 == 0 ? s0 : m / 9 == 1 ? s1 : s2) + m / 3 % 3 * pitch +
+                           (m % 3 - 1) * d;
                 };
-                const int o = base + (sub && 2 * p + 1 < 9 ? tap(2 * p + 1) : tap(2 * p));
+                const int o = base + (sub && 2 * p + 1 < NS ? tap(2 * p + 1) : tap(2 * p));
+                const bool first = p == 0 || p == 5 || p == 9;    // taps 0 1, 10 11, 18 19
+                const bool again = p == 3 || p == 8 || p == 12;   // taps 6 7, 16 17, 24 25
+                if (first)
 #pragma unroll
-                for (int row = 0; row < NR + 2; ++row)
+                    for (int row = 0; row < NR + 2; ++row)
+#pragma unroll
+                        for (int k = 0; k < NB; ++k) keep[k][row] = flat[o + row * pitch + 16 * k];
+#pragma unroll
+                for (int j = 0; j < NR; ++j)
 #pragma unroll
                     for (int k = 0; k < NB; ++k) {
-                        bf16x8 b = flat[o + row * pitch + 16 * k];
-                        if (2 * p + 1 >= 9 && sub) b = bf16x8{};  // the pair's missing tap
-#pragma unroll
-                        for (int dy = 0; dy < 3; ++dy) {
-                            const int j = row - dy;
-                            if (j < 0 || j >= NR) continue;
-                            f32x4 &a = acc[k][j < 0 ? 0 : j < NR ? j : 0];
-                            a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[p][dy], b, a, 0, 0, 0);
-                        }
+                        bf16x8 b = first   ? keep[k][j]
+                                   : again ? keep[k][j + 2]
+                                           : flat[o + j * pitch + 16 * k];
+                        if (2 * p + 1 >= NS && sub) b = bf16x8{};  // the pair's missing tap
+                        acc[k][j] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[p], b, acc[k][j], 0, 0, 0);
                     }
             }
             const int64_t zb = tb + plane * (w.rz + d * zz);
@@ -357,15 +369,18 @@ k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
 // The 3-tap time convolution.  A wavefront owns 64 consecutive cells of the 3D
 // grid (four tiles of 16) and marches through the t steps of one class mod d,
 // the BF16 inputs at t - d, t, t + d in registers and the next one requested a
-// step ahead, so every input is read once.  MFMA 16x16x16, one tap each: a
-// lane's operand (4 channels of one cell) has the layout of the result, so
-// loads, residual and stores are all 8 or 16 bytes per lane of one contiguous
-// stretch.  Bound by memory: forward 32 + 64 bytes read and 64 + 32 written
-// per cell (64^4: 0.52 ms, 6.2 TB/s; 1.03 ms before, reading each input three
-// times in FP32).
+// step ahead, so every input is read once.  An MFMA takes the taps t - d (lanes
+// 0..31) and t (lanes 32..63), a second one t + d alone.  A load brings the two
+// 16-byte halves of 32 cells; a swap of the wavefront's halves turns it into
+// the operands of two tiles with the cells in both halves, from which each tap
+// takes its own.  Residual and stores have the layout of the result, 8 or 16
+// bytes per lane of one contiguous stretch.  Bound by memory: forward 32 + 64
+// bytes read and 64 + 32 written per cell.  64^4: 0.56 ms, 5.7 TB/s, the head's
+// step 0.40 (1.03 ms before, reading each input three times in FP32).
 // TM_FWD: v = res + (conv + bias); out_f (optional) = v, out_b (optional) =
-// bf16(v); flow (optional) = the head of v, FP32 on the matrix cores
-// (16x16x4: the head's 4 outputs are rows 0..3 of the result).
+// bf16(v); flow (optional) = the head of v: every lane gathers its cell's 16
+// channels from the four lanes that hold them and sums one of the outputs,
+// channel after channel.
 // TM_BWD: v = conv where the mask tensor is positive, else 0; out_b = bf16(v),
 // and the workgroup's column sums of v (the space bias gradient).
 enum { TM_FWD = 0, TM_BWD = 1 };
@@ -376,9 +391,9 @@ struct TimeGeo {
     int klen, nseg;  // steps of a class per segment, segments
     int total;       // workgroups of 4 stretches: ceil(nch / 4) * d * nseg
 };
-template <bool LIFT, int MODE>
+template <bool LIFT, int MODE, bool HEAD>
 __global__ void __launch_bounds__(256)
-k_time(const unsigned short *__restrict__ in, const s16x4 *__restrict__ wf,
+k_time(const unsigned short *__restrict__ in, const bf16x8 *__restrict__ wf,
        const float *__restrict__ bias, const float *__restrict__ res, In lin,
        const unsigned short *__restrict__ mask, float *__restrict__ out_f,
        unsigned short *__restrict__ out_b, const float *__restrict__ P,
@@ -394,19 +409,16 @@ k_time(const unsigned short *__restrict__ in, const s16x4 *__restrict__ wf,
     const int kc = (G.T - rt + G.d - 1) / G.d;  // steps of the class
     const int k0 = seg * G.klen, k1 = min(k0 + G.klen, kc);
     if (ch < G.nch && rt < G.T && k0 < k1) {
-        const s16x4 w0 = wf[lane], w1 = wf[64 + lane], w2 = wf[128 + lane];
+        const bf16x8 w0 = wf[lane], w1 = wf[64 + lane];
         f32x4 bs = {0.f, 0.f, 0.f, 0.f};
         if (MODE == TM_FWD)
 #pragma unroll
             for (int r = 0; r < 4; ++r) bs[r] = bias[4 * grp + r];
-        float wh[4];
-        f32x4 bh = {0.f, 0.f, 0.f, 0.f};
-        if (flow) {
+        float wh[C], bh = 0.f;
+        if (HEAD) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                wh[r] = (lane & 15) < 4 ? P[OFF_WH + (4 * grp + r) * 4 + (lane & 15)] : 0.f;
-                bh[r] = grp == 0 ? P[OFF_BH + r] : 0.f;
-            }
+            for (int i = 0; i < C; ++i) wh[i] = P[OFF_WH + i * 4 + grp];
+            bh = P[OFF_BH + grp];
         }
         float l0[4], l1[4], lb[4];
         if (LIFT) {
@@ -425,23 +437,44 @@ k_time(const unsigned short *__restrict__ in, const s16x4 *__restrict__ wf,
             ok[j] = c3[j] < G.n3;
             if (!ok[j]) c3[j] = 0;
         }
-        s16x4 am[4], ac[4], ap[4];
-        auto load = [&](s16x4 (&a)[4], int k) {
+        // the 16-byte half (lane >> 4) & 1 of cells 32 q + 16 (lane >> 5) + lane % 16
+        const bool upper = lane >= 32;
+        int64_t cl[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            cl[q] = (int64_t)ch * 64 + 32 * q + (upper ? 16 : 0) + (lane & 15);
+            if (cl[q] >= G.n3) cl[q] = 0;
+        }
+        auto load = [&](u32x4 (&a)[2], int k) {
             const int t = rt + G.d * k;
             const bool in_t = k >= 0 && t < G.T;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                a[j] = s16x4{0, 0, 0, 0};
-                if (in_t) a[j] = *(const s16x4 *)(in + (c3[j] + G.n3 * t) * C + 4 * grp);
+            for (int q = 0; q < 2; ++q) {
+                a[q] = u32x4{0, 0, 0, 0};
+                if (in_t) a[q] = *(const u32x4 *)(in + (cl[q] + G.n3 * t) * C + 8 * (grp & 1));
             }
         };
-        load(am, k0 - 1);
-        load(ac, k0);
-        load(ap, k0 + 1);
+        // the four tiles of a step, each in both halves of the wavefront
+        auto spread = [&](const u32x4 (&a)[2], u32x4 (&b)[4]) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const auto v = __builtin_amdgcn_permlane32_swap(a[q][r], a[q][r], false, false);
+                    b[2 * q][r] = v[0];
+                    b[2 * q + 1][r] = v[1];
+                }
+        };
+        u32x4 raw[2], am[4], ac[4], ap[4];
+        load(raw, k0 - 1);
+        spread(raw, am);
+        load(raw, k0);
+        spread(raw, ac);
+        load(raw, k0 + 1);
         for (int k = k0; k < k1; ++k) {
             const int t = rt + G.d * k;
-            s16x4 an[4];
-            if (k + 1 < k1) load(an, k + 2);
+            spread(raw, ap);
+            if (k + 1 < k1) load(raw, k + 2);
             f32x4 rs[4];
             s16x4 mk[4];
 #pragma unroll
@@ -460,9 +493,16 @@ k_time(const unsigned short *__restrict__ in, const s16x4 *__restrict__ wf,
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 f32x4 v = {0.f, 0.f, 0.f, 0.f};
-                v = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w0, am[j], v, 0, 0, 0);
-                v = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w1, ac[j], v, 0, 0, 0);
-                v = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w2, ap[j], v, 0, 0, 0);
+                u32x4 b0, b1;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    b0[r] = upper ? ac[j][r] : am[j][r];
+                    b1[r] = upper ? 0u : ap[j][r];
+                }
+                v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, __builtin_bit_cast(bf16x8, b0), v,
+                                                            0, 0, 0);
+                v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, __builtin_bit_cast(bf16x8, b1), v,
+                                                            0, 0, 0);
                 const int64_t c = c3[j] + G.n3 * t;
                 if (MODE == TM_FWD) {
 #pragma unroll
@@ -471,12 +511,25 @@ k_time(const unsigned short *__restrict__ in, const s16x4 *__restrict__ wf,
                         if (out_f) *(f32x4 *)(out_f + c * C + 4 * grp) = v;
                         if (out_b) *(u16x4 *)(out_b + c * C + 4 * grp) = pack4(v);
                     }
-                    if (flow) {
-                        f32x4 f = bh;
+                    if (HEAD) {
+                        // hv[4 g + r]: channel r of lane group g
+                        float hv[C];
 #pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            f = __builtin_amdgcn_mfma_f32_16x16x4f32(wh[r], v[r], f, 0, 0, 0);
-                        if (ok[j] && grp == 0) flow[c] = make_float4(f[0], f[1], f[2], f[3]);
+                        for (int r = 0; r < 4; ++r) {
+                            const unsigned u = __float_as_uint(v[r]);
+                            const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+#pragma unroll
+                            for (int g = 0; g < 2; ++g) {
+                                const auto e = __builtin_amdgcn_permlane16_swap(h[g], h[g], false,
+                                                                                false);
+                                hv[8 * g + r] = __uint_as_float(e[0]);
+                                hv[8 * g + 4 + r] = __uint_as_float(e[1]);
+                            }
+                        }
+                        float f = bh;
+#pragma unroll
+                        for (int i = 0; i < C; ++i) f += wh[i] * hv[i];
+                        if (ok[j]) ((float *)flow)[4 * c + grp] = f;
                     }
                 } else {
 #pragma unroll
@@ -488,7 +541,6 @@ k_time(const unsigned short *__restrict__ in, const s16x4 *__restrict__ wf,
                 }
                 am[j] = ac[j];
                 ac[j] = ap[j];
-                ap[j] = an[j];
             }
         }
     }
@@ -506,40 +558,26 @@ k_time(const unsigned short *__restrict__ in, const s16x4 *__restrict__ wf,
     }
 }
 
-// A fragments of a space conv (16x16x32, two taps) from W[tap][in][out]
-// (FP32).  transpose: the backward data pass, whose "out" channel is W's
-// input channel and whose taps are mirrored.
-__global__ void k_pack_frag(const float *__restrict__ W, bf16x8 *__restrict__ wf, int transpose)
+// A fragments of a conv (16x16x32, two taps) from W[tap][in][out] (FP32).
+// transpose: the backward data pass, whose "out" channel is W's input channel
+// and whose taps are mirrored.
+__global__ void k_pack_frag(const float *__restrict__ W, bf16x8 *__restrict__ wf, int ntaps,
+                            int npairs, int transpose)
 {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= PAIRS_S * 3 * 64) return;
-    const int p = idx / 192, dy = idx / 64 % 3, lane = idx & 63;
+    if (idx >= npairs * 64) return;
+    const int p = idx >> 6, lane = idx & 63;
     const int o = lane & 15, grp = lane >> 4;
-    const int zx = 2 * p + (grp >> 1);  // the (z, x) tap
-    const int m = zx / 3 * 9 + dy * 3 + zx % 3;
+    const int m = 2 * p + (grp >> 1);
     float v[8];
     for (int q = 0; q < 8; ++q) {
         const int ii = 8 * (grp & 1) + q;
         float w = 0.f;
-        if (zx < 9)
-            w = transpose ? W[((NS - 1 - m) * C + o) * C + ii] : W[(m * C + ii) * C + o];
+        if (m < ntaps)
+            w = transpose ? W[((ntaps - 1 - m) * C + o) * C + ii] : W[(m * C + ii) * C + o];
         v[q] = w;
     }
     wf[idx] = pack8(make_float4(v[0], v[1], v[2], v[3]), make_float4(v[4], v[5], v[6], v[7]));
-}
-// the same for the time conv (16x16x16, one tap)
-__global__ void k_pack_frag_t(const float *__restrict__ W, s16x4 *__restrict__ wf, int transpose)
-{
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= NTT * 64) return;
-    const int m = idx >> 6, lane = idx & 63;
-    const int o = lane & 15, grp = lane >> 4;
-    u16x4 u;
-    for (int q = 0; q < 4; ++q) {
-        const int ii = 4 * grp + q;
-        u[q] = to_bf16(transpose ? W[((NTT - 1 - m) * C + o) * C + ii] : W[(m * C + ii) * C + o]);
-    }
-    wf[idx] = __builtin_bit_cast(s16x4, u);
 }
 
 // ---------------------------------------------------------------------------
@@ -975,8 +1013,7 @@ struct flof_warmnet {
 namespace {
 
 // 16-byte fragment slots per block: space fwd, space bwd, time fwd, time bwd
-// (the time fragments are 8 bytes per lane)
-constexpr int FRAG_S = PAIRS_S * 3 * 64, FRAG_T = NTT * 64 / 2;
+constexpr int FRAG_S = PAIRS_S * 64, FRAG_T = PAIRS_T * 64;
 constexpr int FRAG_BLK = 2 * FRAG_S + 2 * FRAG_T;
 
 void pack_all(flof_warmnet *net)
@@ -986,13 +1023,13 @@ void pack_all(flof_warmnet *net)
         const float *blk = net->P + OFF_BLK + b * BLK_SIZE;
         bf16x8 *f = net->frag + (size_t)b * FRAG_BLK;
         hipLaunchKernelGGL(k_pack_frag, dim3((FRAG_S + 255) / 256), dim3(256), 0, ctx->stream,
-                           blk + BLK_WS, f, 0);
+                           blk + BLK_WS, f, NS, PAIRS_S, 0);
         hipLaunchKernelGGL(k_pack_frag, dim3((FRAG_S + 255) / 256), dim3(256), 0, ctx->stream,
-                           blk + BLK_WS, f + FRAG_S, 1);
-        hipLaunchKernelGGL(k_pack_frag_t, dim3(1), dim3(256), 0, ctx->stream, blk + BLK_WT,
-                           (s16x4 *)(f + 2 * FRAG_S), 0);
-        hipLaunchKernelGGL(k_pack_frag_t, dim3(1), dim3(256), 0, ctx->stream, blk + BLK_WT,
-                           (s16x4 *)(f + 2 * FRAG_S + FRAG_T), 1);
+                           blk + BLK_WS, f + FRAG_S, NS, PAIRS_S, 1);
+        hipLaunchKernelGGL(k_pack_frag, dim3(1), dim3(256), 0, ctx->stream, blk + BLK_WT,
+                           f + 2 * FRAG_S, NTT, PAIRS_T, 0);
+        hipLaunchKernelGGL(k_pack_frag, dim3(1), dim3(256), 0, ctx->stream, blk + BLK_WT,
+                           f + 2 * FRAG_S + FRAG_T, NTT, PAIRS_T, 1);
     }
     check_launch("k_pack_frag");
     net->frag_ok = true;
@@ -1088,8 +1125,11 @@ void time_fwd(flof_ctx *ctx, const unsigned short *a, const bf16x8 *wf, const fl
               float4 *flow, const Geo &g)
 {
     const TimeGeo G = time_geo(g);
-    auto k = res ? k_time<false, TM_FWD> : k_time<true, TM_FWD>;
-    hipLaunchKernelGGL(k, dim3(G.total), dim3(256), 0, ctx->stream, a, (const s16x4 *)wf, bias,
+    // (the lift feeds block 0, the head follows block 3)
+    auto k = flow  ? k_time<false, TM_FWD, true>
+             : res ? k_time<false, TM_FWD, false>
+                   : k_time<true, TM_FWD, false>;
+    hipLaunchKernelGGL(k, dim3(G.total), dim3(256), 0, ctx->stream, a, wf, bias,
                        res, lin, nullptr, hf, hb, P, flow, nullptr, G);
     check_launch("k_time");
 }
@@ -1228,8 +1268,8 @@ double loss_grad(flof_warmnet *net, const float *i0, const float *i1, const floa
         {
             const TimeGeo G = time_geo(g);
             Tmp cp(ctx, (size_t)G.total * C * 4);
-            hipLaunchKernelGGL((k_time<false, TM_BWD>), dim3(G.total), dim3(256), 0, ctx->stream,
-                               u16p(dhb), (const s16x4 *)(f + 2 * FRAG_S + FRAG_T), nullptr,
+            hipLaunchKernelGGL((k_time<false, TM_BWD, false>), dim3(G.total), dim3(256), 0, ctx->stream,
+                               u16p(dhb), f + 2 * FRAG_S + FRAG_T, nullptr,
                                nullptr, lin, u16p(A.ab[b]), nullptr, u16p(dsb), nullptr, nullptr,
                                cp.as<float>(), G);
             check_launch("k_time (backward)");

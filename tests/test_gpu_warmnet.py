@@ -1,6 +1,10 @@
 """The learned warm start on the GPU: the matrix-core forward and backward
 kernels against the CPU restatement (oracle/warmnet.py), a training run that
 lowers the loss, and the warm-started solve against the plain one."""
+import hashlib
+import json
+import os
+
 import numpy as np
 import pytest
 
@@ -223,3 +227,32 @@ def test_trained_network_saves_iterations_on_heldout_pairs():
     say("finest-level iterations, 3 held-out pairs: cold %d net %d (ratio %.3f)"
         % (cold_it, net_it, cold_it / net_it))
     assert net_it < cold_it
+
+
+FLOW_SHAPES = [(6, 8, 8, 16), (9, 18, 3, 65), (17, 2, 33, 5), (5, 9, 8, 48), (3, 20, 18, 30)]
+
+
+def flow_digest(shape):
+    """sha256 of the network's flow on a drop pair, by weights and inputs of
+    their own seeds."""
+    s, a, b, g0, g1 = _case(shape, seed=40)
+    net = WS.WarmNet(seed=9)
+    r = np.random.default_rng(41)
+    net.set_params((r.standard_normal(WS.num_params()) * 0.2).astype(np.float32))
+    flow = s.create(M.Grid4Vec4)
+    net.forward(g0, g1, flow)
+    return hashlib.sha256(np.ascontiguousarray(flow.to_numpy()).tobytes()).hexdigest()
+
+
+@pytest.mark.parametrize("shape", FLOW_SHAPES)
+def test_flow_is_the_gathering_kernels_flow(shape):
+    """The digests were recorded on an MI355X with convolutions that gathered
+    every tap of a 16-cell tile from memory, two consecutive taps per MFMA in
+    the order of the taps, and a head that summed a cell's channels one after
+    another.  Which kernel stages the inputs must not change a bit: another
+    order rounds some activations to the other BF16 neighbour, and the flow
+    then differs by parts in a thousand."""
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden",
+                        "warmnet_flow.json")
+    say("warmnet flow digest", shape)
+    assert flow_digest(shape) == json.load(open(path))["x".join(map(str, shape))]
