@@ -1774,7 +1774,8 @@ __device__ __forceinline__ void m5_load(float (&R)[25], const float *__restrict_
                                         const Dims4 &D, int p, unsigned es, unsigned off,
                                         bool ym, bool yp)
 {
-    const unsigned bytes = (unsigned)D.st * es;  // < 2^32 (checked by the host)
+    // (the host checks that no row's offset, in the plane or next to it, wraps)
+    const unsigned bytes = (unsigned)D.st * es;
     const bool in = p >= 0 && p < D.T;
     const char *b = (const char *)src + (in ? (int64_t)D.st * p * es : 0);
     const __amdgpu_buffer_rsrc_t rs =
@@ -1782,7 +1783,7 @@ __device__ __forceinline__ void m5_load(float (&R)[25], const float *__restrict_
 #pragma unroll
     for (int r = 0; r < 25; ++r) {
         const int dz = r / 5 - 2, dy = r % 5 - 2;
-        const unsigned row = (unsigned)((int)(D.sz * dz + D.X * dy) * (int)es);
+        const unsigned row = (unsigned)((D.sz * dz + (int64_t)D.X * dy) * (int)es);
         // the zero column's offset stays beyond the plane whatever the row
         unsigned o = off == 0xffffffffu ? off : off + row;
         if (dy == -2 && ym) o = 0xffffffffu;
@@ -1945,8 +1946,11 @@ void gaussian_blur(flof_ctx *ctx, void *a, const Dims4 &D, bool vec4, float sigm
     Blur5W w5{};
     Tmp wsum5;
     March3 M5{};
-    // (grids whose t-plane does not fit a 32-bit buffer take the gathering form)
-    const bool march5 = s == 2 && D.st * (vec4 ? 16 : 4) < (1ll << 32) - 64;
+    // A row's byte offset must not wrap: a plane and the two layers and rows by
+    // which a window can leave it stay below 2^32 (other grids take the
+    // gathering form)
+    const bool march5 =
+        s == 2 && (D.st + 2 * D.sz + 2 * (int64_t)D.X) * (vec4 ? 16 : 4) < (1ll << 32) - 64;
     if (march5) {
         for (int d = 0; d < 17; ++d) w5.w[d] = wh[d];
         std::vector<float> ws(256);

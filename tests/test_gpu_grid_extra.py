@@ -387,3 +387,34 @@ def test_marches_at_wavefront_and_segment_edges_bit_exact(shape):
     rd, rv = O.corr_vels_of4d(vel0, phiOrg, phiTgt, threshPhi=1.5, postVelBlur=0.0, maxIter=40)
     assert np.array_equal(dst.to_numpy(), rd)
     assert np.array_equal(vel.to_numpy(), rv)
+
+
+def test_blur_5_window_on_a_plane_near_the_buffer_limit():
+    """sigma 2 on a Vec4 grid whose t-planes (3.2 GB) end less than an xy
+    layer below 2^32 bytes: the window's z rows outside the grid count as
+    absent there too.  On a constant grid every cell away from the x and y
+    faces takes the value it takes on a small grid; a row that wrapped round
+    into the plane would change the rows next to the first and last."""
+    def blurred(n):
+        s = M.Solver(gridSize=M.vec3(n, n, 3), fourthDim=3)
+        g = s.create(M.Grid4Vec4)
+        g.setConst(M.Vec4(1.0, 3.0, -0.7, 4.0))
+        M.gaussianBlur4d(g, 2.0, 1)
+        return g
+
+    N = 8200
+    assert N * N * 3 * 16 < 2 ** 32 - 64 < N * N * 4 * 16
+    want = blurred(24).to_numpy()[1, 1, 12, 12]
+    say("blur on", (N, N, 3, 3), "expected", want)
+    g = blurred(N)
+    try:
+        mid = np.empty((N, N, 4), np.float32)  # z = 1, t = 1
+        p = _lib.lib().flof_grid4d_device_ptr(g.h) + 4 * mid.nbytes
+        _lib.check(_lib.lib().flof_dev_download(g.ctx, mid.ctypes.data_as(C.c_void_p),
+                                                C.c_void_p(p), mid.nbytes), g.ctx)
+        bad = int((mid[8:-8, 8:-8] != want).any(-1).sum())
+        say("cells that differ:", bad)
+        assert bad == 0
+    finally:
+        del g
+        _lib.lib().flof_ctx_trim(M.context())
