@@ -668,8 +668,10 @@ void advect_cfl(flof_ctx *ctx, const float4 *vel, void *grid, const Dims4 &D,
     const size_t bytes = (size_t)n * (vec4 ? 16 : 4);
     Tmp tmp(ctx, bytes);
     void *cur = grid, *next = tmp.p;
+    // a velocity that advects itself: each substep's is the last one's result
+    const bool self = (const void *)v == grid;
     for (int s = 0; s < steps; ++s) {
-        launch_advect(ctx, v, 1.f, cur, next, D, vec4, sdt);
+        launch_advect(ctx, self ? (const float4 *)cur : v, 1.f, cur, next, D, vec4, sdt);
         std::swap(cur, next);
     }
     if (cur != grid)

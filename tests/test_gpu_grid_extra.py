@@ -418,3 +418,26 @@ def test_blur_5_window_on_a_plane_near_the_buffer_limit():
     finally:
         del g
         _lib.lib().flof_ctx_trim(M.context())
+
+
+@pytest.mark.parametrize("steps", [1, 2, 3, 4])
+def test_advect_cfl_of_a_velocity_by_itself(steps):
+    """advectCfl4d of a velocity grid by itself: every substep moves the
+    velocities along those that the substep before left (the reference
+    advects in place, optflow4d.cpp:2170-2180), after odd and even numbers of
+    substeps."""
+    say("self-advection, substeps", steps)
+    T, Z, Y, X = 5, 6, 7, 9
+    rng = np.random.default_rng(50 + steps)
+    v = rng.standard_normal((T, Z, Y, X, 4)).astype(np.float32)
+    big = np.float32(np.sqrt((v * v).sum(-1)).max())
+    s = M.Solver(gridSize=M.vec3(X, Y, Z), fourthDim=T)
+    g = s.create(M.Grid4Vec4)
+    g.from_numpy(v)
+    cfl = float(big) / (steps - 0.5)
+    _lib.check(_lib.lib().flof_advect_cfl4d(g.h, g.h, cfl, 1.0, 1.0), g.ctx)
+    ref = v
+    dt = float(np.float32(1.0) / np.float32(steps))
+    for _ in range(steps):
+        ref = O.advect4d(ref, ref, dt=1.0, dtFac=dt)
+    assert np.array_equal(g.to_numpy(), ref)
