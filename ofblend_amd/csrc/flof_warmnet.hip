@@ -140,10 +140,12 @@ __device__ __forceinline__ float lift(const float *__restrict__ P, int o, float 
 struct SpaceGeo {
     int X, Y, Z, T, d;
     int nxt, XW;      // x tiles and their width
+    int nry, nrz;     // y and z classes that hold rows: min(d, Y), min(d, Z)
     int nyt, nzs;     // y tiles per y class, z segments per z class
     int zlen;         // planes per z segment
     int pitch;        // XW + 2 d
-    int total;        // work items
+    int total;        // work items: fewer than the cells
+    int first;        // the launch's first item
 };
 constexpr int SP_W = 64, SP_DMAX = 8;
 template <int TY> struct SpLds {
@@ -161,12 +163,12 @@ __device__ __forceinline__ bool sp_item(const SpaceGeo &S, int L, SpItem &w)
     int r = L;
     const int yt = r % S.nyt;
     r /= S.nyt;
-    w.ry = r % S.d;
-    r /= S.d;
+    w.ry = r % S.nry;
+    r /= S.nry;
     const int zs = r % S.nzs;
     r /= S.nzs;
-    w.rz = r % S.d;
-    r /= S.d;
+    w.rz = r % S.nrz;
+    r /= S.nrz;
     const int xt = r % S.nxt;
     w.t = r / S.nxt;
     w.x0 = xt * S.XW;
@@ -198,7 +200,7 @@ k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int grp = lane >> 4, sub = grp >> 1, half = grp & 1;
     const int per = (int)gridDim.x / FLOF_NXCD;  // the grid is a multiple of 8
-    const int L = ((int)blockIdx.x % FLOF_NXCD) * per + (int)blockIdx.x / FLOF_NXCD;
+    const int L = S.first + ((int)blockIdx.x % FLOF_NXCD) * per + (int)blockIdx.x / FLOF_NXCD;
     f32x4 cs = {0.f, 0.f, 0.f, 0.f};
     SpItem w;
     if (L < S.total && sp_item<TY>(S, L, w)) {  // uniform over the workgroup
@@ -360,7 +362,7 @@ k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
             for (int r = 0; r < 4; ++r) sh[wave][4 * grp + r] = cs[r];
         __syncthreads();
         if (tid < C)
-            colsum[(int64_t)blockIdx.x * C + tid] =
+            colsum[((int64_t)S.first + blockIdx.x) * C + tid] =
                 sh[0][tid] + sh[1][tid] + sh[2][tid] + sh[3][tid];
     }
 }
@@ -387,9 +389,10 @@ enum { TM_FWD = 0, TM_BWD = 1 };
 struct TimeGeo {
     int64_t n3;
     int T, d;
+    int nr;          // t classes that hold steps: min(d, T)
     int nch;         // stretches of 64 cells
     int klen, nseg;  // steps of a class per segment, segments
-    int total;       // workgroups of 4 stretches: ceil(nch / 4) * d * nseg
+    int total;       // workgroups of 4 stretches: ceil(nch / 4) * nr * nseg
 };
 template <bool LIFT, int MODE, bool HEAD>
 __global__ void __launch_bounds__(256)
@@ -404,7 +407,7 @@ k_time(const unsigned short *__restrict__ in, const bf16x8 *__restrict__ wf,
     int r_ = blockIdx.x;
     const int ch = (r_ % nwg) * 4 + wave;
     r_ /= nwg;
-    const int rt = r_ % G.d, seg = r_ / G.d;
+    const int rt = r_ % G.nr, seg = r_ / G.nr;
     f32x4 cs = {0.f, 0.f, 0.f, 0.f};
     const int kc = (G.T - rt + G.d - 1) / G.d;  // steps of the class
     const int k0 = seg * G.klen, k1 = min(k0 + G.klen, kc);
@@ -772,12 +775,12 @@ k_wgrad_time(const unsigned short *__restrict__ in, const unsigned short *__rest
     f32x4 acc[NTT];
 #pragma unroll
     for (int m = 0; m < NTT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int items = G.nch * G.d * G.nseg;
+    const int items = G.nch * G.nr * G.nseg;
     for (int it = blockIdx.x * 4 + wave; it < items; it += gridDim.x * 4) {
         int r_ = it;
         const int chn = r_ % G.nch;
         r_ /= G.nch;
-        const int rt = r_ % G.d, seg = r_ / G.d;
+        const int rt = r_ % G.nr, seg = r_ / G.nr;
         const int kc = (G.T - rt + G.d - 1) / G.d;
         const int k0 = seg * G.klen, k1 = min(k0 + G.klen, kc);
         if (rt >= G.T || k0 >= k1) continue;
@@ -1053,16 +1056,19 @@ SpaceGeo space_geo(const Geo &g, int ty, int want)
     S.d = g.dil;
     S.nxt = (g.X + SP_W - 1) / SP_W;
     S.XW = (g.X + S.nxt - 1) / S.nxt;
+    S.nry = std::min(g.dil, g.Y);
+    S.nrz = std::min(g.dil, g.Z);
     S.nyt = ((g.Y + g.dil - 1) / g.dil + ty - 1) / ty;
     const int zc = (g.Z + g.dil - 1) / g.dil;
-    const int64_t cols = (int64_t)g.T * S.nxt * S.nyt * g.dil * g.dil;
+    const int64_t cols = (int64_t)g.T * S.nxt * S.nyt * S.nry * S.nrz;
     const int most = std::max(1, zc / 4);
     S.nzs = (int)std::max<int64_t>(1, std::min<int64_t>(most, (want + cols - 1) / cols));
     S.zlen = (zc + S.nzs - 1) / S.nzs;
     S.nzs = (zc + S.zlen - 1) / S.zlen;
     S.pitch = S.XW + 2 * g.dil;
-    FLOF_REQUIRE(cols * S.nzs < (1ll << 31), FLOF_ERR_DIM, "warm-start net: grid too large");
+    // nyt nry <= Y and nzs nrz <= Z
     S.total = (int)(cols * S.nzs);
+    S.first = 0;
     return S;
 }
 int space_blocks(const SpaceGeo &S)
@@ -1077,14 +1083,15 @@ TimeGeo time_geo(const Geo &g)
     G.n3 = (int64_t)g.X * g.Y * g.Z;
     G.T = g.T;
     G.d = g.dil;
+    G.nr = std::min(g.dil, g.T);
     G.nch = (int)((G.n3 + 63) / 64);
     const int kc = (g.T + g.dil - 1) / g.dil;
-    const int64_t cols = (int64_t)G.nch * g.dil;
+    const int64_t cols = (int64_t)G.nch * G.nr;
     G.nseg = (int)std::max<int64_t>(
         1, std::min<int64_t>(std::max(1, kc / 4), (8192 + cols - 1) / cols));
     G.klen = (kc + G.nseg - 1) / G.nseg;
     G.nseg = (kc + G.klen - 1) / G.klen;
-    G.total = (G.nch + 3) / 4 * g.dil * G.nseg;
+    G.total = (G.nch + 3) / 4 * G.nr * G.nseg;
     return G;
 }
 
@@ -1102,8 +1109,17 @@ void launch_space(flof_ctx *ctx, const In &in, const bf16x8 *wf, const float *bi
              : S.XW <= 32 ? k_space<LIFT, MODE, 4, 1>
              : S.XW <= 48 ? k_space<LIFT, MODE, 2, 3>
                           : k_space<LIFT, MODE, 8, 1>;
-    hipLaunchKernelGGL(k, dim3(space_blocks(S)), dim3(256), 0, ctx->stream, in.b, in.i0, in.i1,
-                       in.P, wf, bias, res, out_f, out_b, colsum, S);
+    // A launch takes fewer than 2^32 threads, more would run as what is left
+    // of the count modulo 2^32: 2^23 workgroups each (thin grids with a long t).
+    constexpr int MOST = 1 << 23;
+    SpaceGeo part = S;
+    for (int at = 0; at < S.total; at += MOST) {
+        part.first = at;
+        part.total = std::min(S.total, at + MOST);
+        const int nb = (part.total - at + FLOF_NXCD - 1) / FLOF_NXCD * FLOF_NXCD;
+        hipLaunchKernelGGL(k, dim3(nb), dim3(256), 0, ctx->stream, in.b, in.i0, in.i1, in.P, wf,
+                           bias, res, out_f, out_b, colsum, part);
+    }
     check_launch("k_space");
 }
 
@@ -1219,7 +1235,7 @@ void wgrad_time(flof_ctx *ctx, const unsigned short *in, const unsigned short *d
                 float *dW)
 {
     const TimeGeo G = time_geo(g);
-    const int nbk = wgrad_blocks(ctx, (G.nch * G.d * G.nseg + 3) / 4);
+    const int nbk = wgrad_blocks(ctx, (G.nch * G.nr * G.nseg + 3) / 4);
     Tmp part(ctx, (size_t)nbk * 4 * NTT * C * C * 4);
     hipLaunchKernelGGL(k_wgrad_time, dim3(nbk), dim3(256), 0, ctx->stream, in, dout,
                        part.as<float>(), G);

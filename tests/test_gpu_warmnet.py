@@ -256,3 +256,52 @@ def test_flow_is_the_gathering_kernels_flow(shape):
                         "warmnet_flow.json")
     say("warmnet flow digest", shape)
     assert flow_digest(shape) == json.load(open(path))["x".join(map(str, shape))]
+
+
+@pytest.mark.parametrize("size", [(2, 2, 2, 270000), (1, 3, 2, 300001), (2, 270001, 2, 1)])
+def test_network_on_long_thin_grids(size):
+    """Grids of a few cells across and a long t (or y): more tiles times
+    dilation classes than one launch takes workgroups.  The flow of an inner
+    stretch is that of the stretch alone (the network sees 30 cells to each
+    side), and a training step's loss is the mean squared error of the flow."""
+    X, Y, Z, T = size
+    say("warmnet thin grid", size)
+    r = np.random.default_rng(60)
+    net = WS.WarmNet(seed=9)
+    net.set_params((r.standard_normal(WS.num_params()) * 0.2).astype(np.float32))
+
+    def run(a, b):
+        t, z, y, x = a.shape
+        s = M.Solver(gridSize=M.vec3(x, y, z), fourthDim=t)
+        g0, g1, fl = s.create(M.Grid4Real), s.create(M.Grid4Real), s.create(M.Grid4Vec4)
+        g0.from_numpy(a)
+        g1.from_numpy(b)
+        net.forward(g0, g1, fl)
+        return s, g0, g1, fl
+
+    a = r.standard_normal((T, Z, Y, X)).astype(np.float32)
+    b = r.standard_normal((T, Z, Y, X)).astype(np.float32)
+    s, g0, g1, fl = run(a, b)
+    flow = fl.to_numpy()
+    ax = 0 if T > Y else 2
+    n = max(T, Y)
+    for c in (n // 3, n - 200, 0):
+        cut = [slice(None)] * 4
+        cut[ax] = slice(max(0, c - 64), min(n, c + 200))
+        part = run(np.ascontiguousarray(a[tuple(cut)]), np.ascontiguousarray(b[tuple(cut)]))[3]
+        lo, hi = (0 if c == 0 else 64), (200 if c != n - 200 else 264)
+        want = [slice(None)] * 4
+        want[ax] = slice(c if c else 0, c + hi - lo if c else hi - 64)
+        got = [slice(None)] * 4
+        got[ax] = slice(lo, lo + want[ax].stop - want[ax].start)
+        if c != n - 200:  # the last 31 cells of an inner stretch see its end
+            want[ax] = slice(want[ax].start, want[ax].stop - 32)
+            got[ax] = slice(got[ax].start, got[ax].stop - 32)
+        assert np.array_equal(part.to_numpy()[tuple(got)], flow[tuple(want)]), (size, c)
+    tgt = r.standard_normal((T, Z, Y, X, 4)).astype(np.float32)
+    tg = s.create(M.Grid4Vec4)
+    tg.from_numpy(tgt)
+    loss = net.loss_grad(g0, g1, tg)
+    ref = ((flow.astype(np.float64) - tgt) ** 2).mean()
+    assert abs(loss - ref) <= 1e-6 * ref
+    assert np.isfinite(net.get_grads()).all()
