@@ -432,6 +432,12 @@ int flof_corr_vels_of4d(flof_grid4d *dst, flof_grid4d *vel,
                         float resetBndWidth, int maxIter);
 
 /* ---- full-resolution frames (optflow4d.cpp:1445-1595,1622-2105) -------- */
+/* The calls of this section enqueue on phi's context and return.  Work on an
+ * array of flof_dev_alloc of that context, and on its grids, may then still be
+ * under way: calls of the same context are ordered behind it, other streams
+ * (the null stream among them) have to wait with flof_sync().  With memory from
+ * elsewhere, or an array or deformation of another context, a call returns only
+ * when its work is done. */
 /* loadPlaceGrid4d with the frame files already decoded into device memory:
  * `frames_dev` holds (fileIdxEnd - fileIdxStart) frames of sx*sy*sz floats,
  * frame f at offset f*sx*sy*sz (file index fileIdxStart + f). */

@@ -6,6 +6,7 @@
 // (interpolation), source/plugin/optflow4d.cpp (advection 1275-1321,
 // resampling 40-57, calcLsDiff 895-927).
 
+#include <map>
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -17,6 +18,45 @@
 #include "flof_internal.h"
 
 namespace flof {
+
+// ---------------------------------------------------------------------------
+// The live arrays of flof_dev_alloc and the context each belongs to.  A call
+// that only enqueues may leave work on such an array of its own context under
+// way, because that context's calls are ordered behind it; on any other memory
+// it waits before it returns.
+namespace {
+struct OwnedArray {
+    const flof_ctx *ctx;
+    size_t bytes;
+};
+std::mutex g_arrays_lock;
+std::map<uintptr_t, OwnedArray> g_arrays;
+}  // namespace
+
+void own_array(const flof_ctx *ctx, const void *p, size_t bytes)
+{
+    std::lock_guard<std::mutex> l(g_arrays_lock);
+    g_arrays[(uintptr_t)p] = OwnedArray{ctx, bytes};
+}
+void disown_array(const void *p)
+{
+    std::lock_guard<std::mutex> l(g_arrays_lock);
+    g_arrays.erase((uintptr_t)p);
+}
+void disown_arrays_of(const flof_ctx *ctx)
+{
+    std::lock_guard<std::mutex> l(g_arrays_lock);
+    for (auto it = g_arrays.begin(); it != g_arrays.end();)
+        it = it->second.ctx == ctx ? g_arrays.erase(it) : std::next(it);
+}
+bool owns_array(const flof_ctx *ctx, const void *p)
+{
+    std::lock_guard<std::mutex> l(g_arrays_lock);
+    auto it = g_arrays.upper_bound((uintptr_t)p);
+    if (it == g_arrays.begin()) return false;
+    --it;
+    return it->second.ctx == ctx && (uintptr_t)p < it->first + it->second.bytes;
+}
 
 // ---------------------------------------------------------------------------
 // pool / errors / timing
@@ -1147,6 +1187,7 @@ int flof_ctx_create(flof_ctx **out, int device)
 int flof_ctx_destroy(flof_ctx *ctx)
 {
     if (!ctx) return FLOF_ERR_ARG;
+    disown_arrays_of(ctx);
     for (flof_ctx *w : ctx->workers) flof_ctx_destroy(w);
     ctx->workers.clear();
     (void)hipStreamSynchronize(ctx->stream);
@@ -1891,6 +1932,7 @@ int flof_dev_alloc(flof_ctx *ctx, size_t bytes, void **out)
     FLOF_REQUIRE(ctx && out, FLOF_ERR_ARG, "flof_dev_alloc: null argument");
     *out = nullptr;
     FLOF_HIP(hipMalloc(out, bytes));
+    own_array(ctx, *out, bytes);
     FLOF_HIP(hipMemsetAsync(*out, 0, bytes, ctx->stream));
     API_CATCH(ctx)
 }
@@ -1900,7 +1942,10 @@ int flof_dev_free(flof_ctx *ctx, void *p)
     API_TRY
     FLOF_REQUIRE(ctx, FLOF_ERR_ARG, "flof_dev_free: null context");
     FLOF_HIP(hipStreamSynchronize(ctx->stream));
-    if (p) FLOF_HIP(hipFree(p));
+    if (p) {
+        disown_array(p);
+        FLOF_HIP(hipFree(p));
+    }
     API_CATCH(ctx)
 }
 

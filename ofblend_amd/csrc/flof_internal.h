@@ -626,6 +626,11 @@ __device__ __forceinline__ float block_min(float v)
 void set_error(flof_ctx *ctx, const Error &e);
 void *reduce_scratch(flof_ctx *ctx, size_t bytes);
 void check_launch(const char *what);
+// arrays of flof_dev_alloc by context
+void own_array(const flof_ctx *ctx, const void *p, size_t bytes);
+void disown_array(const void *p);
+void disown_arrays_of(const flof_ctx *ctx);
+bool owns_array(const flof_ctx *ctx, const void *p);
 float host_max_norm_vec4(flof_ctx *ctx, const float4 *v, int64_t n);
 double host_ls_diff(flof_ctx *ctx, const float *a, const float *b, float *out,
                     const Dims4 &D, float corr, int bnd);

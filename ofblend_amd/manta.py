@@ -558,13 +558,6 @@ def placeGrid3d(src, dst, dstt):
           dst.ctx)
 
 
-def _settle(phi, arr):
-    """Waits for the work on phi's stream that uses an array of another
-    context, whose own calls would not wait for it."""
-    if arr.ctx.value != phi.ctx.value:
-        check(_lib.lib().flof_sync(phi.ctx), phi.ctx)
-
-
 def loadPlaceGrid4dFrames(frames, phi, offset, scale, fileIdxStart=-1,
                           fileIdxEnd=-1, debugSkipLoad=999999, spread=1.,
                           overrideSize=Vec4(-1.), overrideTimeOff=0.,
@@ -580,7 +573,6 @@ def loadPlaceGrid4dFrames(frames, phi, offset, scale, fileIdxStart=-1,
         fileIdxStart, fileIdxEnd, debugSkipLoad, spread, floats(*overrideSize),
         overrideTimeOff, overrideGoodRegion, loadTimeScale,
         int(rescaleSdfValues), sdfIsoOff, repeatStartFrame), phi.ctx)
-    _settle(phi, frames)
 
 
 def loadAdvectTimeSliceFromDefo(defo, dst, phi, time, blendAlpha,
@@ -604,7 +596,6 @@ def loadAdvectTimeSliceFromDefo(defo, dst, phi, time, blendAlpha,
             floats(*defoOffset), floats(*defoScale), floats(*defoFactor),
             floats(*overrideSize), overrideTimeOff, int(zeroVel), defoAniFac)
     check(rc, phi.ctx)
-    _settle(phi, dst)
 
 
 def repeatFrame4d(phi, srct, range=0., bnd=0):
@@ -705,7 +696,6 @@ def loadAdvectTimeSlice_OptRun(ID, fname, dst, phi, time, blendAlpha, loadTimeSc
         floats(*defoOffset), floats(*defoScale), floats(*defoFactor),
         floats(*overrideSize), overrideTimeOff, int(zeroVel), thirdAlpha, bordSkip,
         fourthAlpha, defoAniFac), phi.ctx)
-    _settle(phi, dst)
 
 
 def loadAdvectTimeSliceFromDefoVols(vols, dst, phi, time, blendAlpha, loadTimeScale=1.,
@@ -723,7 +713,6 @@ def loadAdvectTimeSliceFromDefoVols(vols, dst, phi, time, blendAlpha, loadTimeSc
         floats(*defoOffset), floats(*defoScale), floats(*defoFactor),
         floats(*overrideSize), overrideTimeOff, int(zeroVel), bordSkip, defoAniFac,
         int(doAligned), partialLoadFac, thirdAlpha, fourthAlpha), phi.ctx)
-    _settle(phi, dst)
 
 
 def loadAdvectTimeSlice(dummyID, fname, dst, phi, time, blendAlpha, loadTimeScale,

@@ -441,3 +441,74 @@ def test_advect_cfl_of_a_velocity_by_itself(steps):
     for _ in range(steps):
         ref = O.advect4d(ref, ref, dt=1.0, dtFac=dt)
     assert np.array_equal(g.to_numpy(), ref)
+
+
+@pytest.mark.parametrize("entry", ["slice_opt", "slice", "vols", "slices_opt", "place"])
+def test_frame_calls_end_with_the_work_on_memory_of_others(entry):
+    """The warps and the placement only enqueue, except on arrays that are not
+    phi's context's own: with an array of another context, a grid's memory or
+    a deformation of another context they return with phi's stream idle (work
+    of some 20 ms is queued before).  The results are those with own arrays."""
+    L = _lib.lib()
+    L.hipStreamQuery.argtypes = [C.c_void_p]
+    X, Y, Z, T = 48, 40, 44, 24
+    rng = np.random.default_rng(70)
+    s = M.Solver(gridSize=M.vec3(X, Y, Z), fourthDim=T)
+    phi, busy = s.create(M.Grid4Real), s.create(M.Grid4Real)
+    phi.from_numpy(rng.standard_normal((T, Z, Y, X)).astype(np.float32))
+    defo = s.create(M.Grid4Vec4)
+    defo.from_numpy(rng.standard_normal((T, Z, Y, X, 4)).astype(np.float32))
+    other = C.c_void_p()
+    assert L.flof_ctx_create(C.byref(other), 0) == 0
+    defo2 = C.c_void_p()
+    assert L.flof_grid4d_create(other, X, Y, Z, T, M.Grid4Vec4.ELEM, 0, C.byref(defo2)) == 0
+    a = defo.to_numpy()
+    assert L.flof_grid4d_upload(defo2, a.ctypes.data_as(C.c_void_p), a.nbytes) == 0
+    init = rng.standard_normal((2, Z, Y, X)).astype(np.float32)
+    mem = M.Grid4Real(s, (X, Y, Z, 2))
+    mem.from_numpy(init)
+    F = _lib.floats
+    z4, one = F(0, 0, 0, 0), F(1, 1, 1, 1)
+
+    def call(ptr, d):
+        if entry == "slice_opt":
+            return L.flof_advect_time_slice_opt(d, ptr, X, Y, Z, phi.h, 3.0, 0.5, 1.0, z4, one,
+                                                one, F(-1, -1, -1, -1), 0.0, 0, 1, 1.0)
+        if entry == "slice":
+            return L.flof_advect_time_slice(d, ptr, X, Y, Z, phi.h, 3.0, 0.5, 1.0, z4, one, one,
+                                            F(-1, -1, -1, -1), 0.0, 0, 1.0)
+        if entry == "vols":
+            v = (C.c_void_p * 2)(defo.h.value, getattr(d, "value", d))
+            return L.flof_advect_time_slice_vols(v, 2, ptr, X, Y, Z, phi.h, 3.0, 0.5, 1.0, z4,
+                                                 one, one, F(-1, -1, -1, -1), 0.0, 0, 1, 1.0, 0,
+                                                 0.5, 0.3, 0.2)
+        if entry == "slices_opt":
+            return L.flof_advect_time_slices_opt(d, ptr, X, Y, Z, 2, 2.0, 1.0, phi.h, 0.5, 1.0,
+                                                 z4, one, one, 1, 1.0)
+        return L.flof_load_place_grid4d(ptr, X, Y, Z, busy.h, z4, one, 0, 2, 999999, 1.0,
+                                        F(-1, -1, -1, -1), 0.0, 0, 1.0, 0, 0.0, 0.0)
+
+    def result(arr):
+        return busy.to_numpy() if entry == "place" else arr
+
+    own = M.DeviceArray.from_numpy(init)
+    assert call(own.ptr, defo.h) == 0
+    want = result(own.to_numpy())
+    foreign = M.DeviceArray.from_numpy(init, other)
+    cases = [("array of another context", foreign.ptr, defo.h),
+             ("memory of a grid", C.c_void_p(L.flof_grid4d_device_ptr(mem.h)), defo.h)]
+    if entry != "place":
+        cases.append(("deformation of another context", own.ptr, defo2))
+    for what, ptr, d in cases:
+        say("frame call", entry, what)
+        own.copyFrom(M.DeviceArray.from_numpy(init))
+        for _ in range(200):
+            M.advect4d(defo, busy)
+        assert call(ptr, d) == 0
+        assert L.hipStreamQuery(L.flof_ctx_stream(phi.ctx)) == 0
+        got = {foreign.ptr.value: foreign, own.ptr.value: own}.get(ptr.value)
+        got = got.to_numpy() if got is not None else mem.to_numpy()
+        assert np.array_equal(result(got), want)
+    del foreign
+    assert L.flof_grid4d_destroy(defo2) == 0
+    assert L.flof_ctx_destroy(other) == 0
