@@ -176,9 +176,9 @@ int flof_ctx_tuned_shape(const flof_ctx *ctx, int X, int Y, int Z, int T, int *t
  * caches, FLOF_STENCIL_AUTO (the default) runs all iterations of a level as
  * one launch where its vectors fit the registers and LDS of the chip (up to
  * about 1.3 million interior cells, FP32 direction storage, no timing of the
- * iteration's kernels), takes the LDS tiles for levels where they are faster (FP32 direction storage, t segments of 16 or more
- * steps, X filling 90% of the 64-wide tiles) and the t-marching kernels
- * elsewhere; FLOF_STENCIL_QARRAY is the first GPU form (three streaming
+ * iteration's kernels), takes the LDS tiles for levels where they are faster
+ * (FP32 direction storage, t segments of 16 or more steps, X filling 90% of the
+ * 64-wide tiles) and the t-marching kernels elsewhere; FLOF_STENCIL_QARRAY is the first GPU form (three streaming
  * kernels that store q = A p and g, 208 B per cell and iteration, FP32
  * direction storage only), kept for comparison. */
 enum flof_stencil {
@@ -188,6 +188,15 @@ enum flof_stencil {
     FLOF_STENCIL_QARRAY = 3
 };
 int flof_ctx_set_stencil(flof_ctx *ctx, int kind);
+/* The one-launch form of FLOF_STENCIL_AUTO (no reference counterpart; results
+ * are identical): its workgroups wait for each other up to `seconds` (2 by
+ * default, at most 60), after which the level is set up again and iterated by
+ * the other kernels; 0 makes every level of several workgroups take that way,
+ * negative values leave the form out. */
+int flof_ctx_set_resident_wait(flof_ctx *ctx, double seconds);
+/* Levels iterated in one launch by this context and its workers so far, and
+ * levels that were set up again because their launch was refused or gave up. */
+int flof_ctx_resident_counts(const flof_ctx *ctx, int64_t *resident, int64_t *redone);
 
 /* ---- level-set mesh of a 3D frame and its .bobj.gz file ---------------- */
 typedef struct flof_mesh flof_mesh;

@@ -49,6 +49,8 @@ SIGNATURES = {
     "flof_ctx_tuned_blocks": ([_P, _I, _I, _I, _I], _I),
     "flof_ctx_tuned_shape": ([_P, _I, _I, _I, _I, _IP, _IP, _IP], _I),
     "flof_ctx_set_stencil": ([_P, _I], _I),
+    "flof_ctx_set_resident_wait": ([_P, C.c_double], _I),
+    "flof_ctx_resident_counts": ([_P, _I64P, _I64P], _I),
     "flof_stream_bandwidth": ([_P, _I, C.c_int64, _I, _DP], _I),
     "flof_check_reciprocal": ([_P, C.c_uint32, C.c_uint32, C.POINTER(_U64)], _I),
     "flof_create_mesh": ([_P, _P, _I, _I, _I, C.POINTER(_P)], _I),

@@ -1225,6 +1225,27 @@ int flof_ctx_set_stencil(flof_ctx *ctx, int kind)
     return FLOF_OK;
 }
 
+int flof_ctx_set_resident_wait(flof_ctx *ctx, double seconds)
+{
+    if (!ctx || seconds != seconds) return FLOF_ERR_ARG;
+    ctx->resident_wait = seconds;
+    for (flof_ctx *w : ctx->workers) flof_ctx_set_resident_wait(w, seconds);
+    return FLOF_OK;
+}
+
+int flof_ctx_resident_counts(const flof_ctx *ctx, int64_t *resident, int64_t *redone)
+{
+    if (!ctx) return FLOF_ERR_ARG;
+    int64_t a = ctx->resident_levels, b = ctx->resident_redone;
+    for (const flof_ctx *w : ctx->workers) {
+        a += w->resident_levels;
+        b += w->resident_redone;
+    }
+    if (resident) *resident = a;
+    if (redone) *redone = b;
+    return FLOF_OK;
+}
+
 int flof_ctx_tuned_blocks(const flof_ctx *ctx, int X, int Y, int Z, int T)
 {
     if (!ctx) return FLOF_ERR_ARG;

@@ -113,6 +113,12 @@ struct flof_ctx {
     // images of the call in progress stored as bfloat16 with binary16
     // gradients (the mixed-precision solve, flof_of_params.precision)
     bool img_bf16 = false;
+    // the resident PCG (flof_resident.hip): seconds a workgroup waits for
+    // another one before the level takes the launched form (negative: always
+    // the launched form), and the levels so far that ran resident / were set
+    // up again for the launched form
+    double resident_wait = 2.;
+    int64_t resident_levels = 0, resident_redone = 0;
 };
 
 // the kernel variant part of the autotuner's key of a grid shape

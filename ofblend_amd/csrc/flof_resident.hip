@@ -37,9 +37,10 @@
 // was given scratch memory all the same is not launched.
 //
 // The launch is cooperative, so all workgroups are resident together.  A
-// workgroup that still waits after two seconds gives up and says so in a word
-// that all poll, so every wavefront ends whatever happens; the caller then
-// sets the level up again and uses the other form.
+// workgroup that still waits after two seconds (flof_ctx_set_resident_wait)
+// gives up and says so in a word that all poll, so every wavefront ends
+// whatever happens; the caller then sets the level up again and uses the other
+// form.
 
 #include <algorithm>
 #include <cstring>
@@ -174,7 +175,8 @@ __host__ __device__ inline int part_at(int n, int parts, int i)
 // XG: x stays in memory (the thread's own cells) instead of registers
 template <int CPT, bool XG>
 __global__ void __launch_bounds__(RT)
-k_cg_resident(const ResItem *__restrict__ items, int nitems, unsigned *abort_word)
+k_cg_resident(const ResItem *__restrict__ items, int nitems, unsigned *abort_word,
+              unsigned long long wait_ticks)
 {
     __shared__ float4 lp[R_CELLS];
     __shared__ short4 nbr[R_ROWS];   // LDS distance to the rows y-1, y+1, z-1, z+1
@@ -341,8 +343,8 @@ k_cg_resident(const ResItem *__restrict__ items, int nitems, unsigned *abort_wor
         if (nwg > 1 && wave < 4 && wave * 64 < nwg) {
             DD s{0., 0.};
             float m = -INFINITY;
-            bool fail = false;
-            if (tid < nwg) {
+            bool fail = wait_ticks == 0;
+            if (tid < nwg && !fail) {
                 int p = slot0 + tid * R_SLOT;
                 fresh(p);
                 const unsigned tag = epoch & 0xff;
@@ -364,10 +366,10 @@ k_cg_resident(const ResItem *__restrict__ items, int nitems, unsigned *abort_wor
                         break;
                     }
                     if ((++spins & 63) == 0) {
-                        // two seconds of the 100 MHz clock, or another one gave up
+                        // waited long enough, or another one gave up
                         if (__hip_atomic_load(abort_word, __ATOMIC_RELAXED,
                                               __HIP_MEMORY_SCOPE_AGENT) != 0 ||
-                            wall_clock64() - begin > 200000000ull) {
+                            wall_clock64() - begin > wait_ticks) {
                             fail = true;
                             break;
                         }
@@ -703,7 +705,9 @@ bool resident_iterate(flof_ctx *ctx, const std::vector<ResLevel> &levels,
     FLOF_HIP(hipStreamSynchronize(ctx->stream));  // h lives on the stack
     const ResItem *dt = tab.as<ResItem>();
     int ni = n;
-    void *args[] = {(void *)&dt, (void *)&ni, (void *)&abort_word};
+    // of the 100 MHz clock
+    unsigned long long ticks = (unsigned long long)(std::min(ctx->resident_wait, 60.) * 1e8);
+    void *args[] = {(void *)&dt, (void *)&ni, (void *)&abort_word, (void *)&ticks};
     const int cpt = (most + RT - 1) / RT;
     const void *k = cpt <= 1   ? (const void *)k_cg_resident<1, false>
                     : cpt <= 2 ? (const void *)k_cg_resident<2, false>

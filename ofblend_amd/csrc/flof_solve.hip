@@ -2748,7 +2748,7 @@ static ResPlan resident_level_plan(const flof_ctx *ctx, const LevelCg &L, int bu
     for (int k : {FLOF_KT_CG_APPLY, FLOF_KT_CG_UPDATE, FLOF_KT_CG_DIR})
         if (ctx->timers[k].on) return ResPlan{};
     if (!ctx->use_tmarch || ctx->stencil != FLOF_STENCIL_AUTO || L.pstore != FLOF_PSTORE_F32 ||
-        L.hs.done)
+        L.hs.done || ctx->resident_wait < 0.)
         return ResPlan{};
     return resident_plan(L.D, budget, fewest);
 }
@@ -2764,7 +2764,11 @@ static bool resident_levels(flof_ctx *ctx, const std::vector<LevelCg *> &Ls,
                               W.prec.as<float4>(), W.x.as<float4>(), W.r.as<float4>(),
                               W.p.as<float4>(), W.q.as<float4>(), L->st()});
     }
-    if (!resident_iterate(ctx, lv, plans)) return false;
+    if (!resident_iterate(ctx, lv, plans)) {
+        ctx->resident_redone += (int64_t)Ls.size();
+        return false;
+    }
+    ctx->resident_levels += (int64_t)Ls.size();
     for (LevelCg *L : Ls)
         FLOF_HIP(hipMemcpyAsync(&L->hs, L->st(), sizeof(CgState), hipMemcpyDeviceToHost,
                                 ctx->stream));
@@ -3507,6 +3511,7 @@ static flof_ctx *worker_ctx(flof_ctx *ctx, int w)
         c->lds_blocks_per_cu = ctx->lds_blocks_per_cu;
         c->lds_xcd = ctx->lds_xcd;
         c->autotune = ctx->autotune;
+        c->resident_wait = ctx->resident_wait;
         ctx->workers.push_back(c);
     }
     return ctx->workers[w];

@@ -594,10 +594,20 @@ def test_non_finite_image_gives_the_references_zero_flow(where, bad):
     assert lv["iters"] == [it] == [0]
 
 
+def resident_counts():
+    """Levels iterated in one launch so far, and levels set up again."""
+    import ctypes as C
+    from ofblend_amd import _lib
+    a, b = C.c_int64(), C.c_int64()
+    assert _lib.lib().flof_ctx_resident_counts(M.context(), C.byref(a), C.byref(b)) == 0
+    return a.value, b.value
+
+
 @pytest.mark.parametrize("shape,smooth", [
     ((3, 3, 3, 4), 0.1), ((5, 4, 3, 9), 0.1), ((16, 30, 4, 36), 0.1), ((100, 8, 8, 12), 0.1),
     ((9, 23, 4, 6), 0.0), ((24, 23, 25, 22), 0.1), ((30, 27, 26, 29), 0.1),
-    ((29, 28, 29, 29), 0.1), ((32, 31, 30, 33), 0.1), ((31, 33, 30, 47), 0.1)])
+    ((29, 28, 29, 29), 0.1), ((32, 31, 30, 33), 0.1), ((31, 33, 30, 47), 0.1),
+    ((32, 32, 32, 48), 0.1)])
 def test_resident_pcg_matches_launched_pcg(shape, smooth):
     """The resident PCG (one launch per level) on levels of one workgroup, of
     one-row and one-plane boxes, of boxes with 1 to 11 cells per thread and
@@ -605,7 +615,8 @@ def test_resident_pcg_matches_launched_pcg(shape, smooth):
     incoming flow, to convergence and to caps after an odd and an even
     iteration: the flow, the iterations and the residuals are those of the
     t-marching launches bit for bit (which the oracle pins above); the small
-    ones are compared with the oracle directly."""
+    ones are compared with the oracle directly.  Every AUTO solve here ran
+    resident, and none was set up again."""
     from ofblend_amd import _lib
     from ofblend_amd.abi import FLOF_STENCIL_AUTO, FLOF_STENCIL_TMARCH
     X, Y, Z, T = shape
@@ -614,6 +625,7 @@ def test_resident_pcg_matches_launched_pcg(shape, smooth):
     s = solver(X, Y, Z, T)
     ga, gb = real(s, a), real(s, b)
     L, ctx = _lib.lib(), M.context()
+    before = resident_counts()
     for cap in (1, 2, 150):
         res = []
         for code in (FLOF_STENCIL_AUTO, FLOF_STENCIL_TMARCH):
@@ -626,6 +638,9 @@ def test_resident_pcg_matches_launched_pcg(shape, smooth):
             finally:
                 L.flof_ctx_set_stencil(ctx, FLOF_STENCIL_AUTO)
             res.append((vel.to_numpy(), M.getLastSolveInfo().summary()["levels"][0]))
+            now = resident_counts()
+            assert now == (before[0] + (code == FLOF_STENCIL_AUTO), before[1])
+            before = now
         assert res[0][1] == res[1][1]
         assert np.array_equal(res[0][0], res[1][0])
     if X * Y * Z * T < 40000:
@@ -634,3 +649,57 @@ def test_resident_pcg_matches_launched_pcg(shape, smooth):
             ref, it, _, st = O.optical_flow4d(vin, a, b, p)
         assert res[0][1]["iters"] == [it] and res[0][1]["status"] == [st]
         assert np.array_equal(res[0][0], ref)
+
+
+def test_resident_pcg_that_gives_up_is_set_up_again():
+    """With no time to wait, a resident launch of several workgroups gives up
+    at its first exchange: the levels are set up again and iterated by the
+    other kernels.  Single levels, warm-started levels and a fused batch (one
+    level of it on one workgroup, which has nobody to wait for) then give the
+    flows and records that they give without the resident form."""
+    from ofblend_amd import _lib
+    L, ctx = _lib.lib(), M.context()
+    prm = dict(wSmooth=0.1, wEnergy=1e-4, cgAccuracy=1e-5, minGridSize=8, multiStep=1,
+               postVelBlur=0.0, doFinalProject=False, resetBndWidth=-1.0, cfl=999.0)
+    shapes = [(20, 18, 16, 14), (24, 24, 20, 22), (8, 7, 6, 8)]
+    sol = [solver(*sh) for sh in shapes]
+    imgs = [(real(s, O.drop_sdf(*sh, seed=90 + k)), real(s, O.drop_sdf(*sh, seed=95 + k)))
+            for k, (s, sh) in enumerate(zip(sol, shapes))]
+    X, Y, Z, T = shapes[0]
+    guess = vec4(sol[0], (np.random.default_rng(96).standard_normal((T, Z, Y, X, 4)) * 0.3)
+                 .astype(np.float32))
+
+    def run():
+        out = []
+        vel = sol[0].create(M.Grid4Vec4)
+        M.opticalFlow4d(vel, *imgs[0], wSmooth=0.1, wEnergy=1e-4, cgAccuracy=1e-5)
+        out.append((vel.to_numpy(), M.getLastSolveInfo().summary()))
+        vel = sol[0].create(M.Grid4Vec4)
+        e = M.opticalFlowMultiscale4d(vel=vel, i0=imgs[0][0], i1=imgs[0][1], warm=guess, **prm)
+        out.append((vel.to_numpy(), e, M.getLastSolveInfo().summary()))
+        vels = [s.create(M.Grid4Vec4) for s in sol]
+        errs, infos = M.opticalFlowMultiscale4dFused(vels, [i[0] for i in imgs],
+                                                     [i[1] for i in imgs], **prm)
+        out += [(v.to_numpy(), e, i.summary()) for v, e, i in zip(vels, errs, infos)]
+        return out
+
+    res, total = {}, 0
+    try:
+        for wait in (2.0, 0.0, -1.0):
+            say("resident wait", wait)
+            assert L.flof_ctx_set_resident_wait(ctx, wait) == 0
+            a = resident_counts()
+            res[wait] = run()
+            b = resident_counts()
+            ran, redone = b[0] - a[0], b[1] - a[1]
+            say("levels resident", ran, "set up again", redone)
+            # (a level that one workgroup iterates alone runs in any case)
+            total = ran if wait > 0 else total
+            assert total > 0 and (redone > 0) == (wait == 0)
+            assert ran + redone == (total if wait >= 0 else 0)
+    finally:
+        assert L.flof_ctx_set_resident_wait(ctx, 2.0) == 0
+    for wait in (0.0, -1.0):
+        for g, w in zip(res[wait], res[2.0]):
+            assert np.array_equal(g[0], w[0]) and g[1:] == w[1:]
+    assert L.flof_ctx_set_resident_wait(ctx, float("nan")) != 0
