@@ -191,8 +191,9 @@ int flof_ctx_set_stencil(flof_ctx *ctx, int kind);
 /* The one-launch form of FLOF_STENCIL_AUTO (no reference counterpart; results
  * are identical): its workgroups wait for each other up to `seconds` (2 by
  * default, at most 60), after which the level is set up again and iterated by
- * the other kernels; 0 makes every level of several workgroups take that way,
- * negative values leave the form out. */
+ * the other kernels, as are the context's next levels for a minute; 0 makes a
+ * level of several workgroups take that way, negative values leave the form
+ * out.  Setting the wait ends such a minute. */
 int flof_ctx_set_resident_wait(flof_ctx *ctx, double seconds);
 /* Levels iterated in one launch by this context and its workers so far, and
  * levels that were set up again because their launch was refused or gave up. */

@@ -1229,6 +1229,7 @@ int flof_ctx_set_resident_wait(flof_ctx *ctx, double seconds)
 {
     if (!ctx || seconds != seconds) return FLOF_ERR_ARG;
     ctx->resident_wait = seconds;
+    ctx->resident_after = {};
     for (flof_ctx *w : ctx->workers) flof_ctx_set_resident_wait(w, seconds);
     return FLOF_OK;
 }

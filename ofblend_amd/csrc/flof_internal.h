@@ -7,6 +7,7 @@
 // correctly rounded sums (double-double accumulation, see dd_* below).
 #pragma once
 
+#include <chrono>
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -119,6 +120,9 @@ struct flof_ctx {
     // up again for the launched form
     double resident_wait = 2.;
     int64_t resident_levels = 0, resident_redone = 0;
+    // after a launch that was refused or gave up (a chip shared with others):
+    // the launched form until then
+    std::chrono::steady_clock::time_point resident_after{};
 };
 
 // the kernel variant part of the autotuner's key of a grid shape

@@ -2742,13 +2742,21 @@ static void level_iterate(flof_ctx *ctx, LevelCg &L, int maxIter)
 // level_iterate against the resident form: 8^4 14.8 and 5.5 us, 16^4 16.8 and
 // 7.9, 24^4 29.4 and 13.5, 32^4 50.7 and 18.8, 32^3 x 48 65.4 and 26.3: it is
 // the better one wherever it fits, up to 256 boxes of 11 cells per thread.
+// A launch that gave up has cost the wait and a second set-up, and the next
+// would too while others hold CUs of the chip: the context then stays with the
+// launches for 30 times the default wait, which bounds the loss to 3%.
+constexpr std::chrono::seconds RESIDENT_PAUSE(60);
+static bool resident_allowed(const flof_ctx *ctx)
+{
+    return ctx->resident_wait >= 0. && std::chrono::steady_clock::now() >= ctx->resident_after;
+}
 static ResPlan resident_level_plan(const flof_ctx *ctx, const LevelCg &L, int budget,
                                    bool fewest = false)
 {
     for (int k : {FLOF_KT_CG_APPLY, FLOF_KT_CG_UPDATE, FLOF_KT_CG_DIR})
         if (ctx->timers[k].on) return ResPlan{};
     if (!ctx->use_tmarch || ctx->stencil != FLOF_STENCIL_AUTO || L.pstore != FLOF_PSTORE_F32 ||
-        L.hs.done || ctx->resident_wait < 0.)
+        L.hs.done || !resident_allowed(ctx))
         return ResPlan{};
     return resident_plan(L.D, budget, fewest);
 }
@@ -2766,6 +2774,7 @@ static bool resident_levels(flof_ctx *ctx, const std::vector<LevelCg *> &Ls,
     }
     if (!resident_iterate(ctx, lv, plans)) {
         ctx->resident_redone += (int64_t)Ls.size();
+        ctx->resident_after = std::chrono::steady_clock::now() + RESIDENT_PAUSE;
         return false;
     }
     ctx->resident_levels += (int64_t)Ls.size();
@@ -3383,6 +3392,10 @@ static void multiscale_fused(flof_ctx *ctx, int np, float4 *const *vel_top,
         std::stable_sort(res.begin(), res.end(),
                          [&](size_t a, size_t b) { return Ls[a]->n > Ls[b]->n; });
         for (size_t at = 0; at < res.size();) {
+            if (!resident_allowed(ctx)) {  // a group gave up: the others are set up
+                for (; at < res.size(); ++at) need[res[at]] = 0;
+                break;
+            }
             int sum = 0;
             size_t end = at;
             while (end < res.size() && sum + need[res[end]] <= ctx->num_cu)
