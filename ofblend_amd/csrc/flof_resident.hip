@@ -36,7 +36,11 @@
 // without conditions and the vectors declared inside the loop; a kernel that
 // was given scratch memory all the same is not launched.
 //
-// The launch is cooperative, so all workgroups are resident together.  A
+// The launch is cooperative, so all workgroups are resident together, and the
+// runtime runs such launches of several streams one after another: worker
+// streams gain by it too (16 solves of 16^4 on one, 2, 4 and 16 streams 51, 43,
+// 43, 44 ms and launched 123, 66, 48, 162; of 24^4 128, 118, 117, 118 and 308,
+// 178, 144, 322).  A
 // workgroup that still waits after two seconds (flof_ctx_set_resident_wait)
 // gives up and says so in a word that all poll, so every wavefront ends
 // whatever happens; the caller then sets the level up again and uses the other

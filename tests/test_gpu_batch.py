@@ -42,13 +42,16 @@ def test_batch_equals_single_solves():
         assert infos[n].summary()["levels"] == inf["levels"]
 
 
+@pytest.mark.parametrize("resident_wait", [2.0, -1.0])
 @pytest.mark.parametrize("shape", [(24, 24, 24, 20), (70, 16, 16, 24)])
-def test_autotune_keeps_results(shape):
+def test_autotune_keeps_results(shape, resident_wait):
     """The launch-shape autotuner changes timing only: a solve with it on is
     identical to one with it off, and it records a valid choice for the
     finest level's shape (t-marching workgroups per CU; LDS-tiled or
     t-marching stencil kernels and the tiles' t-segment length).  The
-    second shape has a ragged second 64-wide x tile."""
+    second shape has a ragged second 64-wide x tile.  Levels of these sizes
+    iterate in one launch, which has no shape to tune: with that form left out
+    (wait -1) the tuned launches run."""
     import ctypes as C
     from ofblend_amd import _lib
     X, Y, Z, T = shape
@@ -62,6 +65,7 @@ def test_autotune_keeps_results(shape):
     L = _lib.lib()
     ctx = M.context()
     L.flof_ctx_set_autotune(ctx, 1)
+    L.flof_ctx_set_resident_wait(ctx, resident_wait)
     try:
         v.clear()
         M.opticalFlowMultiscale4d(vel=v, i0=g0, i1=g1, **P)
@@ -80,6 +84,41 @@ def test_autotune_keeps_results(shape):
         assert np.array_equal(v.to_numpy(), ref)
     finally:
         L.flof_ctx_set_autotune(ctx, 0)
+        L.flof_ctx_set_resident_wait(ctx, 2.0)
+
+
+def test_batch_of_levels_that_fill_the_chip():
+    """Worker streams whose levels each want every CU for one launch (the
+    runtime runs such launches one after another): the single solves' results,
+    every level in one launch, none set up again."""
+    import ctypes as C
+    from ofblend_amd import _lib
+    L, ctx = _lib.lib(), M.context()
+    jobs = _jobs([(32, 30, 28, 26), (26, 32, 28, 30), (28, 28, 32, 28), (30, 26, 28, 32)], 20)
+    prm = dict(P, cgMaxIter=200)
+
+    def counts():
+        a, b = C.c_int64(), C.c_int64()
+        assert L.flof_ctx_resident_counts(ctx, C.byref(a), C.byref(b)) == 0
+        return a.value, b.value
+
+    ref = []
+    for s, g0, g1, v, a, b in jobs:
+        v.clear()
+        e = M.opticalFlowMultiscale4d(vel=v, i0=g0, i1=g1, **prm)
+        ref.append((e, v.to_numpy(), M.getLastSolveInfo().summary()))
+    for j in jobs:
+        j[3].clear()
+    before = counts()
+    print("batch of chip-filling levels", flush=True)
+    errs, infos = M.opticalFlowMultiscale4dBatch([j[3] for j in jobs], [j[1] for j in jobs],
+                                                 [j[2] for j in jobs], concurrency=4, **prm)
+    now = counts()
+    for n, j in enumerate(jobs):
+        assert errs[n] == ref[n][0] and np.array_equal(j[3].to_numpy(), ref[n][1])
+        assert infos[n].summary()["levels"] == ref[n][2]["levels"]
+    assert now[0] - before[0] == sum(len(r[2]["levels"]) for r in ref)
+    assert now[1] == before[1]
 
 
 def _jobs(shapes, seed0, nspheres=1):
@@ -98,7 +137,7 @@ def _jobs(shapes, seed0, nspheres=1):
 
 
 @pytest.mark.parametrize("precision", [0, 2])
-def test_fused_batch_matches_oracle(precision):
+def test_fused_batch_matches_oracle(precision, pcg_form):
     """The fused batch (shared PCG launches per level) on uneven small
     problems with different pyramid depths (3, 2 and 1 levels): each flow,
     iteration record and error is the oracle's (correctly rounded sums), bit

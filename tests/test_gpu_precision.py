@@ -68,9 +68,11 @@ def test_bf16_direction_multiscale_bit_exact_and_error():
 
 # ---------------------------------------------------------------------------
 # the mixed-precision solve: bfloat16 images, binary16 gradients of i1, FP32
-# stencil arithmetic, FP64 CG scalars (precision FLOF_PREC_IMG_BF16)
+# stencil arithmetic, FP64 CG scalars (precision FLOF_PREC_IMG_BF16).  Grids of
+# these sizes iterate in one launch, larger ones by the t-marching kernels: each
+# case runs both ways.
 
-def test_mixed_images_level_solve_bit_exact():
+def test_mixed_images_level_solve_bit_exact(pcg_form):
     from ofblend_amd.abi import FLOF_PREC_IMG_BF16
     N, T = 14, 12
     i0 = O.drop_sdf(N, N, N, T, seed=7, nspheres=2, rmin=0.08, rmax=0.18)
@@ -93,7 +95,7 @@ def test_mixed_images_level_solve_bit_exact():
 
 
 @pytest.mark.parametrize("multiStep,blur", [(1, 0.0), (3, 2.0)])
-def test_mixed_images_multiscale_bit_exact_and_error(multiStep, blur):
+def test_mixed_images_multiscale_bit_exact_and_error(multiStep, blur, pcg_form):
     """24^3 x 20, the mixed-precision generator (2 spheres, radii 0.08N-0.18N): the
     mixed-precision solve equals the oracle that rounds at the same points
     (images stored as bfloat16 at the start, at each pyramid level and after
@@ -127,7 +129,7 @@ def test_mixed_images_multiscale_bit_exact_and_error(multiStep, blur):
         np.sqrt((d32 ** 2).mean()), np.abs(f64).max()))
 
 
-def test_mixed_images_golden_digest():
+def test_mixed_images_golden_digest(pcg_form):
     """The mixed-precision solve of the 32^3 x 32 two-sphere pair (seeds 7,
     8) is bit-identical to the oracle's (digest recorded by
     tests/golden/make_digests.py, with both solves' distances to FP64)."""
