@@ -599,9 +599,13 @@ void launch_neumann_bf16(flof_ctx *ctx, void *g, const Dims4 &D, int w)
 // values, bound it by latency: a thread takes KZ cells of one column, whose
 // velocities and then samples are under way together; scalars are gathered in
 // pairs of x neighbours, and every XCD works through a contiguous run of the
-// grid so that its L2 holds the rows that the samples share.  KZ = 1, 2, 4 (and
-// one cell per thread and iteration, before): 64^4 218, 203, 196 us (270), 32^3
-// x 48 12.0, 12.0, 13.4 (14.9), batches of 14 to 28^4 5.8, 6.0, 7.4 (6.4): 2.
+// inner time slices so that its L2 holds the rows that the samples share (the
+// two outer slices, which only become 0, are dealt out on their own: among the
+// others they would leave XCDs without work, at 64^3 x 4 half of them).
+// KZ = 1, 2, 4 for scalars (and one cell per thread and iteration, before): 64^4
+// 218, 203, 196 us (270), 32^3 x 48 12.0, 12.0, 13.4 (14.9), batches of 14 to
+// 28^4 5.8, 6.0, 7.4 (6.4): 2.  Vec4 samples hold 64 registers of corners: 1,
+// and there the outer cells return at once (64^4 of rough flow 1055 -> 921 us, 64^3 x 4 57 -> 35).
 // What is left is the address unit, a line per lane and gather where the flow
 // is rough.
 template <class T, class S> struct Sample4 {
@@ -622,17 +626,33 @@ template <class S> struct Sample4<float, S> {
 template <class T, class S, int KZ>
 __global__ void __launch_bounds__(256)
 k_advect(S *__restrict__ dst, const S *__restrict__ src, const float4 *__restrict__ vel,
-         float4 vscale, int use_vscale, Dims4 D, Coord4 C, uint32_t threads, float dt)
+         float4 vscale, int use_vscale, Dims4 D, Coord4 C, uint32_t inner, uint32_t inner_blocks,
+         uint32_t outer, float dt)
 {
-    // gridDim.x is a multiple of the XCDs
-    const uint32_t b = (blockIdx.x % FLOF_NXCD) * (gridDim.x / FLOF_NXCD) + blockIdx.x / FLOF_NXCD;
-    const uint32_t u = b * 256u + threadIdx.x;
-    if (u >= threads) return;
     int i, j, kg, t;
-    decompose(u, C, i, j, kg, t);  // C: z in groups of KZ
+    if (blockIdx.x >= inner_blocks) {  // the outer time slices
+        const uint32_t u = (blockIdx.x - inner_blocks) * 256u + threadIdx.x;
+        if (u >= outer) return;
+        decompose(u, C, i, j, kg, t);  // C: z in groups of KZ
+        const int64_t c = (int64_t)i + (int64_t)D.X * j + D.sz * kg * KZ + D.st * (t ? D.T - 1 : 0);
+#pragma unroll
+        for (int q = 0; q < KZ; ++q)
+            if (kg * KZ + q < D.Z) dst[c + D.sz * q] = Stor<T, S>::st(VOps<T>::zero());
+        return;
+    }
+    // inner_blocks is a multiple of the XCDs
+    const uint32_t b = (blockIdx.x % FLOF_NXCD) * (inner_blocks / FLOF_NXCD) + blockIdx.x / FLOF_NXCD;
+    const uint32_t u = b * 256u + threadIdx.x;
+    if (u >= inner) return;
+    decompose(u, C, i, j, kg, t);
+    t += 1;
     const int k0 = kg * KZ;
     const int64_t c0 = (int64_t)i + (int64_t)D.X * j + D.sz * k0 + D.st * t;
-    const bool col = i >= 1 && j >= 1 && t >= 1 && i < D.X - 1 && j < D.Y - 1 && t < D.T - 1;
+    const bool col = i >= 1 && j >= 1 && i < D.X - 1 && j < D.Y - 1;
+    if (KZ == 1 && !(col && k0 >= 1 && k0 < D.Z - 1)) {
+        dst[c0] = Stor<T, S>::st(VOps<T>::zero());
+        return;
+    }
     // no cell waits behind a branch: the outer layer and the planes behind the
     // last one are sampled too (any position clamps into the grid) and dropped
     float4 v[KZ];
@@ -663,12 +683,14 @@ static void advect_kz(flof_ctx *ctx, S *dst, const S *src, const float4 *vel, fl
                       int use_vscale, const Dims4 &D, float dt)
 {
     const int zg = (D.Z + KZ - 1) / KZ;
-    const uint32_t threads = (uint32_t)((int64_t)D.X * D.Y * zg * D.T);
-    uint32_t blocks = (threads + 255u) / 256u;
+    const uint32_t slice = (uint32_t)((int64_t)D.X * D.Y * zg);
+    const uint32_t inner = slice * (uint32_t)std::max(0, D.T - 2);
+    const uint32_t outer = slice * (uint32_t)std::min(2, D.T);
+    uint32_t blocks = (inner + 255u) / 256u;
     blocks = (blocks + FLOF_NXCD - 1) / FLOF_NXCD * FLOF_NXCD;
     const Coord4 C{make_fastdiv(D.X), make_fastdiv(D.Y), make_fastdiv((uint32_t)zg)};
-    klaunch(ctx, FLOF_KT_ADVECT, k_advect<T, S, KZ>, dim3(blocks), dim3(256), dst, src, vel,
-            vscale, use_vscale, D, C, threads, dt);
+    klaunch(ctx, FLOF_KT_ADVECT, k_advect<T, S, KZ>, dim3(blocks + (outer + 255u) / 256u),
+            dim3(256), dst, src, vel, vscale, use_vscale, D, C, inner, blocks, outer, dt);
 }
 
 void launch_advect(flof_ctx *ctx, const float4 *vel, float vel_scale, void *grid,

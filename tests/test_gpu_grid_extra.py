@@ -512,3 +512,24 @@ def test_frame_calls_end_with_the_work_on_memory_of_others(entry):
     del foreign
     assert L.flof_grid4d_destroy(defo2) == 0
     assert L.flof_ctx_destroy(other) == 0
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 2, 2), (3, 2, 5, 3), (2, 6, 7, 9), (3, 3, 3, 70),
+                                   (4, 5, 4, 66), (9, 4, 3, 5), (70, 3, 4, 3)])
+def test_advect_edges(shape):
+    """advect4d where the outer time slices are all or most of the grid, with
+    odd and even plane counts and rows over one wavefront, scalar and Vec4,
+    against the oracle."""
+    T, Z, Y, X = shape
+    say("advect", shape)
+    rng = np.random.default_rng(80)
+    v = (rng.standard_normal((T, Z, Y, X, 4)) * 1.5).astype(np.float32)
+    s = M.Solver(gridSize=M.vec3(X, Y, Z), fourthDim=T)
+    vel = s.create(M.Grid4Vec4)
+    vel.from_numpy(v)
+    for kind, tail in ((M.Grid4Real, ()), (M.Grid4Vec4, (4,))):
+        a = rng.standard_normal((T, Z, Y, X) + tail).astype(np.float32)
+        g = s.create(kind)
+        g.from_numpy(a)
+        M.advect4d(vel, g, dtFac=0.7)
+        assert np.array_equal(g.to_numpy(), O.advect4d(v, a, dt=1.0, dtFac=0.7))
