@@ -48,7 +48,8 @@ __global__ void k_repeat_frame(float *__restrict__ phi, Dims4 D, float srct, int
 // cells on it.  The distances are made by one pass per axis (a byte per cell
 // wherever 254 is out of reach), which leaves a pass per layer for the values
 // only, layer d from layer d - 1: 1 instead of 4 bytes per cell to look at.
-// 40^3 x 60, 40 layers: 7.6 -> 3.8 us per layer, 310 -> 180 us in all.
+// 40^3 x 60, 40 layers: 7.6 -> 3.8 us per layer, 310 -> 180 us in all.  Few
+// layers, few cells or long lines grow layer by layer (extrap_grow).
 //
 // Distances above any layer, and the outer cells': never a layer's number.
 template <class U> constexpr U EX_FAR = (U)~(U)0;
@@ -194,6 +195,89 @@ k_extrap_layer(float *__restrict__ phi, const U *__restrict__ dist, Dims4 D, int
         }
         __syncthreads();
     }
+}
+
+// The same layers grown one after another: a byte per cell (wherever 253 is out
+// of reach) holds its layer, "free" (interior, not reached yet) or "outer", and a
+// pass turns the free cells next to layer d - 1 into layer d.  Two dependent
+// accesses per pass: a cell's own byte, then its neighbours' bytes and values
+// together.  (Neighbours may become layer d meanwhile: neither their old nor
+// their new byte is d - 1.)
+template <class U> constexpr U EG_FREE = (U)~(U)0;
+template <class U> constexpr U EG_OUTER = EG_FREE<U> - 1;
+
+template <class U>
+__global__ void __launch_bounds__(256)
+k_extrap_grow_mark(const float *__restrict__ phi, U *__restrict__ layer, Dims4 D, Coord4 C,
+                   int inside)
+{
+    const int64_t n = D.st * D.T;
+    for (int64_t c = blockIdx.x * (int64_t)256 + threadIdx.x; c < n;
+         c += (int64_t)gridDim.x * 256) {
+        int i, j, k, t;
+        decompose((uint32_t)c, C, i, j, k, t);
+        U u = EG_OUTER<U>;
+        if (i >= 1 && j >= 1 && k >= 1 && t >= 1 && i < D.X - 1 && j < D.Y - 1 && k < D.Z - 1 &&
+            t < D.T - 1) {
+            const float v = phi[c];
+            u = (!inside ? v < 0.f : v > 0.f) ? (U)0 : EG_FREE<U>;
+        }
+        layer[c] = u;
+    }
+}
+
+// cells [c0, c1) hold the interior; last: free cells that stay free take `set`
+template <class U>
+__global__ void __launch_bounds__(256)
+k_extrap_grow(float *__restrict__ phi, U *layer, Dims4 D, int64_t c0, int64_t c1, uint32_t d,
+              float direction, int last, float set)
+{
+    const int64_t off[8] = {-1, 1, -(int64_t)D.X, (int64_t)D.X, -D.sz, D.sz, -D.st, D.st};
+    for (int64_t c = c0 + blockIdx.x * (int64_t)256 + threadIdx.x; c < c1;
+         c += (int64_t)gridDim.x * 256) {
+        if (layer[c] != EG_FREE<U>) continue;
+        U b[8];
+        float f[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            b[q] = layer[c + off[q]];
+            f[q] = phi[c + off[q]];
+        }
+        int nbs = 0;
+        float avg = 0.f;
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (b[q] == d - 1) {
+                avg = avg + f[q];
+                nbs++;
+            }
+        if (nbs > 0) {
+            layer[c] = (U)d;
+            if (d >= 2) phi[c] = avg / (float)nbs + direction;  // (the first keeps its values)
+        } else if (last) {
+            phi[c] = set;
+        }
+    }
+}
+
+template <class U>
+static void extrap_grow(flof_ctx *ctx, float *phi, const Dims4 &D, int distance, int layers,
+                        bool inside)
+{
+    const int64_t n = D.st * D.T;
+    if (D.X < 3 || D.Y < 3 || D.Z < 3 || D.T < 3) return;  // no interior cell
+    Tmp tmp(ctx, (size_t)n * sizeof(U));
+    U *layer = tmp.as<U>();
+    const float direction = inside ? -1.f : 1.f;
+    const float set = direction * (float)(distance + 2);
+    hipLaunchKernelGGL(k_extrap_grow_mark<U>, dim3(grid_blocks(ctx, n)), dim3(256), 0,
+                       ctx->stream, (const float *)phi, layer, D, make_coord4(D), inside ? 1 : 0);
+    const int64_t c0 = D.st, c1 = n - D.st;  // (every neighbour of these is in the grid or outer)
+    const int last = std::max(1, layers);
+    for (int d = 1; d <= last; ++d)
+        hipLaunchKernelGGL(k_extrap_grow<U>, dim3(grid_blocks(ctx, c1 - c0)), dim3(256), 0,
+                           ctx->stream, phi, layer, D, c0, c1, (uint32_t)d, direction,
+                           d == last ? 1 : 0, set);
 }
 
 template <class U>
@@ -415,10 +499,26 @@ int flof_extrap4d_ls_simple(flof_grid4d *phi, int distance, int inside)
     // no interior cell is farther from another
     const int64_t farthest = (int64_t)D.X + D.Y + D.Z + D.T - 12;
     const int far = (int)std::max<int64_t>(0, std::min<int64_t>(farthest, 0x7fffffff));
-    if (std::min(distance, far) < 255)
-        extrap_layers<uint8_t>(ctx, (float *)phi->data, D, distance, far, inside != 0);
+    const int layers = std::min(distance, far);
+    // The distances cost their serial passes along y, z and t (0.16 us per cell
+    // of a line), and save about 1 us per layer beyond the fifth and million
+    // interior cells.  Calls of 1, 4, 16, 40 layers, grown / by distances, us:
+    // 16^4 17, 25, 67, 124 / 27, 44, 82, 138; 64^3 x 4 18, 30, 77, 166 / 42, 57,
+    // 119, 236; 40^3 x 60 32, 73, 259, 423 / 70, 99, 216, 314; 64^4 69, 202, 797,
+    // 1884 / 140, 222, 671, 1398.
+    const int64_t interior = (int64_t)std::max(0, D.X - 2) * std::max(0, D.Y - 2) *
+                             std::max(0, D.Z - 2) * std::max(0, D.T - 2);
+    const bool grow = (double)(layers - 5) * (double)interior <=
+                      160000. * ((double)D.Y + D.Z + D.T);
+    float *p = (float *)phi->data;
+    if (grow && layers < 254)
+        extrap_grow<uint8_t>(ctx, p, D, distance, layers, inside != 0);
+    else if (grow)
+        extrap_grow<uint32_t>(ctx, p, D, distance, layers, inside != 0);
+    else if (layers < 255)
+        extrap_layers<uint8_t>(ctx, p, D, distance, far, inside != 0);
     else
-        extrap_layers<uint32_t>(ctx, (float *)phi->data, D, distance, far, inside != 0);
+        extrap_layers<uint32_t>(ctx, p, D, distance, far, inside != 0);
     check_launch("k_extrap_*");
     API_CATCH(ctx)
 }

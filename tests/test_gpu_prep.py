@@ -65,11 +65,16 @@ def test_extrap_ls_simple_bit_exact(inside):
 @pytest.mark.parametrize("shape,marks,distance", [
     ((3, 3, 3, 3), 1, 4), ((2, 5, 5, 5), 0, 4), ((7, 5, 6, 9), 0, 3), ((66, 4, 5, 19), 2, 40),
     ((131, 5, 3, 20), 3, 60), ((64, 7, 4, 5), 2, 1), ((65, 3, 4, 5), 2, 0), ((129, 6, 3, 3), 1, -3),
-    ((300, 4, 4, 5), 1, 254), ((300, 4, 4, 5), 1, 255), ((7, 4, 290, 5), 1, 1000)])
+    ((300, 4, 4, 5), 1, 254), ((300, 4, 4, 5), 1, 255), ((7, 4, 290, 5), 1, 1000),
+    ((300, 4, 4, 5), 1, 253), ((400, 5, 5, 5), 2, 250), ((700, 5, 4, 6), 1, 400),
+    ((500, 6, 5, 7), 3, 120), ((1031, 4, 4, 5), 1, 253), ((1031, 4, 4, 5), 1, 254),
+    ((1031, 4, 4, 5), 1, 255), ((38, 30, 31, 29), 2, 40), ((2000, 3, 3, 3), 1, 900)])
 def test_extrap_layers_at_distance_and_row_edges_bit_exact(shape, marks, distance):
     """Rows of one to five wavefronts of cells, no, one and a few marked cells,
     distances of 0 to beyond the grid and around the largest that a byte holds,
-    NaN among the values: the oracle's layers bit for bit, both ways round."""
+    NaN among the values: the oracle's layers bit for bit, both ways round.  The
+    cases from 400 cells on, and the one of 38 x 30 x 31 x 29, take the layers
+    from distances, the others grow them."""
     X, Y, Z, T = shape
     rng = np.random.default_rng(sum(shape) + distance)
     a = rng.uniform(0.5, 9.0, (T, Z, Y, X)).astype(np.float32)
