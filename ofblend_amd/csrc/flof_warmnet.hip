@@ -367,6 +367,82 @@ k_space(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
     }
 }
 
+// The forward space convolution of grids whose tiles would stay nearly empty:
+// with few rows or planes per class of equal (y mod d, z mod d) a tile of k_space
+// holds little else than halo (8 x 8 x 8 x 400, d = 8: 8 outputs of 128).  A
+// wavefront takes 16 cells in a row and gathers their taps from memory, two per
+// MFMA in the same order, all loads under way together.
+template <bool LIFT>
+__global__ void __launch_bounds__(256)
+k_space_gather(const unsigned short *__restrict__ inb, const float *__restrict__ i0,
+               const float *__restrict__ i1, const float *__restrict__ P,
+               const bf16x8 *__restrict__ wf, const float *__restrict__ bias,
+               unsigned short *__restrict__ out_b, Geo g, Coord4 D4)
+{
+    const int lane = threadIdx.x & 63;
+    const int grp = lane >> 4, sub = grp >> 1, half = grp & 1;
+    bf16x8 wr[PAIRS_S];
+#pragma unroll
+    for (int p = 0; p < PAIRS_S; ++p) wr[p] = wf[p * 64 + lane];
+    const int waves = gridDim.x * 4;
+    const int ntiles = (g.n + 15) >> 4;
+    const int plane = g.X * g.Y;
+    for (int tile = blockIdx.x * 4 + (threadIdx.x >> 6); tile < ntiles; tile += waves) {
+        const int c = tile * 16 + (lane & 15);
+        const bool live = c < g.n;
+        int x, y, z, t;
+        decompose((uint32_t)(live ? c : 0), D4, x, y, z, t);
+        bool ok[PAIRS_S];
+        int nc[PAIRS_S];
+#pragma unroll
+        for (int p = 0; p < PAIRS_S; ++p) {
+            const int m0 = 2 * p, m1 = 2 * p + 1 < NS ? 2 * p + 1 : 2 * p;
+            const int dx = g.dil * (sub ? m1 % 3 - 1 : m0 % 3 - 1);
+            const int dy = g.dil * (sub ? m1 / 3 % 3 - 1 : m0 / 3 % 3 - 1);
+            const int dz = g.dil * (sub ? m1 / 9 - 1 : m0 / 9 - 1);
+            ok[p] = live && !(2 * p + 1 >= NS && sub) && x + dx >= 0 && x + dx < g.X &&
+                    y + dy >= 0 && y + dy < g.Y && z + dz >= 0 && z + dz < g.Z;
+            nc[p] = ok[p] ? c + dx + g.X * dy + plane * dz : 0;
+        }
+        bf16x8 b[PAIRS_S];
+        if (LIFT) {
+            float x0[PAIRS_S], x1[PAIRS_S];
+#pragma unroll
+            for (int p = 0; p < PAIRS_S; ++p) {
+                x0[p] = i0[nc[p]] * 0.25f;
+                x1[p] = i1[nc[p]] * 0.25f;
+            }
+#pragma unroll
+            for (int p = 0; p < PAIRS_S; ++p) {
+                float v[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) v[q] = lift(P, 8 * half + q, x0[p], x1[p]);
+                b[p] = pack8(make_float4(v[0], v[1], v[2], v[3]),
+                             make_float4(v[4], v[5], v[6], v[7]));
+            }
+        } else {
+#pragma unroll
+            for (int p = 0; p < PAIRS_S; ++p)
+                b[p] = __builtin_bit_cast(
+                    bf16x8, *(const u32x4 *)(inb + (int64_t)nc[p] * C + 8 * half));
+        }
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < PAIRS_S; ++p)
+            v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[p], ok[p] ? b[p] : bf16x8{}, v, 0, 0,
+                                                        0);
+        if (!live) continue;
+        u16x4 u;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            v[r] += bias[4 * grp + r];
+            u[r] = to_bf16(fmaxf(v[r], 0.f));
+            if (v[r] > 0.f && u[r] == 0) u[r] = 1;
+        }
+        *(u16x4 *)(out_b + (int64_t)c * C + 4 * grp) = u;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // The 3-tap time convolution.  A wavefront owns 64 consecutive cells of the 3D
 // grid (four tiles of 16) and marches through the t steps of one class mod d,
@@ -1127,12 +1203,28 @@ void launch_space(flof_ctx *ctx, const In &in, const bf16x8 *wf, const float *bi
 void space_fwd(flof_ctx *ctx, const In &in, bool first, const bf16x8 *wf, const float *bias,
                unsigned short *out, const Geo &g)
 {
+    const SpaceGeo S = space_geo(g, 8, 2048);
+    // A plane of a tile stands for 128 outputs per x block of 16.  Counting the
+    // two planes of halo, tiles that are to fill fewer than 32 of them each take
+    // longer than the gathering form.  The network's flow, tiles only / by this
+    // rule, us: 8 x 8 x 8 x 400 411 / 142, 3 x 3 x 3 x 3000 662 / 95, 16^3 x 64
+    // 169 / 133, 33 x 17 x 9 x 40 178 / 140, 24^4 175 / 164; full tiles are 2.5
+    // times as fast as gathers (32^4 299 / 465 if all were gathered).
+    const int64_t planes = (int64_t)S.total * (S.zlen + 2) * ((S.XW + 15) / 16);
+    if (32 * planes > (int64_t)g.n) {
+        const int64_t tiles = ((int64_t)g.n + 15) / 16;
+        const Coord4 D4{make_fastdiv((uint32_t)g.X), make_fastdiv((uint32_t)g.Y),
+                        make_fastdiv((uint32_t)g.Z)};
+        hipLaunchKernelGGL(first ? k_space_gather<true> : k_space_gather<false>,
+                           dim3(grid_blocks(ctx, tiles * 64, 256, 4)), dim3(256), 0, ctx->stream,
+                           in.b, in.i0, in.i1, in.P, wf, bias, out, g, D4);
+        check_launch("k_space_gather");
+        return;
+    }
     if (first)
-        launch_space<true, SP_FWD>(ctx, in, wf, bias, nullptr, nullptr, out, nullptr,
-                                   space_geo(g, 8, 2048));
+        launch_space<true, SP_FWD>(ctx, in, wf, bias, nullptr, nullptr, out, nullptr, S);
     else
-        launch_space<false, SP_FWD>(ctx, in, wf, bias, nullptr, nullptr, out, nullptr,
-                                    space_geo(g, 8, 2048));
+        launch_space<false, SP_FWD>(ctx, in, wf, bias, nullptr, nullptr, out, nullptr, S);
 }
 
 // h' = res + (time conv of a + bias): FP32 and / or BF16, or its head

@@ -78,12 +78,14 @@ def test_gradients_match_oracle():
 
 
 @pytest.mark.parametrize("shape", [(3, 5, 9, 17), (9, 18, 3, 65), (17, 2, 33, 5), (1, 9, 8, 48),
-                                   (2, 3, 11, 61)])
+                                   (2, 3, 11, 61), (1, 33, 63, 17), (1, 32, 63, 65)])
 def test_network_tile_edges_match_oracle(shape):
     """Forward pass and gradients on grids whose rows fill the 16-cell tiles
     unevenly (17, 48 and 5 wide), span two x tiles (65), have fewer rows,
     planes or t steps than the widest tap spacing (8), or end a stretch of 64
-    cells early: the bounds of the two tests above."""
+    cells early: the bounds of the two tests above.  (The forward convolutions
+    of the small ones gather their taps, those of the last two use tiles at
+    every spacing; the backward ones always do.)"""
     say("warmnet tile edges", shape)
     s, a, b, g0, g1 = _case(shape)
     net = WS.WarmNet(seed=9)
@@ -229,7 +231,11 @@ def test_trained_network_saves_iterations_on_heldout_pairs():
     assert net_it < cold_it
 
 
-FLOW_SHAPES = [(6, 8, 8, 16), (9, 18, 3, 65), (17, 2, 33, 5), (5, 9, 8, 48), (3, 20, 18, 30)]
+# small grids and thin ones, whose taps are gathered, wholly or at the wider
+# spacings; then grids of full tiles one to three x blocks and tiles wide
+FLOW_SHAPES = [(6, 8, 8, 16), (9, 18, 3, 65), (17, 2, 33, 5), (5, 9, 8, 48), (3, 20, 18, 30),
+               (1, 35, 61, 13), (1, 33, 63, 17), (1, 33, 60, 47), (1, 32, 63, 65),
+               (1, 40, 58, 97), (2, 31, 62, 129)]
 
 
 def flow_digest(shape):
@@ -247,7 +253,7 @@ def flow_digest(shape):
 @pytest.mark.parametrize("shape", FLOW_SHAPES)
 def test_flow_is_the_gathering_kernels_flow(shape):
     """The digests were recorded on an MI355X with convolutions that gathered
-    every tap of a 16-cell tile from memory, two consecutive taps per MFMA in
+    and rounded every FP32 tap of a 16-cell tile from memory, two consecutive taps per MFMA in
     the order of the taps, and a head that summed a cell's channels one after
     another.  Which kernel stages the inputs must not change a bit: another
     order rounds some activations to the other BF16 neighbour, and the flow
