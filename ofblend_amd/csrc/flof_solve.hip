@@ -1607,10 +1607,12 @@ k_march3(const T *__restrict__ a, T *__restrict__ out,
     }
 }
 
-// The t segments: a CU runs one workgroup per 4 wavefronts of a segment, and
-// its VALUs are what bounds the pass, so the length is the one that gives the
-// busiest CU the fewest steps, counting 0.7 step per segment for its start
-// (32^3 x 48: 7 steps, 64^4: 16).
+// The t segments: a wavefront alone needs about 3 us per step and two for its
+// start (latency), the busiest CU a step's worth of VALU time per workgroup and
+// step and 1.5 for each one's start; the length with the smaller of the two
+// partly hidden behind the larger is taken.  (With the CU's steps alone short
+// grids ran few, long segments: blurs of 130 x 20^3 scalars 38 us instead of 56,
+// of 36 x 30 x 28 x 40 Vec4 82 instead of 97, of 16^4 24 instead of 26.)
 static March3 make_march3(const flof_ctx *ctx, const Dims4 &D)
 {
     March3 M;
@@ -1620,7 +1622,8 @@ static March3 make_march3(const flof_ctx *ctx, const Dims4 &D)
     for (int len = std::min(64, D.T); len >= 1; --len) {
         const int nseg = (D.T + len - 1) / len;
         const int64_t rounds = ((int64_t)M.nwg * nseg + ctx->num_cu - 1) / ctx->num_cu;
-        const double cost = (double)rounds * (len + 0.7);
+        const double alone = 3. * (len + 2), busy = (double)rounds * (len + 1.5);
+        const double cost = std::max(alone, busy) + 0.6 * std::min(alone, busy);
         if (cost < best) {
             best = cost;
             M.seglen = len;
@@ -1700,8 +1703,8 @@ k_blur4d(const T *__restrict__ src, T *__restrict__ dst, Dims4 D, Coord4 C, int 
 // then return 0; rows outside in y get such an address.  The weight sum of a
 // clipped window depends only on how far the faces clip it: `wsum` holds it
 // for each of the 4^4 clipping patterns (per dimension the window of an
-// interior cell is [-1, 2], [-2, 1], [-2, 2] or [-1, 1]), summed on the host
-// in the reference's order.
+// interior cell is [-1, 2], [-2, 1], [-2, 2] or [-1, 1]), summed in the
+// reference's order (k_blur5_wsum).
 struct Blur5W {
     float w[17];  // weight by squared distance 0..16
 };
@@ -1887,8 +1890,46 @@ k_march5(const float *__restrict__ src, float *__restrict__ dst, int ncomp, Dims
     }
 }
 
-// The t segments of k_march5, as make_march3 picks them; a segment's two ends
-// cost about 2.5 steps (their planes serve fewer outputs)
+// The weight sums of the 4^4 clipping patterns, a thread each, in the
+// reference's order.  (The reads of a z step's weights are under way together;
+// as plain loops over each pattern's bounds the 625 reads stood one behind
+// another, 26 us, and on the host the sums took 50.)
+__global__ void __launch_bounds__(256) k_blur5_wsum(const float *__restrict__ w, float *__restrict__ sum)
+{
+    __shared__ float sw[17];
+    if (threadIdx.x < 17) sw[threadIdx.x] = w[threadIdx.x];
+    __syncthreads();
+    const int p = threadIdx.x;
+    int lo[4], hi[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // t, z, y, x
+        const int pat = p >> (2 * (3 - q)) & 3;
+        lo[q] = -(pat / 2 + 1);
+        hi[q] = pat % 2 + 1;
+    }
+    float weight = 0.f;
+    for (int vt = lo[0]; vt <= hi[0]; ++vt)
+        for (int zk = lo[1]; zk <= hi[1]; ++zk) {
+            float v[9];
+#pragma unroll
+            for (int d = 0; d < 9; ++d) v[d] = sw[vt * vt + zk * zk + d];
+#pragma unroll
+            for (int yj = -2; yj <= 2; ++yj)
+#pragma unroll
+                for (int xi = -2; xi <= 2; ++xi) {
+                    const bool in = yj >= lo[2] && yj <= hi[2] && xi >= lo[3] && xi <= hi[3];
+                    const float next = weight + v[yj * yj + xi * xi];
+                    weight = in ? next : weight;
+                }
+        }
+    sum[p] = weight;
+}
+
+// The t segments of k_march5: a wavefront alone takes about 6 us per step up to
+// 4 (their planes serve few outputs, each a chain of its own) and 2.1 for each
+// further one, the busiest CU 2 us per workgroup and 1.5 per step of it.  (By
+// the CU's time alone, calls of two passes on scalars: 16^4 92 -> 82 us, 24^4
+// 115 -> 103, 130 x 20^3 160 -> 150, 50 x 46 x 44 x 40 369 -> 355.)
 static March3 make_march5(const flof_ctx *ctx, const Dims4 &D, int ncomp)
 {
     March3 M;
@@ -1899,7 +1940,9 @@ static March3 make_march5(const flof_ctx *ctx, const Dims4 &D, int ncomp)
     for (int len = D.T; len >= 1; --len) {
         const int nseg = (D.T + len - 1) / len;
         const int64_t rounds = ((int64_t)M.nwg * nseg + ctx->num_cu - 1) / ctx->num_cu;
-        const double cost = (double)rounds * (len + 2.5);
+        const double ends = std::min(len, 4), steps = std::max(0, len - 4);
+        const double cost =
+            std::max(6. * ends + 2.1 * steps, (double)rounds * (2. + 1.5 * (ends + steps)));
         if (cost < best) {
             best = cost;
             M.seglen = len;
@@ -1953,30 +1996,10 @@ void gaussian_blur(flof_ctx *ctx, void *a, const Dims4 &D, bool vec4, float sigm
         s == 2 && (D.st + 2 * D.sz + 2 * (int64_t)D.X) * (vec4 ? 16 : 4) < (1ll << 32) - 64;
     if (march5) {
         for (int d = 0; d < 17; ++d) w5.w[d] = wh[d];
-        std::vector<float> ws(256);
-        for (int pt = 0; pt < 4; ++pt)
-            for (int pz = 0; pz < 4; ++pz)
-                for (int py = 0; py < 4; ++py)
-                    for (int px = 0; px < 4; ++px) {
-                        float weight = 0.f;
-                        const int pat[4] = {pt, pz, py, px};
-                        int lo[4], hi[4];
-                        for (int q = 0; q < 4; ++q) {
-                            lo[q] = -(pat[q] / 2 + 1);
-                            hi[q] = pat[q] % 2 + 1;
-                        }
-                        for (int vt = lo[0]; vt <= hi[0]; ++vt)
-                            for (int zk = lo[1]; zk <= hi[1]; ++zk)
-                                for (int yj = lo[2]; yj <= hi[2]; ++yj)
-                                    for (int xi = lo[3]; xi <= hi[3]; ++xi)
-                                        weight = weight +
-                                                 wh[vt * vt + zk * zk + yj * yj + xi * xi];
-                        ws[((pt * 4 + pz) * 4 + py) * 4 + px] = weight;
-                    }
         wsum5 = Tmp(ctx, 256 * sizeof(float));
-        FLOF_HIP(hipMemcpyAsync(wsum5.p, ws.data(), 256 * sizeof(float),
-                                hipMemcpyHostToDevice, ctx->stream));
-        FLOF_HIP(hipStreamSynchronize(ctx->stream));  // ws lives on the stack
+        hipLaunchKernelGGL(k_blur5_wsum, dim3(1), dim3(256), 0, ctx->stream,
+                           (const float *)wdev.as<float>(), wsum5.as<float>());
+        check_launch("k_blur5_wsum");
         M5 = make_march5(ctx, D, vec4 ? 4 : 1);
     }
     auto pass = [&](const void *src, void *dst) {
