@@ -488,10 +488,21 @@ k_resample(S *__restrict__ dst, Dims4 Dd, Coord4 Cd, const S *__restrict__ src, 
     };
     const int ta = seg * len, tb = min(ta + len, Dd.T);
     S *__restrict__ out = dst + (int64_t)i + (int64_t)Dd.X * j + Dd.sz * k;
+    auto store = [&](int t, const T &z0, float g0, const T &z1, float g1) {
+        T v = O::add(O::muls(z0, g0), O::muls(z1, g1));
+        if (use_post) v = O::muls(v, post);
+        out[Dd.st * t] = L::st(v);
+    };
+    float g0, g1;
+    if (len == 1) {  // without a branch between the slices: all gathers under way at once
+        const int ti = axis((float)ta * fac.w + off.w, Ds.T, g0, g1);
+        const T z0 = slice(ti), z1 = slice(ti + 1);
+        store(ta, z0, g0, z1, g1);
+        return;
+    }
     int tc = -2;  // z0 is the sample of slice tc, z1 that of the next
     T z0 = O::zero(), z1 = O::zero();
     for (int t = ta; t < tb; ++t) {
-        float g0, g1;
         const int ti = axis((float)t * fac.w + off.w, Ds.T, g0, g1);
         if (ti != tc) {
             if (ti == tc + 1) z0 = z1;
@@ -499,9 +510,7 @@ k_resample(S *__restrict__ dst, Dims4 Dd, Coord4 Cd, const S *__restrict__ src, 
             z1 = slice(ti + 1);
             tc = ti;
         }
-        T v = O::add(O::muls(z0, g0), O::muls(z1, g1));
-        if (use_post) v = O::muls(v, post);
-        out[Dd.st * t] = L::st(v);
+        store(t, z0, g0, z1, g1);
     }
 }
 
@@ -509,9 +518,15 @@ template <class T, class S = T>
 static void resample(flof_ctx *ctx, void *dst, const Dims4 &Dd, const void *src, const Dims4 &Ds,
                      float4 fac, float4 off, float post, int use_post)
 {
-    // eight wavefronts per SIMD, if the grid has them
-    const int64_t want = (int64_t)ctx->num_cu * 2048;
-    const int64_t segs = std::min<int64_t>(Dd.T, std::max<int64_t>(1, (want + Dd.st - 1) / Dd.st));
+    // twice eight wavefronts per SIMD, if the grid has them (the steps of a march
+    // wait for their gathers one after another); a source twice as fine in t
+    // shares no slices between outputs: a thread each.  Calls with Real grids, one
+    // cell per thread and iteration / this: 64^4 to 32^4 23.4 / 23.4 us, to 32^3 x
+    // 64 24.6 / 24.4, 40^3 x 60 to 100^3 x 60 243 / 137.
+    const int64_t want = (int64_t)ctx->num_cu * 4096;
+    const int64_t segs =
+        fac.w >= 2.f ? Dd.T
+                     : std::min<int64_t>(Dd.T, std::max<int64_t>(1, (want + Dd.st - 1) / Dd.st));
     const int len = (int)((Dd.T + segs - 1) / segs);
     const uint32_t threads = (uint32_t)(Dd.st * ((Dd.T + len - 1) / len));
     hipLaunchKernelGGL((k_resample<T, S>), dim3((threads + 255u) / 256u), dim3(256), 0,

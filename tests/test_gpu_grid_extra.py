@@ -113,9 +113,10 @@ def test_advect_columns_at_edges_bit_exact(shape):
 
 @pytest.mark.parametrize("src,dst", [((7, 6, 5, 9), (90, 91, 70, 8)), ((7, 6, 5, 3), (90, 91, 70, 8)),
                                      ((7, 6, 5, 9), (90, 91, 70, 3)), ((20, 3, 2, 17), (21, 40, 3, 35)),
-                                     ((5, 4, 3, 2), (2, 3, 2, 40))])
+                                     ((5, 4, 3, 2), (2, 3, 2, 40)),
+                                     ((7, 6, 5, 9), (103, 102, 101, 5))])
 def test_resample_marches_in_t_bit_exact(src, dst):
-    """Grids of one t segment and of one per slice, up to 13 outputs per source
+    """Grids of one, two and a t segment per slice, up to 13 outputs per source
     slice and several source slices per output: the oracle's values bit for
     bit, scalars and Vec4, with an offset that leaves the grid."""
     rng = np.random.default_rng(32)
