@@ -518,12 +518,14 @@ template <class T, class S = T>
 static void resample(flof_ctx *ctx, void *dst, const Dims4 &Dd, const void *src, const Dims4 &Ds,
                      float4 fac, float4 off, float post, int use_post)
 {
-    // twice eight wavefronts per SIMD, if the grid has them (the steps of a march
-    // wait for their gathers one after another); a source twice as fine in t
-    // shares no slices between outputs: a thread each.  Calls with Real grids, one
-    // cell per thread and iteration / this: 64^4 to 32^4 23.4 / 23.4 us, to 32^3 x
-    // 64 24.6 / 24.4, 40^3 x 60 to 100^3 x 60 243 / 137.
-    const int64_t want = (int64_t)ctx->num_cu * 4096;
+    // Eight wavefronts per SIMD, if the grid has them, for outputs that lie denser
+    // than the source in t and share its slices; twice as many for others (the
+    // steps of a march wait for their gathers one after another), and a thread
+    // each where the source is twice as fine and nothing is shared.  Calls, one
+    // cell per thread and iteration / this: Real 64^4 to 32^4 23.4 / 23.4 us, to
+    // 32^3 x 64 24.6 / 24.4, 40^3 x 60 to 100^3 x 60 243 / 137; Vec4 50^3 x 4 to
+    // 100^3 x 8 79 / 37 (43 with twice the threads).
+    const int64_t want = (int64_t)ctx->num_cu * (fac.w < 1.f ? 2048 : 4096);
     const int64_t segs =
         fac.w >= 2.f ? Dd.T
                      : std::min<int64_t>(Dd.T, std::max<int64_t>(1, (want + Dd.st - 1) / Dd.st));
