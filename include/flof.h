@@ -278,7 +278,8 @@ int flof_stream_bandwidth(flof_ctx *ctx, int mix, int64_t cells, int reps, doubl
 int flof_check_reciprocal(flof_ctx *ctx, uint32_t lo, uint32_t hi, uint64_t *mismatches);
 
 /* ---- Grid4d storage (source/grid4d.h:117-265, source/grid4d.cpp:60-138) - */
-/* Creates a zero-initialised X*Y*Z*T grid (x fastest, then y, z, t). */
+/* Creates a zero-initialised X*Y*Z*T grid (x fastest, then y, z, t).  It is
+ * cleared when the call returns. */
 int flof_grid4d_create(flof_ctx *ctx, int X, int Y, int Z, int T, int elem,
                        int dtype, flof_grid4d **out);
 int flof_grid4d_destroy(flof_grid4d *g);
@@ -625,6 +626,7 @@ int flof_drop_frames3d(flof_ctx *ctx, float *frames_dev, int X, int Y, int Z,
 size_t flof_abi_struct_size(int which);
 
 /* ---- device memory helpers for 3D frames ------------------------------- */
+/* Zero-initialised, and cleared when the call returns. */
 int flof_dev_alloc(flof_ctx *ctx, size_t bytes, void **out);
 int flof_dev_free(flof_ctx *ctx, void *ptr);
 int flof_dev_upload(flof_ctx *ctx, void *dst_dev, const void *src,

@@ -1548,6 +1548,19 @@ int flof_check_reciprocal(flof_ctx *ctx, uint32_t lo, uint32_t hi, uint64_t *mis
     API_CATCH(ctx)
 }
 
+// Zeroes fresh memory and waits for it: the caller may write to the buffer on any
+// stream once it has the address, and a clearing that still runs, or waits its
+// turn on the context's stream, would wipe that out.  (On the null stream where
+// the context has work under way.)
+static void clear_new(flof_ctx *ctx, void *p, size_t bytes)
+{
+    const bool idle = hipStreamQuery(ctx->stream) == hipSuccess;
+    if (!idle) (void)hipGetLastError();
+    const hipStream_t q = idle ? ctx->stream : nullptr;
+    FLOF_HIP(hipMemsetAsync(p, 0, bytes, q));
+    FLOF_HIP(hipStreamSynchronize(q));
+}
+
 int flof_grid4d_create(flof_ctx *ctx, int X, int Y, int Z, int T, int elem, int dtype,
                        flof_grid4d **out)
 {
@@ -1573,7 +1586,7 @@ int flof_grid4d_create(flof_ctx *ctx, int X, int Y, int Z, int T, int elem, int 
     g->dtype = dtype;
     g->bytes = (size_t)g->n() * elem_bytes(elem);
     FLOF_HIP(hipMalloc(&g->data, g->bytes));
-    FLOF_HIP(hipMemsetAsync(g->data, 0, g->bytes, ctx->stream));
+    clear_new(ctx, g->data, g->bytes);
     *out = g;
     }
     catch (const flof::Error &e)
@@ -1994,7 +2007,7 @@ int flof_dev_alloc(flof_ctx *ctx, size_t bytes, void **out)
     *out = nullptr;
     FLOF_HIP(hipMalloc(out, bytes));
     own_array(ctx, *out, bytes);
-    FLOF_HIP(hipMemsetAsync(*out, 0, bytes, ctx->stream));
+    clear_new(ctx, *out, bytes);
     API_CATCH(ctx)
 }
 

@@ -534,3 +534,30 @@ def test_advect_edges(shape):
         g.from_numpy(a)
         M.advect4d(vel, g, dtFac=0.7)
         assert np.array_equal(g.to_numpy(), O.advect4d(v, a, dt=1.0, dtFac=0.7))
+
+
+@pytest.mark.parametrize("kind", ["grid", "array"])
+def test_new_memory_is_cleared_before_its_address_is_known(kind):
+    """A new grid or array is zero, and stays what another stream writes to it
+    right away, while its context has work of some 20 ms queued."""
+    L = _lib.lib()
+    L.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    X, Y, Z, T = 48, 40, 44, 24
+    s = M.Solver(gridSize=M.vec3(X, Y, Z), fourthDim=T)
+    vel, busy = s.create(M.Grid4Vec4), s.create(M.Grid4Real)
+    a = np.random.default_rng(90).standard_normal((4, 5, 6, 7)).astype(np.float32)
+    for written in (False, True):
+        say("new", kind, "written", written)
+        g = None  # (the last one's release would wait for the queue)
+        for _ in range(600):
+            M.advect4d(vel, busy)
+        if kind == "grid":
+            g = M.Grid4Real(s, (7, 6, 5, 4))
+            p = L.flof_grid4d_device_ptr(g.h)
+        else:
+            g = M.DeviceArray(a.shape)
+            p = g.ptr.value
+        if written:  # on the null stream, from the host (hipMemcpyHostToDevice)
+            assert L.hipMemcpy(p, a.ctypes.data_as(C.c_void_p), a.nbytes, 1) == 0
+        _lib.check(L.flof_sync(g.ctx), g.ctx)
+        assert np.array_equal(g.to_numpy(), a if written else np.zeros_like(a))
