@@ -286,11 +286,9 @@ def test_reductions_mult_and_vec4_region():
 @pytest.mark.parametrize("X", [40, 70, 100])
 @pytest.mark.parametrize("sigma", [1.0, 2.0])
 def test_gaussian_blur_two_x_tiles_bit_exact(vec, X, sigma):
-    """gaussianBlur4d at sigma 1 and 2 (the LDS column marches over x tiles
-    with 3^4 and 5^4 windows) on grids 40, 70 and 100 wide (one ragged
-    64-wide tile, three 32-wide tiles, two 64-wide tiles): the seams between
-    the x tiles and the ragged last tile equal the oracle bit for bit, Vec4
-    and Real."""
+    """gaussianBlur4d at sigma 1 and 2 (the marches with 3^4 and 5^4 windows) on
+    grids 40, 70 and 100 wide, whose rows end anywhere in a wavefront's stretch
+    of cells: the oracle bit for bit, Vec4 and Real."""
     Y, Z, T = 9, 10, 11
     rng = np.random.default_rng(12)
     shp = (T, Z, Y, X, 4) if vec else (T, Z, Y, X)
@@ -328,9 +326,8 @@ def test_gaussian_blur_5x5_window_small_dims_bit_exact(shape):
 @pytest.mark.parametrize("vx", [0.0, 1.0])
 @pytest.mark.parametrize("X", [40, 70, 100])
 def test_corr_vels_of4d_two_x_tiles_bit_exact(vx, X):
-    """corrVelsOf4d on grids 40, 70 and 100 wide (the box passes on one
-    ragged 64-wide x tile, three 32-wide tiles, two 64-wide tiles): 4 and 5
-    extrapolation passes, random level sets, bit-exact to the oracle."""
+    """corrVelsOf4d on grids 40, 70 and 100 wide: 4 and 5 extrapolation passes,
+    random level sets, bit-exact to the oracle."""
     Y, Z, T = 10, 9, 8
     rng = np.random.default_rng(13)
     t, z, y, x = np.meshgrid(*[np.arange(s) + 0.5 for s in (T, Z, Y, X)], indexing="ij")
@@ -355,13 +352,16 @@ def test_corr_vels_of4d_two_x_tiles_bit_exact(vx, X):
 
 
 @pytest.mark.parametrize("shape", [(3, 3, 3, 3), (61, 4, 5, 9), (62, 3, 4, 18), (63, 5, 3, 7),
-                                   (31, 6, 7, 33), (7, 30, 3, 70)])
+                                   (31, 6, 7, 33), (7, 30, 3, 70), (70, 33, 20, 14),
+                                   (64, 48, 40, 11), (101, 41, 37, 13)])
 def test_marches_at_wavefront_and_segment_edges_bit_exact(shape):
     """The blur marches (3^4 and 5^4 windows) and the box passes where a
     wavefront's stretch of 62 cells (60 positions for the 5^4 window) ends at,
     just before and just after a row's end, with one interior cell, and with t
     extents that one, two and several t segments cover, infinities and NaN
-    among the values: equal to the oracle bit for bit."""
+    among the values: equal to the oracle bit for bit.  (Small grids march single
+    t steps; the last three segments of 3 to 13, where all three or five outputs
+    of a plane are in flight.)"""
     X, Y, Z, T = shape
     rng = np.random.default_rng(15)
     s = M.Solver(gridSize=M.vec3(X, Y, Z), fourthDim=T)
